@@ -282,6 +282,7 @@ struct Frame {
   contour3d_amd_mesh mesh;  // the frame's triangles, kept between frames
   std::vector<Geom*> geoms_used;  // lattice tables the frame in flight reads
   TessLayout tl;
+  uint32_t ntiles = 0;  // pixel tiles of the frame's images (the resolve's workgroups)
   // the captured launch sequence of the last frame layout, replayed while
   // the layout (sizes, buffers, capacities) stays the same
   hipGraphExec_t gexec = nullptr;
@@ -1354,8 +1355,8 @@ int raster_launch(Lib&, Frame& F, const contour3d_amd_mesh& M, const RasterJob<R
   }
   if (prof_end(F)) return 1;
   if (prof_begin(F, CONTOUR3D_AMD_STAGE_RESOLVE)) return 1;
-  C3D_HIP(launch_resolve<R>(mv, rjobs, njobs, npx, M.meta.as<ObjMeta>(), int(M.base.size()), F.frgb.as<uint8_t>(),
-                            hdr, key, id, 1u << 30, F.st));
+  C3D_HIP(launch_resolve<R>(mv, rjobs, njobs, F.ntiles, M.meta.as<ObjMeta>(), int(M.base.size()),
+                            F.frgb.as<uint8_t>(), hdr, key, id, F.st));
   if (prof_end(F)) return 1;
   return 0;
 }
@@ -1483,6 +1484,7 @@ template <typename R>
 void fill_rjobs(Frame& F, const std::vector<Image>& imgs) {
   std::vector<RasterJob<R>>& rj = F.rjobs_host<R>();
   rj.assign(imgs.size(), RasterJob<R>{});
+  F.ntiles = 0;
   for (size_t q = 0; q < imgs.size(); q++) {
     const Image& im = imgs[q];
     RasterJob<R>& j = rj[q];
@@ -1490,6 +1492,8 @@ void fill_rjobs(Frame& F, const std::vector<Image>& imgs) {
     j.px0 = im.px0;
     j.obj0 = im.obj0;
     j.obj1 = im.obj1;
+    j.tile0 = F.ntiles;
+    F.ntiles += resolve_tiles(im.hv.W, im.hv.H);
     j.rgb = im.rgb_dev ? im.rgb : F.rgb.as<uint8_t>() + 3 * im.px0;
     j.depth = im.depth ? (im.dep_dev ? im.depth : F.depth.as<double>() + im.px0) : nullptr;
     j.bg[0] = im.hv.bg.r;
@@ -1567,8 +1571,8 @@ int fused_launch(Lib& L, Frame& F, const contour3d_amd_mesh& M, const RasterJob<
   }
   if (prof_end(F)) return 1;
   if (prof_begin(F, CONTOUR3D_AMD_STAGE_RESOLVE)) return 1;
-  C3D_HIP(launch_resolve_field<R>(tj, cell, rjobs, njobs, npx, M.meta.as<ObjMeta>(), int(M.base.size()),
-                                  F.frgb.as<uint8_t>(), hdr, key, id, F.st));
+  C3D_HIP(launch_resolve_field<R>(tj, cell, rjobs, njobs, F.ntiles, M.meta.as<ObjMeta>(), F.frgb.as<uint8_t>(), hdr,
+                                  key, id, F.st));
   if (prof_end(F)) return 1;
   return 0;
 }
@@ -1607,7 +1611,7 @@ int graph_frame(Lib& L, Frame& F, contour3d_amd_mesh& M, std::vector<Image>& img
   }
   const uint32_t lines = line_capacity(F);
   const std::vector<uint64_t> sig = {
-      sizeof(R), uint64_t(njobs), npx, F.tl.nbt, F.tl.ntj, uint64_t(F.tl.njobs), uint64_t(F.tl.nobj),
+      sizeof(R), uint64_t(njobs), npx, F.ntiles, F.tl.nbt, F.tl.ntj, uint64_t(F.tl.njobs), uint64_t(F.tl.nobj),
       L.tess_cap, L.tess_grid(F.tl.ntj), L.tess_rows, L.tess_zc, lines, M.cap, F.frag_cap,
       uint64_t(uintptr_t(F.cnt.p)), uint64_t(uintptr_t(F.tiles.p)), uint64_t(uintptr_t(F.tjobs.p)),
       uint64_t(uintptr_t(F.rjobs.p)), uint64_t(uintptr_t(F.hdr.p)), uint64_t(uintptr_t(F.jimg.p)),

@@ -168,6 +168,7 @@ struct RasterJob {
   uint64_t wk0;          // filled on the device by k_plan
   uint64_t px0;
   uint32_t obj0, obj1;
+  uint32_t tile0;        // first of its pixel tiles in the frame (resolve_tiles)
   uint8_t* rgb;          // device, W*H*3 in PPM row order
   double* depth;         // device or null
   uint8_t bg[4];
@@ -235,8 +236,10 @@ hipError_t launch_tess_raster(const TessJob* jobs, int njobs, uint32_t nitems, c
 // smoothing weights are recomputed from the fields (id as launch_tess_raster)
 template <typename R>
 hipError_t launch_resolve_field(const TessJob* jobs, const uint32_t* cell, const RasterJob<R>* rjobs, int njobs,
-                                uint64_t npx_total, const ObjMeta* meta, int nobj, const uint8_t* frag_rgb,
-                                const FrameHdr* hdr, const uint64_t* key, const void* id, hipStream_t st);
+                                uint32_t ntiles, const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr,
+                                const uint64_t* key, const void* id, hipStream_t st);
+// pixel tiles of a W x H image (the resolve's workgroups)
+uint32_t resolve_tiles(uint64_t W, uint64_t H);
 // clears the z-buffer (and the ids: uint64_t per pixel when wide, else
 // uint32_t), the header's fragment count and list-overflow bit, and with
 // fresh (FP64 frames) also its triangle count and capacity bit
@@ -271,9 +274,10 @@ hipError_t launch_frag_ids(const void* frags, bool wide, uint32_t cap, const Fra
 // frame's hdr->ntri triangles
 hipError_t launch_line_frags(const uint32_t* pix, const double* depth, uint32_t cap, const FrameHdr* hdr,
                              int pass, int precision, uint64_t* key, void* id, bool wide, hipStream_t st);
+// resolve of a stored mesh; ntiles: the sum of the images' resolve_tiles
 template <typename R>
-hipError_t launch_resolve(const MeshView<R>& m, const RasterJob<R>* rjobs, int njobs, uint64_t npx_total,
+hipError_t launch_resolve(const MeshView<R>& m, const RasterJob<R>* rjobs, int njobs, uint32_t ntiles,
                           const ObjMeta* meta, int nobj, const uint8_t* frag_rgb, const FrameHdr* hdr,
-                          const uint64_t* key, const uint32_t* id, uint32_t grid, hipStream_t st);
+                          const uint64_t* key, const uint32_t* id, hipStream_t st);
 
 }  // namespace c3d

@@ -530,41 +530,6 @@ __device__ __forceinline__ void slot_positions(const FieldDev& f, const CellLoc&
   }
 }
 
-// The six grid coordinates of cell L (x0 x1 y0 y1 z0 z1) on a grid lattice.
-__device__ __forceinline__ void cell_grid(const FieldDev& f, const CellLoc& L, double g6[6]) {
-  g6[0] = gptr(f.gx)[L.i];
-  g6[1] = gptr(f.gx)[L.i + 1];
-  g6[2] = gptr(f.gy)[L.j];
-  g6[3] = gptr(f.gy)[L.j + 1];
-  g6[4] = gptr(f.gz)[L.k];
-  g6[5] = gptr(f.gz)[L.k + 1];
-}
-
-// slot_positions with the cell's corner values v and, on a grid lattice,
-// its six grid coordinates g6 (cell_grid) already in registers
-template <typename R>
-__device__ __forceinline__ void slot_positions_reg(const FieldDev& f, const CellLoc& L, double thr, uint64_t ent,
-                                                   const double v[8], const double g6[6], V3<R> P[3]) {
-  if (f.cx) {
-    slot_positions<R>(f, L, thr, ent, v, P);
-    return;
-  }
-#pragma unroll
-  for (int vv = 0; vv < 3; vv++) {
-    const uint32_t tail = uint32_t(ent >> (6 * vv)) & 7u;
-    const uint32_t head = uint32_t(ent >> (6 * vv + 3)) & 7u;
-    double vt = v[0], vh = v[0];
-#pragma unroll
-    for (int q = 1; q < 8; q++) {
-      vt = tail == uint32_t(q) ? v[q] : vt;
-      vh = head == uint32_t(q) ? v[q] : vh;
-    }
-    const V3<R> pt = {R(tail & 1u ? g6[1] : g6[0]), R(tail & 2u ? g6[3] : g6[2]), R(tail & 4u ? g6[5] : g6[4])};
-    const V3<R> ph = {R(head & 1u ? g6[1] : g6[0]), R(head & 2u ? g6[3] : g6[2]), R(head & 4u ? g6[5] : g6[4])};
-    P[vv] = interp<R>(thr, pt, vt, ph, vh);
-  }
-}
-
 // The smoothing weight of a triangle: area * unit face normal
 // (triangulate.c:75-93), formed as normal.c:39-40 forms it.  The FP32 form
 // takes the cross product itself (the same vector): a triangle whose
@@ -818,20 +783,6 @@ __device__ __forceinline__ uint32_t ord32(float x) {
 __device__ __forceinline__ float unord32(uint32_t k) {
   const uint32_t u = (k >> 31) ? (k & 0x7fffffffu) : ~k;
   return __uint_as_float(u);
-}
-
-// loads triangle t, projects it and sets up its reference box; false when
-// a vertex is rejected by the projection
-template <typename R>
-__device__ __forceinline__ bool setup_tri(const MeshView<R>& m, uint64_t t, const ViewDev<R>& v, Projected<R>& P,
-                                          R& area) {
-#pragma unroll
-  for (int n = 0; n < 3; n++) {
-    const V3<R> p = {m.pos[t].p[3 * n + 0], m.pos[t].p[3 * n + 1], m.pos[t].p[3 * n + 2]};
-    if (!project(v, p, P.q[n])) return false;
-  }
-  area = raster_box(v, P);
-  return true;
 }
 
 // the image owning raster work item u (the last job starting at or before
@@ -1613,174 +1564,172 @@ __global__ void k_line_frags(const uint32_t* __restrict__ pix, const double* __r
   }
 }
 
-// Final colour of every pixel from the winning fragment.  The vertex normals
-// of a winning triangle are gathered here, on demand: the image needs them
-// only where a triangle is nearest, so the smoothing of normal.c is done for
-// those triangles alone, with the same sums.  rgb rows are written top-down
-// (y index H-1 first) as the PPM writer packs them (output.c:113-123).
+// ----------------------------------------------------------------------
+// resolve: the final colour of every pixel from its winning fragment
+//
+// A workgroup takes a 32 x 8 pixel tile of one image, in three phases:
+//   1. one thread per pixel: the winning triangle, its barycentric weights
+//      at the pixel centre, and the three lattice edges its vertices lie on.
+//      The edges are entered in a hash table in LDS;
+//   2. the tile's distinct edges are shared out over the waves, and each
+//      one's smoothed vertex normal (normal.c:46-165) is formed once;
+//   3. one thread per pixel again: shading (render.c:137-159) and the write,
+//      in PPM row order (output.c:113-123).
+// The normals of normal.c are needed only where a triangle is nearest, and
+// a vertex normal depends on its lattice edge alone: the cells that share
+// the edge are visited in increasing order and their triangles in slot
+// order, whichever cell the vertex is seen from, so one sum serves every
+// triangle with a vertex on the edge, bit for bit.
+//
+// What bounds it: the chain of dependent reads behind a vertex normal
+// (corner values, code, slot masks, slots: 4, 2 or 1 cells per edge).  With
+// one thread gathering all three normals of a pixel's triangle the chains
+// ran one after the other and neighbouring pixels repeated them; a tile's
+// 768 vertices are a few hundred distinct edges at a pixel per cell and a
+// few dozen on a close-up.
+constexpr uint32_t kTileW = 32, kTileH = kThreads / 32;  // pixels of a workgroup's tile
+constexpr uint32_t kVtxSlots = 1024;                     // hash slots, at least 3 per pixel
+static_assert(kTileW * kTileH == kThreads && kVtxSlots > 3 * kThreads, "the tile's vertices fit the hash table");
+
+// The distinct vertices of a pixel tile: open addressing over vertex keys,
+// each occupied slot numbered in order of entry (idx), and the numbered
+// slots and their normals.
 template <typename R>
-__global__ __launch_bounds__(kThreads) void k_resolve(MeshView<R> m, const RasterJob<R>* __restrict__ rjobs, int njobs,
-                                                      uint64_t npx_total, const ObjMeta* __restrict__ meta, int nobj,
-                                                      const uint8_t* __restrict__ frag_rgb,
-                                                      const FrameHdr* __restrict__ hdr,
-                                                      const uint64_t* __restrict__ key,
-                                                      const uint32_t* __restrict__ idbuf) {
-  // a frame whose triangles outgrew the mesh is rendered again: skip it
-  if (hdr->overflow & 1u) return;
-  const uint64_t ntri = hdr->ntri;
-  for (uint64_t p0 = uint64_t(blockIdx.x) * kThreads; p0 < npx_total; p0 += uint64_t(gridDim.x) * kThreads) {
-    // images start on workgroup boundaries of the pixel space, so the
-    // image of a workgroup round is uniform
-    int jb = 0;
-    if (njobs > 1) {
-      int lo = 0, hi = njobs - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (rjobs[mid].px0 <= p0) lo = mid;
-        else hi = mid - 1;
-      }
-      jb = lo;
-    }
-    const RasterJob<R>& J = rjobs[jb];
-    const ViewDev<R> v = J.v;
-    const uint64_t p = p0 + threadIdx.x;
-    const uint64_t lp = p - J.px0;
-    if (lp >= uint64_t(v.W) * uint64_t(v.H)) continue;
-    const int32_t j = int32_t(lp / uint64_t(v.W));
-    const int32_t i = int32_t(lp - uint64_t(j) * uint64_t(v.W));
-    const uint64_t k = key[p];
-    uint32_t id;
-    double dep;
-    if constexpr (sizeof(R) == 8) {
-      id = idbuf[p];
-      dep = unord64(k);
-    } else {
-      id = uint32_t(k);
-      dep = id ? double(unord32(uint32_t(k >> 32))) : -DBL_MAX;
-    }
-    uint8_t r = J.bg[0], gg = J.bg[1], b = J.bg[2];
-    if (id != 0 && id <= ntri) {
-      const uint64_t t = id - 1;
-      int lo = 0, hi = nobj - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (meta[mid].base <= t) lo = mid;
-        else hi = mid - 1;
-      }
-      const ObjMeta om = meta[lo];
-      Projected<R> P;
-      R area;
-      setup_tri(m, t, v, P, area);
-      R w0, w1, w2;
-      pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2);
-      const uint32_t c = m.aux[t].cell;
-      const uint32_t ed = edges_of(m, t);
-      V3<R> nv[3];
-#pragma unroll 1
-      for (int n = 0; n < 3; n++) nv[n] = vertex_normal<R>(m, om, c, (ed >> (5 * n)) & 31u);
-      const V3<R> n = vunit(vadd(vscale(w0, nv[0]), vadd(vscale(w1, nv[1]), vscale(w2, nv[2]))));
-      const V3<R> light = {v.light[0], v.light[1], v.light[2]};
-      const R fct = fmax(R(0.15), fabs(vdot(n, light)));
-      r = uint8_t(fct * R(om.rgb[0]));
-      gg = uint8_t(fct * R(om.rgb[1]));
-      b = uint8_t(fct * R(om.rgb[2]));
-    } else if (id > ntri) {
-      const uint64_t f = id - ntri - 1;
-      r = frag_rgb[3 * f + 0];
-      gg = frag_rgb[3 * f + 1];
-      b = frag_rgb[3 * f + 2];
-    }
-    const uint64_t o = (uint64_t(v.H - 1 - j) * uint64_t(v.W) + uint64_t(i)) * 3;
-    J.rgb[o + 0] = r;
-    J.rgb[o + 1] = gg;
-    J.rgb[o + 2] = b;
-    if (J.depth) J.depth[lp] = dep;
+struct VtxTable {
+  unsigned long long key[kVtxSlots];
+  uint16_t idx[kVtxSlots];
+  uint16_t slot[3 * kThreads];
+  R n[3 * kThreads][3];
+  uint32_t count;
+};
+
+constexpr unsigned long long kNoVtx = ~0ull;
+
+// A vertex's lattice edge as object, cell and direction: the edge runs from
+// corner 0 of that cell to corner `dir` (1-7).  An interior cell's edges
+// all start at corner 0 of a cell of the lattice.
+__device__ __forceinline__ unsigned long long vtx_key(uint32_t obj, uint32_t cell, uint32_t dir) {
+  return (unsigned long long)obj << 36 | (unsigned long long)cell << 4 | dir;
+}
+
+// the cell whose corner 0 is corner `lo` of cell c
+__device__ __forceinline__ uint32_t corner_cell(uint32_t c, uint32_t lo, uint32_t ncx, uint32_t ncy) {
+  return c + (lo & 1u) + (lo & 2u ? ncx : 0u) + (lo & 4u ? ncx * ncy : 0u);
+}
+
+// the lower corner and the direction of cell-local edge e
+__device__ __forceinline__ void edge_lo_dir(uint32_t e, uint32_t& lo, uint32_t& dir) {
+  if (e < 4u) {
+    lo = 2u * e;
+    dir = 1u;
+  } else if (e < 8u) {
+    lo = (e & 1u) | ((e - 4u) >> 1) << 2;
+    dir = 2u;
+  } else if (e < 12u) {
+    lo = e - 8u;
+    dir = 4u;
+  } else if (e < 14u) {
+    lo = e - 12u;
+    dir = 6u;
+  } else if (e < 16u) {
+    lo = (e - 14u) << 1;
+    dir = 5u;
+  } else if (e < 18u) {
+    lo = (e - 16u) << 2;
+    dir = 3u;
+  } else {
+    lo = 0u;
+    dir = 7u;
   }
 }
 
-// Vertex normal of the vertex on cell-local edge e of cell c, recomputed
-// from the field: the cells sharing the edge in increasing linear order
-// (normal.c:78-158), in each the triangles of threshold thr with a vertex
-// on the edge in slot order (c_emask lists them), their smoothing weights
-// summed from +0 and normalised -- the sums of vertex_normal over a stored
-// mesh, bit for bit.  Lc, vc and code_c are cell c's location, corner
-// values and corner code.
+// enters key k; returns its slot (idx and n are valid after a barrier)
 template <typename R>
-__device__ V3<R> vertex_normal_field(const FieldDev& f, double thr, uint32_t c, const CellLoc& Lc,
-                                     const double vc[8], uint32_t code_c, uint32_t e) {
-  const int64_t sy = f.ncx, sz = int64_t(f.ncx) * f.ncy;
-  V3<R> sum = {R(0), R(0), R(0)};
-  const int nn = c_nbr.n[e];
-  for (int q = 0; q < nn; q++) {
-    const int dk = c_nbr.v[e][q][0], dj = c_nbr.v[e][q][1], di = c_nbr.v[e][q][2];
-    const uint32_t want = uint32_t(c_nbr.v[e][q][3]);
-    const bool self = (dk | dj | di) == 0;
-    const uint32_t c2 = uint32_t(int64_t(c) + dk * sz + dj * sy + di);
-    const CellLoc L2 = self ? Lc : locate(f, c2);
-    double v2[8];
-    if (self) {
+__device__ __forceinline__ uint32_t vtx_enter(VtxTable<R>& T, unsigned long long k) {
+  uint32_t s = uint32_t((k * 0x9e3779b97f4a7c15ull) >> 54);
+  static_assert(kVtxSlots == 1u << 10, "the hash keeps 10 bits");
+  for (;;) {
+    const unsigned long long was = atomicCAS(&T.key[s], kNoVtx, k);
+    if (was == k) return s;
+    if (was == kNoVtx) {
+      const uint32_t u = atomicAdd(&T.count, 1u);
+      T.idx[s] = uint16_t(u);
+      T.slot[u] = uint16_t(s);
+      return s;
+    }
+    s = (s + 1u) & (kVtxSlots - 1u);
+  }
+}
+
+// The q-th of the n cells sharing the lattice edge from corner 0 of a cell
+// in direction dir, in increasing linear order (normal.c:78-158): the edge
+// starts at corner `lo` of that cell.  An axis edge is shared by four cells,
+// a face diagonal by two, the body diagonal belongs to one.
+__device__ __forceinline__ uint32_t sharing_corner(uint32_t dir, uint32_t q, uint32_t& n) {
+  const uint32_t free = 7u ^ dir, a = free & (0u - free), b = free & (free - 1u);
+  n = 1u << __popc(free);
+  const uint32_t back = n - 1u - q;
+  return (back & 1u ? a : 0u) | (back & 2u ? b : 0u);
+}
+
+// cell-local id of the edge from corner lo in direction dir (triangulate.c:23-32)
+__device__ __forceinline__ uint32_t edge_id_at(uint32_t lo, uint32_t dir) {
+  const uint32_t i = lo & 1u, j = (lo >> 1) & 1u, k = lo >> 2;
+  const uint32_t by_axis = dir == 1u ? lo >> 1 : dir == 2u ? 4u + i + 2u * k : 8u + (lo & 3u);
+  const uint32_t by_diag = dir == 6u ? 12u + i : dir == 5u ? 14u + j : dir == 3u ? 16u + k : 18u;
+  return dir == 1u || dir == 2u || dir == 4u ? by_axis : by_diag;
+}
+
+// Scratch of one wave forming vertex normals: the triangles found around
+// its 16 vertices (owner lane | slot << 6; an axis edge has at most 16, and
+// the diagonals fewer) and the smoothing weights of 64 of them.
+template <typename R>
+struct WaveHits {
+  uint16_t hit[256];
+  R w[64][3];
+};
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The winning triangle of one pixel, as phase 1 leaves it for phase 3.
+template <typename R>
+struct PixelTri {
+  bool tri;
+  uint32_t obj;
+  R w0, w1, w2;
+  uint32_t s[3];  // its vertices' slots
+};
+
+// barycentric weights at pixel (i, j) of a triangle with vertices p
+template <typename R>
+__device__ __forceinline__ void weights_at(const ViewDev<R>& v, const V3<R> p[3], int32_t i, int32_t j, PixelTri<R>& X) {
+  Projected<R> P;
 #pragma unroll
-      for (int n = 0; n < 8; n++) v2[n] = vc[n];
-    } else {
-      load_corners(f, L2, v2);
-    }
-    const uint32_t code = self ? code_c : corner_code(thr, v2);
-    uint32_t m = c_emask[code * 19u + want];
-    double g6[6] = {0, 0, 0, 0, 0, 0};
-    if (m && !f.cx) cell_grid(f, L2, g6);
-    for (; m; m &= m - 1u) {
-      const uint64_t ent = c_cslot[code * 12u + uint32_t(__builtin_ctz(m))];
-      V3<R> P[3];
-      slot_positions_reg<R>(f, L2, thr, ent, v2, g6, P);
-      sum = vadd(sum, smoothing_weight<R>(P));
-    }
-  }
-  return vunit(sum);
+  for (int n = 0; n < 3; n++) project(v, p[n], P.q[n]);
+  raster_box(v, P);
+  pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), X.w0, X.w1, X.w2);
 }
 
-// k_resolve for a frame without a stored mesh: the nearest triangle is
-// found from its id (FP64: the object, cell and slot fields of tri_id64;
-// FP32, a serial id: the object among the image's objects by base, the cell
-// from the stored cell index, the slot from the cell store's neighbouring
-// entries) and recomputed from its field.  The kernel is latency-bound (a
-// chain of dependent gathers per pixel), so occupancy pays: the FP32 form
-// runs at 4 waves per SIMD (128 VGPRs, a small spill), the FP64 form at 3.
+// A frame without a stored mesh: triangles are found from their ids (FP64:
+// the object, cell and slot fields of tri_id64; FP32, a serial id: the
+// object among the image's objects by base, the cell from the stored cell
+// index, the slot from the cell store's neighbouring entries) and
+// recomputed from the field.
 template <typename R>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 3 : 4)))
-void k_resolve_field(const TessJob* __restrict__ jobs, const uint32_t* __restrict__ cell,
-                     const RasterJob<R>* __restrict__ rjobs, int njobs, uint64_t npx_total,
-                     const ObjMeta* __restrict__ meta, int nobj, const uint8_t* __restrict__ frag_rgb,
-                     const FrameHdr* __restrict__ hdr, const uint64_t* __restrict__ key,
-                     const void* __restrict__ idv) {
-  (void)nobj;  // objects are found from the image's range (and, in FP64, the id)
-  // a frame whose triangles outgrew the cell store is rendered again: skip it
-  if (hdr->overflow & 1u) return;
-  const uint64_t ntri = hdr->ntri;
-  for (uint64_t p0 = uint64_t(blockIdx.x) * kThreads; p0 < npx_total; p0 += uint64_t(gridDim.x) * kThreads) {
-    int jb = 0;
-    if (njobs > 1) {
-      int lo = 0, hi = njobs - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (rjobs[mid].px0 <= p0) lo = mid;
-        else hi = mid - 1;
-      }
-      jb = lo;
-    }
-    const RasterJob<R>& J = rjobs[jb];
-    const ViewDev<R> v = J.v;
-    const uint64_t p = p0 + threadIdx.x;
-    const uint64_t lp = p - J.px0;
-    if (lp >= uint64_t(v.W) * uint64_t(v.H)) continue;
-    const int32_t j = int32_t(lp / uint64_t(v.W));
-    const int32_t i = int32_t(lp - uint64_t(j) * uint64_t(v.W));
-    const uint64_t k = key[p];
-    uint8_t r = J.bg[0], gg = J.bg[1], b = J.bg[2];
-    double dep;
-    // the winner: a triangle (its object, cell and slot) or a line fragment
-    bool tri = false, line = false;
-    uint32_t obj = 0, c = 0, sl = 0;
-    uint64_t fi = 0;
+struct FieldSource {
+  const TessJob* __restrict__ jobs;
+  const uint32_t* __restrict__ cell;
+  const ObjMeta* __restrict__ meta;
+  const void* __restrict__ idv;
+
+  // the winner at pixel p with key k: a triangle (obj, cell c, slot sl), a
+  // line fragment (fi) or neither
+  __device__ __forceinline__ void winner(const RasterJob<R>& J, uint64_t ntri, uint64_t p, uint64_t k, bool& tri,
+                                         bool& line, uint32_t& obj, uint32_t& c, uint32_t& sl, uint64_t& fi,
+                                         double& dep) const {
     if constexpr (sizeof(R) == 8) {
       // tri_id64: (object + 1) << 40 | cell << 4 | slot
       const uint64_t id = static_cast<const uint64_t*>(idv)[p];
@@ -1807,7 +1756,7 @@ void k_resolve_field(const TessJob* __restrict__ jobs, const uint32_t* __restric
           else hi = mid - 1;
         }
         obj = uint32_t(lo);
-        const ObjMeta& om = meta[lo];
+        const uint64_t base = meta[lo].base;
         c = cell[t];
         // Within an object the cells ascend with the serial position and
         // a cell has at most 12 triangles, so the slot of t is the number
@@ -1815,58 +1764,271 @@ void k_resolve_field(const TessJob* __restrict__ jobs, const uint32_t* __restric
         // same cell.  The 11 loads are independent and share one or two
         // lines.
 #pragma unroll
-        for (uint32_t d = 1; d < 12; d++) sl += t >= om.base + d && cell[t - d] == c ? 1u : 0u;
+        for (uint32_t d = 1; d < 12; d++) sl += t >= base + d && cell[t - d] == c ? 1u : 0u;
         // a position outside the object can only come from a damaged cell
         // store: such a pixel keeps the background
-        tri = t >= om.base && t - om.base < om.count;
+        tri = t >= base && t - base < meta[lo].count;
       }
     }
-    if (tri) {
-      const ObjMeta om = meta[obj];
-      const FieldDev f = jobs[om.job].f;
-      double thr = jobs[om.job].ts.thr[0];
-      for (uint32_t z = 1; z < kMaxThr; z++) thr = om.q == z ? jobs[om.job].ts.thr[z] : thr;
+  }
+
+  // phase 1 of the wave's pixels with a winning triangle (have)
+  __device__ __forceinline__ void triangle(const ViewDev<R>& v, bool have, uint32_t obj, uint32_t c, uint32_t sl,
+                                           int32_t i, int32_t j, VtxTable<R>& T, PixelTri<R>& X) const {
+    const uint32_t job = have ? meta[obj].job : 0u;
+    // one field pass of the wave's pixels at a time (usually all of them),
+    // so that its constants are scalars
+    for (uint64_t todo = __ballot(have); todo;) {
+      const uint32_t jb = uint32_t(__builtin_amdgcn_readlane(int(job), __builtin_ctzll(todo)));
+      const bool mine = have && job == jb;
+      todo &= ~__ballot(mine);
+      const FieldDev& f = jobs[jb].f;
       // a cell index outside the object's field or its interior, or a slot
       // outside its cell, can only come from a damaged id or cell store:
       // such a pixel keeps the background rather than read out of bounds
-      do {
-        if (c >= f.ncells) break;
-        const CellLoc L = locate(f, c);
-        if (!interior_cell(f, L)) break;
-        double cv[8];
-        load_corners(f, L, cv);
-        const uint32_t code = corner_code(thr, cv);
-        if (sl >= c_ntri[code]) break;
-        const uint64_t ent = c_cslot[code * 12u + sl];
-        V3<R> wpos[3];
-        slot_positions<R>(f, L, thr, ent, cv, wpos);
-        Projected<R> P;
+      if (!mine || c >= f.ncells) continue;
+      const double thr = jobs[jb].ts.thr[meta[obj].q & 3u];
+      const CellLoc L = locate(f, c);
+      if (!interior_cell(f, L)) continue;
+      double cv[8];
+      load_corners(f, L, cv);
+      const uint32_t code = corner_code(thr, cv);
+      if (sl >= c_ntri[code]) continue;
+      const uint32_t ent = uint32_t(c_cslot[code * 12u + sl]);
+      V3<R> wpos[3];
+      slot_positions<R>(f, L, thr, ent, cv, wpos);
+      weights_at(v, wpos, i, j, X);
 #pragma unroll
-        for (int n = 0; n < 3; n++) project(v, wpos[n], P.q[n]);
-        raster_box(v, P);
-        R w0, w1, w2;
-        pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2);
-        V3<R> nv[3];
-#pragma unroll 1
-        for (int n = 0; n < 3; n++)
-          nv[n] = vertex_normal_field<R>(f, thr, c, L, cv, code, uint32_t(ent >> (18 + 5 * n)) & 31u);
-        const V3<R> n = vunit(vadd(vscale(w0, nv[0]), vadd(vscale(w1, nv[1]), vscale(w2, nv[2]))));
-        const V3<R> light = {v.light[0], v.light[1], v.light[2]};
-        const R fct = fmax(R(0.15), fabs(vdot(n, light)));
-        r = uint8_t(fct * R(om.rgb[0]));
-        gg = uint8_t(fct * R(om.rgb[1]));
-        b = uint8_t(fct * R(om.rgb[2]));
-      } while (false);
-    } else if (line) {
-      r = frag_rgb[3 * fi + 0];
-      gg = frag_rgb[3 * fi + 1];
-      b = frag_rgb[3 * fi + 2];
+      for (int n = 0; n < 3; n++) {
+        const uint32_t a = (ent >> (6 * n)) & 7u, b = (ent >> (6 * n + 3)) & 7u;
+        X.s[n] = vtx_enter(T, vtx_key(obj, corner_cell(c, a & b, f.ncx, f.ncy), a ^ b));
+      }
+      X.obj = obj;
+      X.tri = true;
     }
-    const uint64_t o = (uint64_t(v.H - 1 - j) * uint64_t(v.W) + uint64_t(i)) * 3;
-    J.rgb[o + 0] = r;
-    J.rgb[o + 1] = gg;
-    J.rgb[o + 2] = b;
-    if (J.depth) J.depth[lp] = dep;
+  }
+
+  // Phase 2: the normals of the table's vertices, 16 a wave at a time.  Four
+  // lanes per vertex read the (at most four) cells sharing its edge and list
+  // the triangles with a vertex on it (c_emask), cell by cell and in slot
+  // order; the listed triangles are then recomputed 64 at a time, one per
+  // lane, and each vertex's first lane adds its own in list order, from +0,
+  // and normalises: the sums of vertex_normal over a stored mesh, bit for
+  // bit.  A lane that walked all of a vertex's cells and triangles itself
+  // had chains four times as long, and the wave ran as many rounds as its
+  // busiest lane.
+  __device__ __forceinline__ void normals(VtxTable<R>& T, WaveHits<R>* scratch) const {
+    const uint32_t lane = threadIdx.x & 63u, nv = T.count;
+    WaveHits<R>& S = scratch[threadIdx.x >> 6];
+    for (uint32_t u0 = (threadIdx.x >> 6) * 16u; u0 < nv; u0 += kThreads / 4u) {
+      const uint32_t u = u0 + (lane >> 2), q = lane & 3u;
+      const bool have = u < nv;
+      const unsigned long long key = have ? T.key[T.slot[u]] : 0ull;
+      const uint32_t obj = uint32_t(key >> 36), c = uint32_t(key >> 4), dir = uint32_t(key) & 7u;
+      const uint32_t job = have ? meta[obj].job : 0u, qt = have ? meta[obj].q & 3u : 0u;
+      // one field pass of the wave's vertices at a time (usually all of them)
+      for (uint64_t todo = __ballot(have); todo;) {
+        const uint32_t jb = uint32_t(__builtin_amdgcn_readlane(int(job), __builtin_ctzll(todo)));
+        const bool mine = have && job == jb;
+        todo &= ~__ballot(mine);
+        const FieldDev& f = jobs[jb].f;
+        uint32_t n, c2 = 0, mask = 0, code = 0;
+        const uint32_t lo = sharing_corner(dir, q, n);
+        if (mine && q < n) {
+          c2 = c - ((lo & 1u) + (lo & 2u ? f.ncx : 0u) + (lo & 4u ? f.ncx * f.ncy : 0u));
+          double v[8];
+          load_corners(f, locate(f, c2), v);
+          code = corner_code(jobs[jb].ts.thr[qt], v);
+          mask = c_emask[code * 19u + edge_id_at(lo, dir)];
+        }
+        // where each lane's triangles start in the wave's list
+        uint32_t end = uint32_t(__popc(mask));
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint32_t y = __shfl_up(end, d, 64);
+          if (lane >= uint32_t(d)) end += y;
+        }
+        uint32_t at = end - uint32_t(__popc(mask));
+        const uint32_t first = at, last = uint32_t(__shfl(int(end), int(lane | 3u)));
+        const uint32_t total = uint32_t(__builtin_amdgcn_readlane(int(end), 63));
+        for (; mask; mask &= mask - 1u) S.hit[at++] = uint16_t(lane | uint32_t(__builtin_ctz(mask)) << 6);
+        V3<R> sum = {R(0), R(0), R(0)};
+        for (uint32_t h0 = 0; h0 < total; h0 += 64u) {
+          wave_lds_fence();  // the list is written, and the last round's weights are added
+          const uint32_t h = h0 + lane;
+          const uint32_t e = S.hit[h < total ? h : total - 1u];
+          const uint32_t cc = uint32_t(__shfl(int(c2), int(e & 63u)));
+          const uint32_t cq = uint32_t(__shfl(int(code | qt << 8), int(e & 63u)));
+          const uint32_t ent = uint32_t(c_cslot[(cq & 255u) * 12u + (e >> 6)]);
+          V3<R> P[3];
+          slot_positions_mem<R>(f, locate(f, cc), jobs[jb].ts.thr[cq >> 8], ent, P);
+          const V3<R> w = smoothing_weight<R>(P);
+          S.w[lane][0] = w.x;
+          S.w[lane][1] = w.y;
+          S.w[lane][2] = w.z;
+          wave_lds_fence();
+          if (q == 0) {
+            const uint32_t a = first > h0 ? first - h0 : 0u, b = last < h0 + 64u ? last : h0 + 64u;
+            for (uint32_t g = a; h0 + g < b; g++) sum = vadd(sum, V3<R>{S.w[g][0], S.w[g][1], S.w[g][2]});
+          }
+        }
+        if (mine && q == 0) {
+          const V3<R> nrm = vunit(sum);
+          T.n[u][0] = nrm.x;
+          T.n[u][1] = nrm.y;
+          T.n[u][2] = nrm.z;
+        }
+        wave_lds_fence();
+      }
+    }
+  }
+};
+
+// A stored mesh: triangles by serial id, with their records.
+template <typename R>
+struct MeshSource {
+  MeshView<R> m;
+  const ObjMeta* __restrict__ meta;
+  int nobj;
+  const uint32_t* __restrict__ idbuf;
+
+  __device__ __forceinline__ void winner(const RasterJob<R>&, uint64_t ntri, uint64_t p, uint64_t k, bool& tri,
+                                         bool& line, uint32_t& obj, uint32_t& c, uint32_t& sl, uint64_t& fi,
+                                         double& dep) const {
+    uint32_t id;
+    if constexpr (sizeof(R) == 8) {
+      id = idbuf[p];
+      dep = unord64(k);
+    } else {
+      id = uint32_t(k);
+      dep = id ? double(unord32(uint32_t(k >> 32))) : -DBL_MAX;
+    }
+    line = id > ntri;
+    fi = id - ntri - 1;
+    tri = id != 0 && !line;
+    c = id - 1u;  // the serial position
+    sl = 0;
+    if (tri) {
+      int lo = 0, hi = nobj - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (meta[mid].base <= c) lo = mid;
+        else hi = mid - 1;
+      }
+      obj = uint32_t(lo);
+    }
+  }
+
+  __device__ __forceinline__ void triangle(const ViewDev<R>& v, bool have, uint32_t obj, uint32_t t, uint32_t,
+                                           int32_t i, int32_t j, VtxTable<R>& T, PixelTri<R>& X) const {
+    if (!have) return;
+    V3<R> p[3];
+#pragma unroll
+    for (int n = 0; n < 3; n++)
+      p[n] = {m.pos[t].p[3 * n + 0], m.pos[t].p[3 * n + 1], m.pos[t].p[3 * n + 2]};
+    weights_at(v, p, i, j, X);
+    const uint32_t c = m.aux[t].cell, ed = edges_of(m, t);
+    const uint32_t ncx = meta[obj].ncx, ncy = meta[obj].ncy;
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+      uint32_t lo, dir;
+      edge_lo_dir((ed >> (5 * n)) & 31u, lo, dir);
+      X.s[n] = vtx_enter(T, vtx_key(obj, corner_cell(c, lo, ncx, ncy), dir));
+    }
+    X.obj = obj;
+    X.tri = true;
+  }
+
+  __device__ __forceinline__ void normals(VtxTable<R>& T, WaveHits<R>*) const {
+    for (uint32_t u = threadIdx.x; u < T.count; u += kThreads) {
+      const unsigned long long key = T.key[T.slot[u]];
+      const V3<R> n = vertex_normal<R>(m, meta[uint32_t(key >> 36)], uint32_t(key >> 4),
+                                       edge_id_at(0u, uint32_t(key) & 7u));
+      T.n[u][0] = n.x;
+      T.n[u][1] = n.y;
+      T.n[u][2] = n.z;
+    }
+  }
+};
+
+template <typename R, typename Source>
+__device__ __forceinline__ void resolve_tile(const Source& src, VtxTable<R>& T, WaveHits<R>* hits,
+                                             const RasterJob<R>* __restrict__ rjobs, int njobs, uint32_t frame_tile,
+                                             const uint8_t* __restrict__ frag_rgb, uint64_t ntri,
+                                             const uint64_t* __restrict__ key) {
+  // the image of this tile
+  int jb = 0;
+  for (int hi = njobs - 1; jb < hi;) {
+    const int mid = (jb + hi + 1) >> 1;
+    if (rjobs[mid].tile0 <= frame_tile) jb = mid;
+    else hi = mid - 1;
+  }
+  const RasterJob<R>& J = rjobs[jb];
+  const ViewDev<R> v = J.v;
+  const uint32_t tile = frame_tile - J.tile0, tw = (uint32_t(v.W) + kTileW - 1u) / kTileW;
+  const uint32_t ty = tile / tw;
+  const int32_t i = int32_t((tile - ty * tw) * kTileW + threadIdx.x % kTileW);
+  const int32_t j = int32_t(ty * kTileH + threadIdx.x / kTileW);
+  const bool inside = i < v.W && j < v.H;
+  const uint64_t lp = uint64_t(j) * uint64_t(v.W) + uint64_t(i);
+
+  bool tri = false, line = false;
+  uint32_t obj = 0, c = 0, sl = 0;
+  uint64_t fi = 0;
+  double dep = 0;
+  if (inside) src.winner(J, ntri, J.px0 + lp, key[J.px0 + lp], tri, line, obj, c, sl, fi, dep);
+  PixelTri<R> X;
+  X.tri = false;
+  // a tile of background and lines has no vertices
+  if (__syncthreads_or(tri)) {
+    for (uint32_t s = threadIdx.x; s < kVtxSlots; s += kThreads) T.key[s] = kNoVtx;
+    if (threadIdx.x == 0) T.count = 0;
+    __syncthreads();
+    src.triangle(v, tri, obj, c, sl, i, j, T, X);
+    __syncthreads();
+    src.normals(T, hits);
+    __syncthreads();
+  }
+  if (!inside) return;
+  uint8_t r = J.bg[0], gg = J.bg[1], b = J.bg[2];
+  if (X.tri) {
+    V3<R> nv3[3];
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+      const R* q = T.n[T.idx[X.s[n]]];
+      nv3[n] = {q[0], q[1], q[2]};
+    }
+    const V3<R> n = vunit(vadd(vscale(X.w0, nv3[0]), vadd(vscale(X.w1, nv3[1]), vscale(X.w2, nv3[2]))));
+    const V3<R> light = {v.light[0], v.light[1], v.light[2]};
+    const R fct = fmax(R(0.15), fabs(vdot(n, light)));
+    const uint8_t* rgb = src.meta[X.obj].rgb;
+    r = uint8_t(fct * R(rgb[0]));
+    gg = uint8_t(fct * R(rgb[1]));
+    b = uint8_t(fct * R(rgb[2]));
+  } else if (line) {
+    r = frag_rgb[3 * fi + 0];
+    gg = frag_rgb[3 * fi + 1];
+    b = frag_rgb[3 * fi + 2];
+  }
+  const uint64_t o = (uint64_t(v.H - 1 - j) * uint64_t(v.W) + uint64_t(i)) * 3;
+  J.rgb[o + 0] = r;
+  J.rgb[o + 1] = gg;
+  J.rgb[o + 2] = b;
+  if (J.depth) J.depth[lp] = dep;
+}
+
+// Occupancy: the FP64 table and scratch (38 KB) allow four workgroups per CU.
+template <typename R, typename Source>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_resolve(
+    Source src, const RasterJob<R>* __restrict__ rjobs, int njobs, uint32_t ntiles,
+    const uint8_t* __restrict__ frag_rgb, const FrameHdr* __restrict__ hdr, const uint64_t* __restrict__ key) {
+  // a frame whose triangles outgrew the cell store is rendered again: skip it
+  if (hdr->overflow & 1u) return;
+  __shared__ VtxTable<R> T;
+  __shared__ WaveHits<R> hits[kThreads / 64];
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    resolve_tile(src, T, hits, rjobs, njobs, tile, frag_rgb, hdr->ntri, key);
+    __syncthreads();  // the next tile reuses the table
   }
 }
 
@@ -2004,12 +2166,20 @@ hipError_t launch_line_frags(const uint32_t* pix, const double* depth, uint32_t 
   return hipGetLastError();
 }
 
+uint32_t resolve_tiles(uint64_t W, uint64_t H) {
+  return uint32_t((W + kTileW - 1) / kTileW * ((H + kTileH - 1) / kTileH));
+}
+
+// a workgroup per tile (the kernel strides past 2^23 of them)
+static dim3 resolve_grid(uint32_t ntiles) { return dim3(ntiles < (1u << 23) ? ntiles : (1u << 23)); }
+
 template <typename R>
-hipError_t launch_resolve(const MeshView<R>& m, const RasterJob<R>* rjobs, int njobs, uint64_t npx_total,
+hipError_t launch_resolve(const MeshView<R>& m, const RasterJob<R>* rjobs, int njobs, uint32_t ntiles,
                           const ObjMeta* meta, int nobj, const uint8_t* frag_rgb, const FrameHdr* hdr,
-                          const uint64_t* key, const uint32_t* id, uint32_t grid, hipStream_t st) {
-  hipLaunchKernelGGL(k_resolve<R>, dim3(grid8((npx_total + kThreads - 1) / kThreads, grid)), dim3(kThreads), 0, st,
-                     m, rjobs, njobs, npx_total, meta, nobj, frag_rgb, hdr, key, id);
+                          const uint64_t* key, const uint32_t* id, hipStream_t st) {
+  const MeshSource<R> src = {m, meta, nobj, id};
+  hipLaunchKernelGGL((k_resolve<R, MeshSource<R>>), resolve_grid(ntiles), dim3(kThreads), 0, st, src, rjobs, njobs,
+                     ntiles, frag_rgb, hdr, key);
   return hipGetLastError();
 }
 
@@ -2054,10 +2224,11 @@ hipError_t launch_tess_raster(const TessJob* jobs, int njobs, uint32_t nitems, c
 
 template <typename R>
 hipError_t launch_resolve_field(const TessJob* jobs, const uint32_t* cell, const RasterJob<R>* rjobs, int njobs,
-                                uint64_t npx_total, const ObjMeta* meta, int nobj, const uint8_t* frag_rgb,
-                                const FrameHdr* hdr, const uint64_t* key, const void* id, hipStream_t st) {
-  hipLaunchKernelGGL(k_resolve_field<R>, dim3(grid8((npx_total + kThreads - 1) / kThreads, 1u << 30)), dim3(kThreads),
-                     0, st, jobs, cell, rjobs, njobs, npx_total, meta, nobj, frag_rgb, hdr, key, id);
+                                uint32_t ntiles, const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr,
+                                const uint64_t* key, const void* id, hipStream_t st) {
+  const FieldSource<R> src = {jobs, cell, meta, id};
+  hipLaunchKernelGGL((k_resolve<R, FieldSource<R>>), resolve_grid(ntiles), dim3(kThreads), 0, st, src, rjobs, njobs,
+                     ntiles, frag_rgb, hdr, key);
   return hipGetLastError();
 }
 
@@ -2067,12 +2238,12 @@ template hipError_t launch_tess_raster<double>(const TessJob*, int, uint32_t, co
 template hipError_t launch_tess_raster<float>(const TessJob*, int, uint32_t, const uint64_t*, uint32_t*, uint64_t,
                                               const RasterJob<float>*, const uint32_t*, FrameHdr*, int, uint64_t*,
                                               void*, void*, uint32_t, uint32_t, hipStream_t);
-template hipError_t launch_resolve_field<double>(const TessJob*, const uint32_t*, const RasterJob<double>*, int,
-                                                 uint64_t, const ObjMeta*, int, const uint8_t*, const FrameHdr*,
-                                                 const uint64_t*, const void*, hipStream_t);
-template hipError_t launch_resolve_field<float>(const TessJob*, const uint32_t*, const RasterJob<float>*, int,
-                                                uint64_t, const ObjMeta*, int, const uint8_t*, const FrameHdr*,
-                                                const uint64_t*, const void*, hipStream_t);
+template hipError_t launch_resolve_field<double>(const TessJob*, const uint32_t*, const RasterJob<double>*, int, uint32_t,
+                                                 const ObjMeta*, const uint8_t*, const FrameHdr*, const uint64_t*,
+                                                 const void*, hipStream_t);
+template hipError_t launch_resolve_field<float>(const TessJob*, const uint32_t*, const RasterJob<float>*, int, uint32_t,
+                                                 const ObjMeta*, const uint8_t*, const FrameHdr*, const uint64_t*,
+                                                 const void*, hipStream_t);
 template hipError_t launch_plan<double>(const uint64_t*, uint64_t, ObjMeta*, int, RasterJob<double>*, int, FrameHdr*,
                                         uint64_t, hipStream_t);
 template hipError_t launch_plan<float>(const uint64_t*, uint64_t, ObjMeta*, int, RasterJob<float>*, int, FrameHdr*,
@@ -2089,12 +2260,12 @@ template hipError_t launch_raster<double>(const MeshView<double>&, const RasterJ
                                           uint64_t*, uint32_t*, Frag*, uint32_t, uint32_t, hipStream_t);
 template hipError_t launch_raster<float>(const MeshView<float>&, const RasterJob<float>*, int, FrameHdr*, int,
                                          uint64_t*, uint32_t*, Frag*, uint32_t, uint32_t, hipStream_t);
-template hipError_t launch_resolve<double>(const MeshView<double>&, const RasterJob<double>*, int, uint64_t,
+template hipError_t launch_resolve<double>(const MeshView<double>&, const RasterJob<double>*, int, uint32_t,
                                            const ObjMeta*, int, const uint8_t*, const FrameHdr*, const uint64_t*,
-                                           const uint32_t*, uint32_t, hipStream_t);
-template hipError_t launch_resolve<float>(const MeshView<float>&, const RasterJob<float>*, int, uint64_t,
-                                          const ObjMeta*, int, const uint8_t*, const FrameHdr*, const uint64_t*,
-                                          const uint32_t*, uint32_t, hipStream_t);
+                                           const uint32_t*, hipStream_t);
+template hipError_t launch_resolve<float>(const MeshView<float>&, const RasterJob<float>*, int, uint32_t,
+                                           const ObjMeta*, int, const uint8_t*, const FrameHdr*, const uint64_t*,
+                                           const uint32_t*, hipStream_t);
 
 hipError_t upload_tables(const NbrTable& nt) {
   // case table of triangulate.c:204-270: reduced mask -> triangles as
