@@ -79,10 +79,75 @@ uint64_t next_buf_gen() {
   return ++g;
 }
 
+// Device blocks of freed meshes, kept for the next mesh: a mesh is built,
+// read and freed again and again (a surface per time step), and at 256^3 and
+// two thresholds the driver took 42 ms to allocate and free what the kernels
+// fill in 1.8 ms.  At most kPoolBytes are held (one FP64 mesh of 512^3 and
+// three thresholds takes 18 GB); the oldest go first, an allocation that
+// fails empties the pool and tries again, and contour3d_amd_finalize gives
+// everything back.  Blocks come here only after the device is done with
+// them, so any stream may take them.
+constexpr size_t kPoolBytes = size_t(24) << 30;
+
+struct BlockPool {
+  struct Block {
+    void* p;
+    size_t bytes;
+  };
+  std::mutex mu;
+  std::vector<Block> blocks;  // oldest first
+  size_t held = 0;
+  // the smallest block of at least `want` bytes that is not more than twice
+  // that (small requests: 64 KiB more)
+  void* take(size_t want, size_t& got) {
+    std::lock_guard<std::mutex> g(mu);
+    size_t best = blocks.size();
+    for (size_t q = 0; q < blocks.size(); q++)
+      if (blocks[q].bytes >= want && blocks[q].bytes <= 2 * want + 65536 &&
+          (best == blocks.size() || blocks[q].bytes < blocks[best].bytes))
+        best = q;
+    if (best == blocks.size()) return nullptr;
+    void* p = blocks[best].p;
+    got = blocks[best].bytes;
+    held -= got;
+    blocks.erase(blocks.begin() + std::ptrdiff_t(best));
+    return p;
+  }
+  void give(void* p, size_t bytes) {
+    std::lock_guard<std::mutex> g(mu);
+    if (bytes > kPoolBytes) {
+      (void)hipFree(p);
+      return;
+    }
+    while (held + bytes > kPoolBytes) {
+      held -= blocks.front().bytes;
+      (void)hipFree(blocks.front().p);
+      blocks.erase(blocks.begin());
+    }
+    blocks.push_back({p, bytes});
+    held += bytes;
+  }
+  // frees every block; false if there was none
+  bool drop() {
+    std::lock_guard<std::mutex> g(mu);
+    const bool any = !blocks.empty();
+    for (const Block& b : blocks) (void)hipFree(b.p);
+    blocks.clear();
+    held = 0;
+    return any;
+  }
+};
+
+BlockPool& block_pool() {
+  static BlockPool p;
+  return p;
+}
+
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
   bool fixed = false;
+  bool pooled = false;  // a stored mesh's buffer: its blocks come from and go to the pool
   uint64_t gen = 0;  // the current allocation's number (0: none)
   ~DevBuf() = default;
   // grows to at least `want` bytes, with a quarter of headroom unless
@@ -98,8 +163,17 @@ struct DevBuf {
       if (e != hipSuccess) return e;
     }
     size_t n = exact ? want : want + want / 4 + 256;
+    if (pooled && (p = block_pool().take(n, n))) {
+      bytes = n;
+      gen = next_buf_gen();
+      return hipSuccess;
+    }
     if (injected_alloc_failure()) return hipErrorOutOfMemory;
     hipError_t e = hipMalloc(&p, n);
+    if (e == hipErrorOutOfMemory && block_pool().drop()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, n);
+    }
     if (e != hipSuccess) {
       p = nullptr;
       gen = 0;
@@ -111,7 +185,8 @@ struct DevBuf {
   }
   void release() {
     if (fixed) return;  // the scratch array lives as long as the process
-    if (p) (void)hipFree(p);
+    if (p && pooled) block_pool().give(p, bytes);
+    else if (p) (void)hipFree(p);
     p = nullptr;
     bytes = 0;
     gen = 0;
@@ -214,6 +289,11 @@ struct contour3d_amd_mesh {
   std::vector<uint32_t> tiles;  // tiles of each object's field
   std::vector<c3d::TileGeo> geo;  // and their layout
   std::vector<contour3d_color_t> color;
+  // a stored mesh: its buffers come from and go to the block pool, so
+  // release() needs the device to be done with them
+  void use_pool() {
+    for (c3d::DevBuf* b : {&pos, &aux, &bstart, &meta, &code, &cstart}) b->pooled = true;
+  }
   void release() {
     pos.release();
     aux.release();
@@ -1966,7 +2046,11 @@ void* snap_take(Server& S, size_t bytes, size_t& got) {
     }
   }
   void* p = nullptr;
-  if (injected_alloc_failure() || hipMalloc(&p, bytes) != hipSuccess || !p) return nullptr;
+  if (injected_alloc_failure()) return nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess || !p) {
+    (void)hipGetLastError();
+    if (!block_pool().drop() || hipMalloc(&p, bytes) != hipSuccess || !p) return nullptr;
+  }
   std::lock_guard<std::mutex> g(S.pool_mu);
   S.snap_all.push_back({p, bytes});
   S.snap_held += bytes;
@@ -2317,6 +2401,7 @@ int contour3d_amd_finalize(void) {
   L.geoms.clear();
   L.main.release();
   L.scratch_frame.release();
+  (void)c3d::block_pool().drop();
   L.ready = false;
   return 0;
 }
@@ -2499,12 +2584,14 @@ int contour3d_amd_mesh_build(const contour3d_contour_obj_t* contour_objs, size_t
   std::lock_guard<std::mutex> g(L.mu);
   if (c3d::ensure_init(L, 0)) return 1;
   auto M = std::make_unique<contour3d_amd_mesh>();
+  M->use_pool();
   const int rc = c3d::build_mesh(L, L.main, *M, contour_objs, num_contours, precision);
   const hipError_t e = hipStreamSynchronize(L.main.st);
   c3d::release_geoms(L.main);
   if (rc || e != hipSuccess) {
     if (!rc) c3d::log_error("mesh build failed on the device");
-    M->release();  // a failed build keeps no device memory
+    M->release();
+    (void)c3d::block_pool().drop();  // a failed build keeps no device memory
     return 1;
   }
   if (c3d::prof_collect(L.main)) return 1;
