@@ -236,6 +236,7 @@ struct Geom {
   uint64_t hash = 0;
   std::vector<double> host;  // the grid values (nx + ny + nz), compared on a hash match
   bool identity = true;
+  bool ordered = false;  // every grid finite and monotonic: a range of cells lies between its ends
   DevBuf grids;  // nx + ny + nz doubles
   DevBuf table;  // 3 * npts doubles when not the identity
   uint64_t stamp = 0;
@@ -273,7 +274,6 @@ struct contour3d_amd_mesh {
   int precision_built = -1;  // form the buffers were sized for
   c3d::DevBuf pos;     // a stored mesh: cap position records (c3d::MeshPos)
   c3d::DevBuf aux;     // and cap gather records (c3d::MeshAux)
-  c3d::DevBuf cell;    // a frame: the cell index of each triangle (cap entries)
   c3d::DevBuf bstart;  // per-tile triangle starts of every object's field
   c3d::DevBuf meta;    // ObjMeta per object
   c3d::DevBuf code;    // a stored mesh: the corner code of every cell of every object (ObjMeta::code_off)
@@ -297,7 +297,6 @@ struct contour3d_amd_mesh {
   void release() {
     pos.release();
     aux.release();
-    cell.release();
     bstart.release();
     meta.release();
     code.release();
@@ -310,15 +309,17 @@ struct contour3d_amd_mesh {
 namespace c3d {
 namespace {
 
-// initial fragment-list entries of an FP64 frame (24 B each; 16 B for a
-// stored mesh): every covered pixel of a 512^3 field's frame at 1920x1080
-// fits
+// initial fragment-list entries of a frame (24 B each; 16 B for a stored
+// FP64 mesh): every fragment of a 512^3 field's frame at 1920x1080 that
+// passes the z-test as it is drawn fits
 constexpr uint32_t kDefaultFragCap = 1u << 24;
 
 // Host-side layout of a frame's tessellation.
 struct TessLayout {
-  uint64_t nbt = 0;  // tile-count entries (the objects' tiles)
-  uint32_t ntj = 0;  // work items of the field passes
+  uint64_t nbt = 0;  // a stored mesh: tile-count entries (the objects' tiles)
+  uint32_t ntj = 0;  // a stored mesh: work items of the field passes
+  uint32_t ngroups = 0;  // a frame: groups of bricks of the field passes
+  uint32_t shift = 0;    // and the log2 of a group's bricks per axis
   int njobs = 0;     // field passes
   int nobj = 0;
 };
@@ -346,7 +347,7 @@ struct Frame {
   bool noalloc = false;
   DevBuf grids;
   std::vector<std::unique_ptr<DevBuf>> uploads;
-  DevBuf cnt, tiles, tjobs, rjobs, hdr, jimg;
+  DevBuf cnt, tiles, tjobs, rjobs, hdr, jimg, order, take;
   DevBuf key, id, rgb, depth, fpix, fdep, frgb, frags, vntmp;
   uint32_t frag_cap = 0;
   HostBuf hrgb, hstage;
@@ -375,7 +376,7 @@ struct Frame {
   Prof prof;
   bool fp64 = true;         // form of the frame in flight
   FrameHdr last{};          // header of the last finished frame
-  bool unread = false;      // the frame in flight was planned with no read back of its totals
+  bool drawn = false;       // the frame in flight has no stored mesh: its triangle total comes with its header
   template <typename R>
   std::vector<RasterJob<R>>& rjobs_host();
   hipError_t create() {
@@ -387,7 +388,7 @@ struct Frame {
     if (st) (void)hipStreamSynchronize(st);
     for (auto& u : uploads) u->release();
     uploads.clear();
-    DevBuf* bufs[] = {&cnt,  &tiles, &tjobs, &rjobs, &hdr,  &jimg, &key,  &id,   &rgb,
+    DevBuf* bufs[] = {&cnt,   &tiles, &tjobs, &rjobs, &hdr, &jimg, &order, &take, &key, &id, &rgb,
                       &depth, &fpix, &fdep,  &frgb, &frags, &vntmp, &grids};
     for (auto* b : bufs) b->release();
     mesh.release();
@@ -435,14 +436,18 @@ struct Lib {
   uint32_t tess_rows = 0;
   uint32_t tess_zc = 0;
   bool graphs = false;  // replay captured launch sequences of repeated frame layouts
-  // Tessellation launches are persistent: by default 128 workgroups per CU,
-  // each walking several tiles, so that its triangle queue carries items
-  // across tiles and drains part-full once, at its end (measured at 512^3:
-  // the fused stage 5.6 -> 5.3 ms against one workgroup per tile)
+  // workgroups of the count and emit kernels: persistent, by default 128 per
+  // CU, each walking several tiles
   uint32_t tess_grid(uint32_t nitems) const {
     const uint32_t cap = tess_cap ? tess_cap : uint32_t(persistent_blocks()) * 16u;
     const uint32_t g = cap < nitems ? cap : nitems;
     return g < 8 ? 8 : g;
+  }
+  // workgroups of a frame's draw: as many as are resident at once (they take
+  // their bricks one by one)
+  uint32_t frame_grid() const {
+    const uint32_t g = uint32_t(persistent_blocks()) / 8u * 6u;
+    return tess_cap && tess_cap < g ? tess_cap : g;
   }
   Frame main;
   Frame scratch_frame;  // the allocation-free entry point's frame
@@ -455,17 +460,19 @@ Lib& lib() {
 }
 
 // Limits of the allocation-free frame (the regions of the scratch array).
-constexpr uint64_t kScratchTiles = uint64_t(1) << 20;      // tile-count entries of all objects
+constexpr uint64_t kScratchTiles = uint64_t(1) << 20;      // tessellation tiles of all objects, and groups of bricks
 constexpr uint32_t kScratchObjs = 64;                      // contour objects
 constexpr uint64_t kScratchPixels = uint64_t(1) << 21;     // z-buffer entries (1920x1080 fits)
-constexpr uint32_t kScratchFrags = 1u << 19;               // fragment list entries
+constexpr uint32_t kScratchFrags = 3u << 20;               // fragment list entries
 constexpr uint64_t kScratchLineFrags = uint64_t(1) << 18;  // line fragments
-constexpr uint64_t kScratchTriangles = uint64_t(1) << 24;  // cell store entries
+constexpr uint64_t kScratchTriangles = uint64_t(1) << 24;  // triangles of an FP32 frame
 constexpr uint64_t kScratchGridValues = uint64_t(1) << 16; // lattice coordinates of all objects
 
 // per device: the scratch array's address there (taken at set-up)
 constexpr int kMaxDevices = 64;
 void* g_scratch[kMaxDevices] = {};
+
+constexpr size_t kTakeBytes = 16 * 64 * sizeof(uint32_t);  // a frame's brick counters (launch_frame_begin)
 
 // Takes the scratch array's address on the current device and cuts it into
 // the buffers of the allocation-free frame F.
@@ -491,9 +498,9 @@ int carve_scratch(Frame& F, int device) {
     off += (bytes + 255) / 256 * 256;
   };
   contour3d_amd_mesh& M = F.mesh;
-  region(F.cnt, (kScratchTiles + 1) * sizeof(uint32_t));
-  region(M.bstart, (kScratchTiles + 1) * sizeof(uint64_t));
-  region(F.tiles, ((kScratchTiles + kScanTile - 1) / kScanTile + 1) * sizeof(uint64_t));
+  region(F.order, kScratchTiles * sizeof(uint2));
+  region(F.take, kTakeBytes);
+  region(M.bstart, 0);
   region(F.tjobs, (kScratchObjs + 1) * sizeof(TessJob));
   region(M.meta, (kScratchObjs + 1) * sizeof(ObjMeta));
   region(F.hdr, sizeof(FrameHdr));
@@ -505,7 +512,6 @@ int carve_scratch(Frame& F, int device) {
   region(F.fdep, (kScratchLineFrags + 1) * sizeof(double));
   region(F.frgb, 3 * (kScratchLineFrags + 1));
   region(F.frags, size_t(kScratchFrags) * sizeof(Frag64));
-  region(M.cell, kScratchTriangles * sizeof(uint32_t));
   region(F.grids, kScratchGridValues * sizeof(double));
   region(F.rgb, 0);
   region(F.depth, 0);
@@ -658,6 +664,19 @@ using ConvFn = contour3d_vector_t (*)(const contour3d_vector_t);
 // (triangulate.c:165-170); it is evaluated once per point and the result
 // cached for as long as the converter, grid pointers and grid values stay
 // the same.  A map that returns every point unchanged needs no table.
+// whether the values are finite and never turn back
+bool ordered_grid(const double* g, size_t n) {
+  bool up = true, down = true, fin = true;
+  for (size_t q = 0; q < n; q++) {
+    fin = fin && std::isfinite(g[q]);
+    if (q) {
+      up = up && g[q] >= g[q - 1];
+      down = down && g[q] <= g[q - 1];
+    }
+  }
+  return fin && (up || down);
+}
+
 int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
   const size_t nx = o.glsizes[0], ny = o.glsizes[1], nz = o.glsizes[2];
   std::vector<double> hg[3];
@@ -710,6 +729,7 @@ int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
   C3D_HIP(hipMemcpy(g->grids.as<double>() + nx, gp[1], ny * sizeof(double), hipMemcpyHostToDevice));
   C3D_HIP(hipMemcpy(g->grids.as<double>() + nx + ny, gp[2], nz * sizeof(double), hipMemcpyHostToDevice));
   g->identity = true;
+  g->ordered = ordered_grid(gp[0], nx) && ordered_grid(gp[1], ny) && ordered_grid(gp[2], nz);
   if (o.converter != contour3d_amd_identity) {
     const ConvFn conv = o.converter;
     const size_t npts = nx * ny * nz;
@@ -863,6 +883,7 @@ ViewDev<R> dev_view(const HostView& h) {
   v.fw = R(double(h.W));
   v.fh = R(double(h.H));
   set_pitch(v);
+  set_cv(v);
   v.W = int32_t(h.W);
   v.H = int32_t(h.H);
   return v;
@@ -969,15 +990,14 @@ bool same_obj(const contour3d_contour_obj_t& a, const contour3d_contour_obj_t& b
          a.color.g == b.color.g && a.color.b == b.color.b;
 }
 
-// A frame keeps only the cell index of each triangle (the fused raster
-// draws triangles from registers): 1.25x the triangles seen.
 // Copies n bytes of host memory to device buffer b at byte offset off on
 // F's stream, unless the same bytes were the last ones copied there and b
 // has not been reallocated since: a repeated frame then sends only the
 // tables that changed (each small copy from pageable memory costs about
 // 12 us of host time, and the device waits for it).  Kernels may rewrite
-// parts of an uploaded table (k_plan: objects' bases and counts, images'
-// triangle ranges) only where every frame that reads them rewrites them.
+// parts of an uploaded table (a stored mesh's k_plan: objects' bases and
+// counts, images' triangle ranges) only where every frame that reads them
+// rewrites them.
 int upload_table(Frame& F, DevBuf& b, size_t off, const void* src, size_t n) {
   if (n == 0) return 0;
   UploadMemo& m = F.memo[{static_cast<const void*>(&b), off}];
@@ -991,15 +1011,6 @@ int upload_table(Frame& F, DevBuf& b, size_t off, const void* src, size_t n) {
 
 // forgets what upload_table last sent to (b, off): something else wrote it
 void forget_table(Frame& F, const DevBuf& b, size_t off) { F.memo.erase({static_cast<const void*>(&b), off}); }
-
-int ensure_cells(contour3d_amd_mesh& M) {
-  if (M.cap >= M.total && M.cap != 0 && M.cell.p) return 0;
-  const uint64_t cap = M.total + M.total / 4 + 1024;
-  M.cap = 0;
-  C3D_HIP(M.cell.ensure(cap * sizeof(uint32_t), true));
-  M.cap = cap;
-  return 0;
-}
 
 template <typename R>
 int ensure_capacity(contour3d_amd_mesh& M) {
@@ -1017,12 +1028,21 @@ int ensure_capacity(contour3d_amd_mesh& M) {
   return 0;
 }
 
-// Host half of a frame's tessellation: validates the objects, resolves
+// Cells from which a frame's bricks get `planes` planes: fewer planes make
+// more bricks, and a small lattice needs them to fill the device.
+uint32_t brick_planes(uint64_t cells) {
+  uint32_t planes = kBrickPlanes;
+  while (planes > 1 && cells / (uint64_t(kBrickColumns) * planes) < 5120) planes /= 2;
+  return planes;
+}
+
+// Host half of a frame's tessellation (or, with `stored`, a mesh's): validates the objects, resolves
 // fields (host fields are uploaded) and lattices, groups thresholds of a
 // shared field into field passes, sizes the buffers and enqueues the uploads
 // of the pass and object tables.  The layout goes to F.tl.
 template <typename R>
-int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<const contour3d_contour_obj_t*>& objs) {
+int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<const contour3d_contour_obj_t*>& objs,
+                 bool stored) {
   const size_t n = objs.size();
   if (F.noalloc && n > F.tjobs.bytes / sizeof(TessJob) - 1) {
     log_error("the allocation-free call takes at most %zu contour objects", F.tjobs.bytes / sizeof(TessJob) - 1);
@@ -1107,6 +1127,9 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
       f.gy = f.gx + f.nx;
       f.gz = f.gy + f.ny;
       f.cx = f.cy = f.cz = nullptr;
+      f.ordered = 1;
+      for (int d = 0; d < 3; d++)
+        if (is_device_ptr(ob.grids[d]) || !ordered_grid(ob.grids[d], ob.glsizes[d])) f.ordered = 0;
     } else if (on_dev[o]) {
       f.f = ob.array;
     } else {
@@ -1135,6 +1158,7 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
       f.gy = f.gx + f.nx;
       f.gz = f.gy + f.ny;
       if (g->identity) {
+        f.ordered = g->ordered;
         f.cx = f.cy = f.cz = nullptr;
       } else {
         const size_t npts = size_t(f.nx) * f.ny * f.nz;
@@ -1156,9 +1180,9 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
     if (group[o] < 0) group[o] = int(o);
   }
   const uint64_t nbt = boff[n];
-  if (F.noalloc && nbt + 1 > F.cnt.bytes / sizeof(uint32_t)) {
-    log_error("the allocation-free call holds at most %zu tessellation tiles; the objects need %llu",
-              F.cnt.bytes / sizeof(uint32_t) - 1, (unsigned long long)nbt);
+  if (F.noalloc && nbt > kScratchTiles) {
+    log_error("the allocation-free call holds at most %llu tessellation tiles; the objects need %llu",
+              (unsigned long long)kScratchTiles, (unsigned long long)nbt);
     return 1;
   }
   M.precision = sizeof(R) == 8 ? CONTOUR3D_AMD_FP64 : CONTOUR3D_AMD_FP32;
@@ -1223,9 +1247,40 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
   M.code_bytes = codes;  // a stored mesh keeps every cell's corner code
   M.starts_ready = false;
 
-  C3D_HIP(F.cnt.ensure((nbt + 1) * sizeof(uint32_t)));
-  C3D_HIP(M.bstart.ensure((nbt + 1) * sizeof(uint64_t)));
-  C3D_HIP(F.tiles.ensure(((nbt + kScanTile - 1) / kScanTile + 1) * sizeof(uint64_t)));
+  if (stored) {
+    C3D_HIP(F.cnt.ensure((nbt + 1) * sizeof(uint32_t)));
+    C3D_HIP(M.bstart.ensure((nbt + 1) * sizeof(uint64_t)));
+    C3D_HIP(F.tiles.ensure(((nbt + kScanTile - 1) / kScanTile + 1) * sizeof(uint64_t)));
+  } else {
+    // bricks, in groups of 4^3 once there are enough of them to order and
+    // share out, of 2^3 below
+    uint64_t cells = 0;
+    for (const TessJob& j : tj) cells += uint64_t(j.f.ncx) * j.f.ncy * j.f.ncz;
+    uint32_t rows = L.tess_rows, planes = L.tess_zc ? L.tess_zc : brick_planes(cells);
+    F.tl.shift = cells / (uint64_t(kBrickColumns) * kBrickPlanes) >= 65536 ? 2 : 1;
+    uint64_t ng = 0;
+    for (int attempt = 0; attempt < 2; attempt++) {
+      ng = 0;
+      for (TessJob& j : tj) {
+        j.bg = make_brick_geo(j.f.ncx, j.f.ncy, j.f.ncz, rows, planes, F.tl.shift);
+        j.group0 = uint32_t(ng);
+        ng += brick_groups(j.bg);
+      }
+      // the allocation-free frame's list holds the groups of every lattice it
+      // takes, but not in any shape that the knobs ask for
+      if (!F.noalloc || ng <= F.order.bytes / sizeof(uint2)) break;
+      rows = 0;
+      planes = kBrickPlanes;
+      F.tl.shift = 2;
+    }
+    if (ng >= (uint64_t(1) << 31) >> (3 * F.tl.shift) || (F.noalloc && ng > F.order.bytes / sizeof(uint2))) {
+      log_error("the frame's %llu groups of bricks exceed what one call holds", (unsigned long long)ng);
+      return 1;
+    }
+    F.tl.ngroups = uint32_t(ng);
+    C3D_HIP(F.order.ensure((ng + 1) * sizeof(uint2)));
+    C3D_HIP(F.take.ensure(kTakeBytes));
+  }
   C3D_HIP(F.tjobs.ensure((tj.size() + 1) * sizeof(TessJob)));
   C3D_HIP(M.meta.ensure((n + 1) * sizeof(ObjMeta)));
   C3D_HIP(F.hdr.ensure(sizeof(FrameHdr)));
@@ -1301,10 +1356,9 @@ int tess_emit(Lib& L, Frame& F, contour3d_amd_mesh& M) {
   return 0;
 }
 
-// Reads the plan's totals back (one synchronisation) and sizes the mesh
-// (only its cell indices for a frame).
+// Reads the plan's totals back (one synchronisation) and sizes the mesh.
 template <typename R>
-int tess_readback(Frame& F, contour3d_amd_mesh& M, FrameHdr& hh, uint64_t nline, bool cells_only = false) {
+int tess_readback(Frame& F, contour3d_amd_mesh& M, FrameHdr& hh) {
   const size_t n = size_t(F.tl.nobj);
   unsigned char* hs = static_cast<unsigned char*>(F.hstage.p);
   C3D_HIP(hipMemcpyAsync(hs, F.hdr.p, sizeof(FrameHdr), hipMemcpyDeviceToHost, F.st));
@@ -1320,12 +1374,11 @@ int tess_readback(Frame& F, contour3d_amd_mesh& M, FrameHdr& hh, uint64_t nline,
   }
   M.total = hh.ntri;
   F.prof.ntri += M.total;
-  if (!frame_ids_fit(M.total, nline)) {
-    log_error("%llu triangles and %llu line fragments exceed the 2^32 ids of one frame",
-              (unsigned long long)M.total, (unsigned long long)nline);
+  if (!frame_ids_fit(M.total, 0)) {
+    log_error("%llu triangles exceed the 2^32 ids of one mesh", (unsigned long long)M.total);
     return 1;
   }
-  return cells_only ? ensure_cells(M) : ensure_capacity<R>(M);
+  return ensure_capacity<R>(M);
 }
 
 // Count, scan, plan and emit every object of `objs` into M.  `rjobs`
@@ -1335,12 +1388,12 @@ int tess_readback(Frame& F, contour3d_amd_mesh& M, FrameHdr& hh, uint64_t nline,
 template <typename R>
 int tessellate(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<const contour3d_contour_obj_t*>& objs,
                RasterJob<R>* rjobs, int njobs, FrameHdr& hh) {
-  if (tess_prepare<R>(L, F, M, objs)) return 1;
+  if (tess_prepare<R>(L, F, M, objs, true)) return 1;
   // a mesh has no line fragments (the plan checks the frame's ids)
   forget_table(F, F.hdr, offsetof(FrameHdr, nline));
   C3D_HIP(hipMemsetAsync(F.hdr.as<unsigned char>() + offsetof(FrameHdr, nline), 0, sizeof(uint32_t), F.st));
   if (tess_head<R>(L, F, M, rjobs, njobs, ~uint64_t(0))) return 1;
-  if (tess_readback<R>(F, M, hh, 0)) return 1;
+  if (tess_readback<R>(F, M, hh)) return 1;
   return tess_emit<R>(L, F, M);
 }
 
@@ -1368,9 +1421,9 @@ int frame_lines(Frame& F, const std::vector<Image>& imgs) {
 }
 
 // Uploads the frame's line fragments (and their count into the header) and
-// sizes the z-buffer and the FP64 fragment list.
+// sizes the z-buffer and the fragment list (of a stored mesh: in FP64).
 template <typename R>
-int raster_prepare(Frame& F, uint64_t npx) {
+int raster_prepare(Frame& F, uint64_t npx, bool stored) {
   const bool fp64 = sizeof(R) == 8;
   const Frags& LF = F.h_frags;
   const uint32_t nf = uint32_t(LF.pix.size());
@@ -1380,8 +1433,8 @@ int raster_prepare(Frame& F, uint64_t npx) {
     return 1;
   }
   C3D_HIP(F.key.ensure(npx * sizeof(uint64_t)));
-  // FP64: 64-bit ids for fused frames (32-bit for stored meshes)
-  if (fp64) C3D_HIP(F.id.ensure(npx * sizeof(uint64_t)));
+  // 64-bit ids for frames (a stored mesh: 32-bit ones, in FP64)
+  if (fp64 || !stored) C3D_HIP(F.id.ensure(npx * sizeof(uint64_t)));
   C3D_HIP(F.fpix.ensure((nf + 1) * sizeof(uint32_t)));
   C3D_HIP(F.fdep.ensure((nf + 1) * sizeof(double)));
   C3D_HIP(F.frgb.ensure(3 * size_t(nf + 1)));
@@ -1392,9 +1445,8 @@ int raster_prepare(Frame& F, uint64_t npx) {
   }
   F.h_nline = nf;
   if (upload_table(F, F.hdr, offsetof(FrameHdr, nline), &F.h_nline, sizeof(uint32_t))) return 1;
-  (void)fp64;
   if (F.frag_cap == 0) F.frag_cap = kDefaultFragCap;
-  C3D_HIP(F.frags.ensure(size_t(F.frag_cap) * (fp64 ? sizeof(Frag64) : sizeof(Frag))));
+  C3D_HIP(F.frags.ensure(size_t(F.frag_cap) * sizeof(Frag64)));
   return 0;
 }
 
@@ -1415,7 +1467,7 @@ int raster_launch(Lib&, Frame& F, const contour3d_amd_mesh& M, const RasterJob<R
   uint64_t* key = F.key.as<uint64_t>();
   const MeshView<R> mv = view_of<R>(M);
   if (prof_begin(F, CONTOUR3D_AMD_STAGE_RASTER)) return 1;
-  C3D_HIP(launch_zinit(key, id, false, npx, fp64 ? 0 : 1, false, hdr, F.st));
+  C3D_HIP(launch_zinit(key, id, npx, fp64 ? 0 : 1, hdr, F.st));
   if constexpr (sizeof(R) == 8) {
     // depth pass keeping the fragments that may end up nearest, then the id
     // pass over that list; when the list overflows, the geometry id pass
@@ -1482,6 +1534,18 @@ void release_geoms(Frame& F) {
   F.geoms_used.clear();
 }
 
+// triangles that a frame may hold: an FP32 frame as many as 32-bit ids named,
+// an allocation-free one its limit
+uint64_t max_triangles(const Frame& F, bool fp64) {
+  if (fp64) return ~uint64_t(0);
+  return F.noalloc ? kScratchTriangles : kMaxFrameTriangles - 1;
+}
+
+// whether the finished frame of header `fin` is one that is refused
+bool frame_refused(const Frame& F, const FrameHdr& fin) {
+  return F.drawn && !F.fp64 && (fin.ntri > max_triangles(F, false) || !frame_ids_fit(fin.ntri, fin.nline));
+}
+
 // Waits for a frame's device work and host copies; grows the fragment list
 // after an overflow.
 int frame_finish(Frame& F) {
@@ -1490,15 +1554,25 @@ int frame_finish(Frame& F) {
   C3D_HIP(e);
   FrameHdr& fin = F.last;
   std::memcpy(&fin, F.hstage.p, sizeof(FrameHdr));
-  if (F.unread && !(fin.overflow & 1u)) {
-    // totals of a frame planned without a read back, from its final header
+  const bool refused = frame_refused(F, fin);
+  if (F.drawn && !refused) {
     F.mesh.total = fin.ntri;
     F.prof.ntri += fin.ntri;
   }
-  F.unread = false;
+  F.drawn = false;
   if ((fin.overflow & 2u) && fin.nfrag > F.frag_cap && !F.noalloc) {
     const uint64_t grow = uint64_t(fin.nfrag) + fin.nfrag / 4;
     F.frag_cap = uint32_t(grow > 0xffffffffull ? 0xffffffffull : grow);
+  }
+  if (refused) {
+    if (F.noalloc)
+      log_error("the allocation-free call holds at most %llu triangles in FP32 (and 2^32 triangle and line ids); the "
+                "frame has %llu triangles", (unsigned long long)kScratchTriangles, (unsigned long long)fin.ntri);
+    else
+      log_error("%llu triangles and %llu line fragments exceed the 2^32 ids of one FP32 frame",
+                (unsigned long long)fin.ntri, (unsigned long long)fin.nline);
+    (void)prof_collect(F);
+    return 1;
   }
   return prof_collect(F);
 }
@@ -1602,110 +1676,70 @@ int upload_pass_images(Frame& F, const std::vector<Image>& imgs) {
   return upload_table(F, F.jimg, 0, J.data(), J.size() * sizeof(uint32_t));
 }
 
-// A frame without a stored mesh: z-buffer clear, the fused tessellation and
-// raster, lines and the FP64 id passes, and the resolve from the fields.
-// `lines` sizes the line kernels' grid (at least the frame's fragments).
+// A frame without a stored mesh: the z-buffer clear and brick order, the
+// fused tessellation and raster, lines, the id passes, and the resolve from
+// the fields.  `lines` sizes the line kernels' grid (at least the frame's
+// fragments).
 template <typename R>
-int fused_launch(Lib& L, Frame& F, const contour3d_amd_mesh& M, const RasterJob<R>* rjobs, int njobs, uint64_t npx,
-                 uint32_t lines) {
+int frame_launch(Lib& L, Frame& F, const RasterJob<R>* rjobs, int njobs, uint64_t npx, uint32_t lines) {
   const bool fp64 = sizeof(R) == 8;
+  const int form = fp64 ? 0 : 1;
   FrameHdr* hdr = F.hdr.as<FrameHdr>();
-  void* id = fp64 ? F.id.p : nullptr;
+  uint64_t* id = F.id.as<uint64_t>();
   uint64_t* key = F.key.as<uint64_t>();
   const TessLayout& tl = F.tl;
   const TessJob* tj = F.tjobs.as<TessJob>();
   const uint32_t* jimg = F.jimg.as<uint32_t>();
-  // FP64 frames name triangles by object, cell and slot: no tile starts
-  // and no cell store
-  const uint64_t* start = fp64 ? nullptr : M.bstart.as<uint64_t>();
-  uint32_t* cell = fp64 ? nullptr : M.cell.as<uint32_t>();
-  const uint32_t grid = L.tess_grid(tl.ntj);
+  uint2* order = F.order.as<uint2>();
+  uint32_t* take = F.take.as<uint32_t>();
+  Frag64* frags = F.frags.as<Frag64>();
   const uint32_t fgrid = std::min<uint32_t>((F.frag_cap + 255) / 256, 4096);
-  void* frags = F.frags.p;
   if (prof_begin(F, CONTOUR3D_AMD_STAGE_RASTER)) return 1;
-  C3D_HIP(launch_zinit(key, id, fp64, npx, fp64 ? 0 : 1, fp64, hdr, F.st));
-  if constexpr (sizeof(R) == 8) {
-    // every covered pixel into the fragment list, then its keys; after an
-    // overflow of the list (which grows for the next frame) the z-test
-    // passes over the geometry run instead (each kernel decides on the
-    // device)
-    if (prof_inner_begin(F, CONTOUR3D_AMD_STAGE_FUSED)) return 1;
-    C3D_HIP(launch_tess_raster<R>(tj, tl.njobs, tl.ntj, start, cell, 0, rjobs, jimg, hdr, kRasterAppend, key, id, frags,
-                                  F.frag_cap, grid, F.st));
-    if (prof_inner_end(F)) return 1;
-    C3D_HIP(launch_frag_keys(frags, true, F.frag_cap, hdr, key, fgrid, F.st));
-    C3D_HIP(launch_tess_raster<R>(tj, tl.njobs, tl.ntj, start, cell, 0, rjobs, jimg, hdr, kRasterKey64, key, id,
-                                  nullptr, 0, grid, F.st));
-    C3D_HIP(launch_line_frags(F.fpix.as<uint32_t>(), F.fdep.as<double>(), lines, hdr, 0, 0, key, id, true, F.st));
-    C3D_HIP(launch_frag_ids(frags, true, F.frag_cap, hdr, key, id, fgrid, F.st));
-    C3D_HIP(launch_tess_raster<R>(tj, tl.njobs, tl.ntj, start, cell, 0, rjobs, jimg, hdr, kRasterId64, key, id,
-                                  nullptr, 0, grid, F.st));
-    C3D_HIP(launch_line_frags(F.fpix.as<uint32_t>(), F.fdep.as<double>(), lines, hdr, 1, 0, key, id, true, F.st));
-  } else {
-    // one pass: the packed key carries the id
-    if (prof_inner_begin(F, CONTOUR3D_AMD_STAGE_FUSED)) return 1;
-    C3D_HIP(launch_tess_raster<R>(tj, tl.njobs, tl.ntj, start, cell, M.cap, rjobs, jimg, hdr, kRasterFp32, key, id,
-                                  nullptr, 0, grid, F.st));
-    if (prof_inner_end(F)) return 1;
-    C3D_HIP(launch_line_frags(F.fpix.as<uint32_t>(), F.fdep.as<double>(), lines, hdr, 0, 1, key, id, false, F.st));
-  }
+  C3D_HIP(launch_frame_begin<R>(tj, tl.njobs, rjobs, jimg, order, take, key, id, npx, hdr, F.st));
+  if (prof_inner_begin(F, CONTOUR3D_AMD_STAGE_FUSED)) return 1;
+  C3D_HIP(launch_frame<R>(tj, order, tl.ngroups, tl.shift, take, rjobs, jimg, hdr, kFrameDraw, key, id, frags,
+                          F.frag_cap, L.frame_grid(), F.st));
+  if (prof_inner_end(F)) return 1;
+  C3D_HIP(launch_line_frags(F.fpix.as<uint32_t>(), F.fdep.as<double>(), lines, hdr, 0, form, key, id, true, F.st));
+  // the ids from the fragment list, or, after an overflow of the list (which
+  // grows for the next frame), from the geometry: each kernel decides on the
+  // device
+  C3D_HIP(launch_frag_ids(frags, true, F.frag_cap, hdr, key, id, fgrid, F.st));
+  C3D_HIP(launch_frame<R>(tj, order, tl.ngroups, tl.shift, take, rjobs, jimg, hdr, kFrameIds, key, id, nullptr, 0,
+                          L.frame_grid(), F.st));
+  C3D_HIP(launch_line_frags(F.fpix.as<uint32_t>(), F.fdep.as<double>(), lines, hdr, 1, form, key, id, true, F.st));
   if (prof_end(F)) return 1;
   if (prof_begin(F, CONTOUR3D_AMD_STAGE_RESOLVE)) return 1;
-  C3D_HIP(launch_resolve_field<R>(tj, cell, rjobs, njobs, F.ntiles, M.meta.as<ObjMeta>(), F.frgb.as<uint8_t>(), hdr,
-                                  key, id, F.st));
+  C3D_HIP(launch_resolve_field<R>(tj, rjobs, njobs, F.ntiles, F.mesh.meta.as<ObjMeta>(), F.frgb.as<uint8_t>(), hdr,
+                                  key, id, max_triangles(F, fp64), F.st));
   if (prof_end(F)) return 1;
   return 0;
 }
 
-// The frame's launch sequence (count ... resolve) as a graph, replayed
-// while its layout stays the same: the kernels' arguments and grids depend
-// only on the layout, and everything else (fields, thresholds, colours,
-// cameras, line fragments, outputs) is read from the device tables uploaded
-// before each launch.  The plan kernel flags a frame whose triangles exceed
-// the capacity reserved by earlier frames; the caller then renders it again
-// eagerly.  The first frame of a layout, and one whose line fragments
-// outgrow their buffers, runs eagerly.
+// The frame's launch sequence as a graph, replayed while its layout stays
+// the same: the kernels' arguments and grids depend only on the layout, and
+// everything else (fields, thresholds, colours, cameras, line fragments,
+// outputs) is read from the device tables uploaded before each launch.  The
+// tables and buffers are ready when this is called.
 template <typename R>
-int graph_frame(Lib& L, Frame& F, contour3d_amd_mesh& M, std::vector<Image>& imgs,
-                const std::vector<const contour3d_contour_obj_t*>& objs, RasterJob<R>* rjd, uint64_t npx,
-                bool& replayed) {
-  const bool fp64 = sizeof(R) == 8;
-  const int njobs = int(imgs.size());
-  if (tess_prepare<R>(L, F, M, objs)) return 1;
-  if (upload_pass_images(F, imgs)) return 1;
-  if (raster_prepare<R>(F, npx)) return 1;
-  // FP64 frames have no cell store to outgrow
-  const bool ready =
-      (fp64 || (M.cap > 0 && M.cell.p && M.cap < kMaxFrameTriangles)) && F.h_nline <= line_capacity(F);
-  if (!ready) {
-    F.drop_graph();
-    if (!fp64) {
-      FrameHdr hh{};
-      if (tess_head<R>(L, F, M, rjd, njobs, ~uint64_t(0))) return 1;
-      if (tess_readback<R>(F, M, hh, F.h_nline, true)) return 1;
-    } else {
-      F.unread = true;
-    }
-    if (fused_launch<R>(L, F, M, rjd, njobs, npx, F.h_nline)) return 1;
-    return raster_copies(F, imgs, fp64);
-  }
+int graph_frame(Lib& L, Frame& F, RasterJob<R>* rjd, int njobs, uint64_t npx) {
+  const contour3d_amd_mesh& M = F.mesh;
   const uint32_t lines = line_capacity(F);
   const std::vector<uint64_t> sig = {
-      sizeof(R), uint64_t(njobs), npx, F.ntiles, F.tl.nbt, F.tl.ntj, uint64_t(F.tl.njobs), uint64_t(F.tl.nobj),
-      L.tess_cap, L.tess_grid(F.tl.ntj), L.tess_rows, L.tess_zc, lines, M.cap, F.frag_cap,
-      uint64_t(uintptr_t(F.cnt.p)), uint64_t(uintptr_t(F.tiles.p)), uint64_t(uintptr_t(F.tjobs.p)),
+      sizeof(R), uint64_t(njobs), npx, F.ntiles, F.tl.ngroups, F.tl.shift, uint64_t(F.tl.njobs), uint64_t(F.tl.nobj),
+      L.frame_grid(), lines, F.frag_cap,
+      uint64_t(uintptr_t(F.order.p)), uint64_t(uintptr_t(F.take.p)), uint64_t(uintptr_t(F.tjobs.p)),
       uint64_t(uintptr_t(F.rjobs.p)), uint64_t(uintptr_t(F.hdr.p)), uint64_t(uintptr_t(F.jimg.p)),
       uint64_t(uintptr_t(F.key.p)), uint64_t(uintptr_t(F.id.p)), uint64_t(uintptr_t(F.frags.p)),
       uint64_t(uintptr_t(F.fpix.p)), uint64_t(uintptr_t(F.fdep.p)), uint64_t(uintptr_t(F.frgb.p)),
-      uint64_t(uintptr_t(M.bstart.p)), uint64_t(uintptr_t(M.meta.p)), uint64_t(uintptr_t(M.cell.p))};
+      uint64_t(uintptr_t(M.meta.p))};
   if (!F.gexec || F.gsig != sig) {
     F.drop_graph();
     (void)persistent_blocks();  // device query outside the capture
     const bool prof_on = F.prof.on;
     F.prof.on = false;
     C3D_HIP(hipStreamBeginCapture(F.st, hipStreamCaptureModeThreadLocal));
-    int rc = fp64 ? 0 : tess_head<R>(L, F, M, rjd, njobs, M.cap);
-    if (!rc) rc = fused_launch<R>(L, F, M, rjd, njobs, npx, lines);
+    const int rc = frame_launch<R>(L, F, rjd, njobs, npx, lines);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(F.st, &g);
     F.prof.on = prof_on;
@@ -1724,17 +1758,13 @@ int graph_frame(Lib& L, Frame& F, contour3d_amd_mesh& M, std::vector<Image>& img
     F.gsig = sig;
   }
   C3D_HIP(hipGraphLaunch(F.gexec, F.st));
-  replayed = true;
-  F.unread = true;
-  return raster_copies(F, imgs, fp64);
+  return 0;
 }
 
 // Tessellate the objects of every image and render them all.
 template <typename R>
-int run_frame_t(Lib& L, Frame& F, contour3d_amd_mesh& M, std::vector<Image>& imgs, bool graph, bool& replayed,
-                bool speculate) {
-  replayed = false;
-  F.unread = false;
+int run_frame_t(Lib& L, Frame& F, std::vector<Image>& imgs, bool graph) {
+  F.drawn = false;
   uint64_t npx = 0;
   if (frame_setup(F, imgs, npx)) return 1;
   // the frame's object list: each image's objects, unless an earlier image
@@ -1765,101 +1795,40 @@ int run_frame_t(Lib& L, Frame& F, contour3d_amd_mesh& M, std::vector<Image>& img
   if (upload_table(F, F.rjobs, 0, F.rjobs_host<R>().data(), imgs.size() * sizeof(RasterJob<R>))) return 1;
   RasterJob<R>* rjd = F.rjobs.as<RasterJob<R>>();
   const int njobs = int(imgs.size());
-  // FP64 ids hold the object index below kLineObj - 1 (tri_id64)
-  if (sizeof(R) == 8 && objs.size() + 1 >= kLineObj) {
+  // ids hold the object index below kLineObj - 1 (tri_id64)
+  if (objs.size() + 1 >= kLineObj) {
     log_error("%zu contour objects exceed a frame's %llu", objs.size(), (unsigned long long)(kLineObj - 2));
     return 1;
   }
-  if (graph) return graph_frame<R>(L, F, M, imgs, objs, rjd, npx, replayed);
-  FrameHdr hh{};
-  if (tess_prepare<R>(L, F, M, objs)) return 1;
+  if (tess_prepare<R>(L, F, F.mesh, objs, false)) return 1;
   if (upload_pass_images(F, imgs)) return 1;
-  // the line fragments' count goes to the header before the plan reads it
-  if (raster_prepare<R>(F, npx)) return 1;
-  if constexpr (sizeof(R) == 8) {
-    // no count, scan or plan: triangles are named by object, cell and slot
-    // (tri_id64), and the frame's triangle total comes with its final
-    // header
-    if (fused_launch<R>(L, F, M, rjd, njobs, npx, F.h_nline)) return 1;
-    replayed = true;
-    F.unread = true;
-    return raster_copies(F, imgs, true);
-  }
-  if (speculate && M.cap > 0 && M.cell.p && M.cap < kMaxFrameTriangles) {
-    // planned against the cell store that earlier frames reserved, with no
-    // read back of the totals (no synchronisation mid-frame); the plan
-    // flags a frame that needs more, and run_frame renders it again
-    if (tess_head<R>(L, F, M, rjd, njobs, M.cap)) return 1;
-    if (fused_launch<R>(L, F, M, rjd, njobs, npx, F.h_nline)) return 1;
-    replayed = true;
-    F.unread = true;
-    return raster_copies(F, imgs, sizeof(R) == 8);
-  }
-  if (tess_head<R>(L, F, M, rjd, njobs, ~uint64_t(0))) return 1;
-  if (tess_readback<R>(F, M, hh, F.h_nline, true)) return 1;
-  if (fused_launch<R>(L, F, M, rjd, njobs, npx, F.h_nline)) return 1;
+  if (raster_prepare<R>(F, npx, false)) return 1;
+  if (graph ? graph_frame<R>(L, F, rjd, njobs, npx) : frame_launch<R>(L, F, rjd, njobs, npx, F.h_nline)) return 1;
+  F.drawn = true;
   return raster_copies(F, imgs, sizeof(R) == 8);
 }
 
 // Renders the images as one frame into F; with wait, also waits for the
 // frame (otherwise frame_finish must be called before F is reused).  With
 // graphs on, a waited frame replays the captured launch sequence of its
-// layout; a replay whose triangles outgrew the reserved capacity is
-// rendered again eagerly.
+// layout.
 int run_frame(Lib& L, Frame& F, std::vector<Image>& imgs, int precision, bool wait = true) {
   if (precision != CONTOUR3D_AMD_FP64 && precision != CONTOUR3D_AMD_FP32) {
     log_error("unknown precision %d", precision);
     return 1;
   }
-  const bool graph = wait && L.graphs;
-  for (int attempt = 0; attempt < 2; attempt++) {
-    bool replayed = false;
-    const bool g = graph && attempt == 0;
-    // a waited frame skips the mid-frame read back while the reserved
-    // capacity holds it; a frame that outgrows it is rendered again
-    const bool spec = wait && attempt == 0;
-    const int rc = precision == CONTOUR3D_AMD_FP64 ? run_frame_t<double>(L, F, F.mesh, imgs, g, replayed, spec)
-                                                   : run_frame_t<float>(L, F, F.mesh, imgs, g, replayed, spec);
-    if (rc) {
-      (void)hipStreamSynchronize(F.st);
-      release_geoms(F);
-      F.drop_graph();
-      return rc;
-    }
-    if (!wait) return 0;
-    if (frame_finish(F)) {
-      F.drop_graph();
-      return 1;
-    }
-    if (!(replayed && (F.last.overflow & 1u))) return 0;
-    F.drop_graph();  // the cell store must grow: render again, with the read back
-  }
-  return 0;
-}
-
-// The allocation-free frame: planned against the scratch array's cell
-// store with no read back of its totals, never re-rendered or grown; a
-// frame beyond a scratch maximum fails with an error.
-int run_frame_noalloc(Lib& L, Frame& F, std::vector<Image>& imgs, int precision) {
-  if (precision != CONTOUR3D_AMD_FP64 && precision != CONTOUR3D_AMD_FP32) {
-    log_error("unknown precision %d", precision);
-    return 1;
-  }
-  bool replayed = false;
-  const int rc = precision == CONTOUR3D_AMD_FP64 ? run_frame_t<double>(L, F, F.mesh, imgs, false, replayed, true)
-                                                 : run_frame_t<float>(L, F, F.mesh, imgs, false, replayed, true);
+  const bool graph = wait && L.graphs && !F.noalloc;
+  const int rc = precision == CONTOUR3D_AMD_FP64 ? run_frame_t<double>(L, F, imgs, graph)
+                                                 : run_frame_t<float>(L, F, imgs, graph);
   if (rc) {
     (void)hipStreamSynchronize(F.st);
+    release_geoms(F);
+    F.drop_graph();
     return rc;
   }
-  if (!replayed) {
-    log_error("allocation-free frame not planned against the scratch array");
-    return 1;
-  }
-  if (frame_finish(F)) return 1;
-  if (F.last.overflow & 1u) {
-    log_error("the allocation-free call holds at most %llu triangles (and 2^32 triangle and line ids); the frame "
-              "has %llu triangles", (unsigned long long)F.mesh.cap, (unsigned long long)F.last.ntri);
+  if (!wait) return 0;
+  if (frame_finish(F)) {
+    F.drop_graph();
     return 1;
   }
   return 0;
@@ -1887,7 +1856,7 @@ int render_mesh_t(Lib& L, Frame& F, const contour3d_amd_mesh& M, std::vector<Ima
     return 1;
   }
   // the line fragments' count goes to the header before the plan reads it
-  if (raster_prepare<R>(F, npx)) return 1;
+  if (raster_prepare<R>(F, npx, true)) return 1;
   // the plan kernel recomputes the ranges from the mesh's tile starts
   C3D_HIP(launch_plan<R>(M.bstart.as<uint64_t>(), M.ntiles, M.meta.as<ObjMeta>(), int(M.base.size()), rjd,
                          int(imgs.size()), F.hdr.as<FrameHdr>(), ~uint64_t(0), F.st));
@@ -1958,8 +1927,6 @@ struct Flight {
   int slot = 0;
   std::vector<std::shared_ptr<Request>> reqs;
   uint64_t bytes = 0;
-  double cells = 0;
-  double triangles = 0;  // of the frame, known once it is enqueued
   bool done = false;     // set by the stream's host function
 };
 
@@ -1974,7 +1941,6 @@ struct Server {
   uint64_t next_ticket = 1;
   bool stop = false;
   Frame frames[2];
-  double tri_per_cell = 0.5;  // running estimate of triangles per cell and threshold
   uint64_t admitted = 0;      // estimated bytes of the frames in flight
   std::vector<double> lat_ms;
   uint64_t completed = 0, failed = 0, batches = 0, images = 0, peak = 0;
@@ -2072,29 +2038,19 @@ void snap_give(Server& S, Request& r) {
 
 std::mutex g_server_mu;  // server start/stop against submit/wait/stats
 
-double obj_cells(const contour3d_contour_obj_t& c) {
-  double n = 1;
-  for (int d = 0; d < 3; d++) n *= c.glsizes[d] > 1 ? double(c.glsizes[d] - 1) : 0.0;
-  return n;
-}
-
-// device bytes a request adds to a frame: the cell index of each triangle
-// (a frame stores no triangles), z-buffer and image buffers, an FP64
-// fragment-list share (four covered pixels per pixel), and host fields to
-// upload
-uint64_t estimate_bytes(const Server& S, const contour3d_amd_image_t& im, int precision) {
-  double tri = 0, upload = 0;
+uint64_t estimate_bytes(const contour3d_amd_image_t& im) {
+  double upload = 0;
   for (size_t o = 0; o < im.num_contours; o++) {
     const contour3d_contour_obj_t& c = im.contour_objs[o];
-    tri += obj_cells(c) * S.tri_per_cell;
     if (!is_device_ptr(c.array)) upload += 8.0 * double(c.glsizes[0]) * double(c.glsizes[1]) * double(c.glsizes[2]);
   }
   const double npx = double(im.screen_sizes[0]) * double(im.screen_sizes[1]);
-  const double per_px = 8 + (precision == CONTOUR3D_AMD_FP64 ? 4 + 4 * 16 : 0) + 3 + (im.depth ? 8 : 0);
-  return uint64_t(1.25 * tri * sizeof(uint32_t) + upload + npx * per_px) + (uint64_t(1) << 20);
+  // z-buffer key and id, four fragments, colour and depth
+  const double per_px = 8 + 8 + 4 * sizeof(Frag64) + 3 + (im.depth ? 8 : 0);
+  return uint64_t(upload + npx * per_px) + (uint64_t(1) << 20);
 }
 
-void complete_locked(Server& S, Flight& f, int rc, double tri_total);
+void complete_locked(Server& S, Flight& f, int rc);
 
 // Runs on a runtime thread once the frame's stream has passed its output
 // copies: the requests' images are in their buffers, so they complete here
@@ -2104,16 +2060,20 @@ void on_frame_done(void* p) {
   Flight* f = static_cast<Flight*>(p);
   std::lock_guard<std::mutex> g(f->srv->m);
   f->done = true;
-  complete_locked(*f->srv, *f, 0, f->triangles);
+  // a frame that is refused for its size fails its requests
+  Frame& F = f->srv->frames[f->slot];
+  FrameHdr fin;
+  std::memcpy(&fin, F.hstage.p, sizeof(FrameHdr));
+  complete_locked(*f->srv, *f, frame_refused(F, fin) ? 1 : 0);
   f->srv->cv_work.notify_all();
 }
 
-void complete(Server& S, Flight& f, int rc, double tri_total) {
+void complete(Server& S, Flight& f, int rc) {
   std::lock_guard<std::mutex> g(S.m);
-  complete_locked(S, f, rc, tri_total);
+  complete_locked(S, f, rc);
 }
 
-void complete_locked(Server& S, Flight& f, int rc, double tri_total) {
+void complete_locked(Server& S, Flight& f, int rc) {
   const double t = now_s();
   for (auto& r : f.reqs) {
     snap_give(S, *r);  // the frame that read the snapshots is done
@@ -2133,10 +2093,6 @@ void complete_locked(Server& S, Flight& f, int rc, double tri_total) {
       S.completed++;
       S.lat_ms.push_back((t - r->t_submit) * 1e3);
     }
-  }
-  if (!rc && f.cells > 0) {
-    const double seen = tri_total / f.cells;
-    S.tri_per_cell = std::max(seen, 0.8 * S.tri_per_cell + 0.2 * seen);
   }
   S.admitted -= f.bytes;
   S.batches++;
@@ -2210,7 +2166,6 @@ void server_loop(Lib& L, Server& S) {
       imgs.reserve(fp->reqs.size());
       for (auto& r : fp->reqs) {
         const contour3d_amd_image_t& im = r->img;
-        for (size_t o = 0; o < im.num_contours; o++) fp->cells += obj_cells(im.contour_objs[o]);
         imgs.push_back(make_image(&im.camera_position, &im.light_direction, im.screen_sizes, &im.screen_center,
                                   im.screen_local, &im.bg_color, im.num_contours, im.contour_objs, im.num_lines,
                                   im.line_objs, im.rgb, im.depth, false));
@@ -2219,7 +2174,6 @@ void server_loop(Lib& L, Server& S) {
       {
         std::lock_guard<std::mutex> g(L.mu);
         rc = run_frame(L, F, imgs, prec, false);
-        fp->triangles = double(F.mesh.total);
       }
       if (!rc && hipLaunchHostFunc(F.st, on_frame_done, fp) != hipSuccess) {
         log_error("server: cannot schedule the completion of a frame");
@@ -2236,7 +2190,7 @@ void server_loop(Lib& L, Server& S) {
             break;
           }
         lk.unlock();
-        if (f2) complete(S, *f2, 1, 0);
+        if (f2) complete(S, *f2, 1);
       }
       lk.lock();
       continue;
@@ -2505,7 +2459,7 @@ int contour3d_amd_execute_rgb_noalloc(const contour3d_vector_t* camera_position,
   std::vector<c3d::Image> imgs{c3d::make_image(camera_position, light_direction, screen_sizes, screen_center,
                                                screen_local, bg_color, num_contours, contour_objs, num_lines,
                                                line_objs, rgb, depth, false)};
-  return c3d::run_frame_noalloc(L, L.scratch_frame, imgs, precision);
+  return c3d::run_frame(L, L.scratch_frame, imgs, precision);
 }
 
 int contour3d_amd_execute_batch(size_t num_images, const contour3d_amd_image_t* images, int precision) {
@@ -2927,7 +2881,7 @@ int server_submit(const contour3d_amd_image_t* image, int precision, const char*
     r->img.rgb = r->pinned;
   }
   r->precision = precision;
-  r->bytes = estimate_bytes(*S, r->img, precision);
+  r->bytes = estimate_bytes(r->img);
   r->t_submit = now_s();
   std::lock_guard<std::mutex> g(S->m);
   if (S->stop) {

@@ -72,6 +72,7 @@ struct ViewDev {
   R nc, d, lxx, lyy;
   R fw, fh;   // width, height as reals
   R pitch;    // max(1 / fw, 1 / fh): the larger pixel spacing (set_pitch)
+  R cv;       // (d - nc)^2 |lx x ly| / (lxx lyy): projected area per volume (set_cv)
   int32_t W, H;
 };
 
@@ -79,6 +80,13 @@ struct ViewDev {
 template <typename R>
 C3D_HD void set_pitch(ViewDev<R>& v) {
   v.pitch = fmax(R(1) / v.fw, R(1) / v.fh);
+}
+
+// fills the area constant of a view whose lx, ly, lxx, lyy, nc and d are set
+template <typename R>
+C3D_HD void set_cv(ViewDev<R>& v) {
+  const V3<R> n = vcross(V3<R>{v.lx[0], v.lx[1], v.lx[2]}, V3<R>{v.ly[0], v.ly[1], v.ly[2]});
+  v.cv = (v.d - v.nc) * (v.d - v.nc) * sqrt(vdot(n, n)) / (v.lxx * v.lyy);
 }
 
 #if defined(__HIP_DEVICE_COMPILE__)

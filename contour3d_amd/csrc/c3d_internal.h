@@ -7,6 +7,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "c3d_bricks.h"
+#include "c3d_cull.h"
 #include "c3d_geom.h"
 #include "c3d_tiles.h"
 
@@ -32,6 +34,7 @@ struct FieldDev {
   uint32_t ncells;
   uint32_t ntiles;                // ncz * tg.cols
   uint32_t nitems;                // tg.cols * tg.nzc
+  uint32_t ordered;               // a grid lattice whose grids are finite and monotonic
   FastDiv div_ncx, div_ncy;
   TileGeo tg;
 };
@@ -46,13 +49,16 @@ struct ThrSet {
 };
 
 // One pass over one field: the unit of work of the tessellation kernels.
-// Jobs are stored in a device table; their work items are numbered
-// consecutively from item0.  xoff is the sum of ceil(items / 8) over the
-// earlier jobs: the job's first position in each XCD's walk over the
-// launch's work items.
+// Jobs are stored in a device table.  The count and emit kernels walk its
+// work items, numbered consecutively from item0; xoff is the sum of
+// ceil(items / 8) over the earlier jobs: the job's first position in each
+// XCD's walk over the launch's work items.  A frame walks its bricks, in
+// groups that take entries group0, ... of the frame's ordered list.
 struct TessJob {
   FieldDev f;
+  BrickGeo bg;
   ThrSet ts;
+  uint32_t group0;
   uint32_t item0;
   uint32_t xoff;
   uint64_t code_off;  // a stored mesh: threshold q's cell codes at code_off + q * f.ncells
@@ -128,7 +134,7 @@ struct Frag {
   uint64_t key;
 };
 
-// A triangle of an FP64 frame is named by tri_id64: (object + 1) << 40 |
+// A triangle of a frame is named by tri_id64: (object + 1) << 40 |
 // cell << 4 | slot.  These ids ascend in the reference's drawing order
 // (contour, then cell index k, j, i, then slot; contour/main.c:49-112), so
 // "largest id" breaks depth ties as its sequential >= test does, and they
@@ -139,7 +145,7 @@ __host__ __device__ inline uint64_t tri_id64(uint32_t obj, uint32_t cell, uint32
   return (uint64_t(obj) + 1u) << 40 | uint64_t(cell) << 4 | slot;
 }
 
-// One covered (pixel, triangle) of a fused FP64 frame.
+// One covered (pixel, triangle) of a frame.
 struct Frag64 {
   uint64_t key;
   uint64_t id;  // tri_id64
@@ -174,10 +180,10 @@ struct RasterJob {
   uint8_t bg[4];
 };
 
-// Frame-wide values on the device.  k_plan writes ntri, nwork and the
-// overflow bit 1 (meshes, FP32 frames); k_zinit clears nfrag and bit 2, and
-// in an FP64 frame, which has no plan, also ntri and bit 1, and its Append
-// pass then adds up ntri; the host writes nline before the plan runs.
+// Frame-wide values on the device.  For a stored mesh k_plan writes ntri,
+// nwork and the overflow bit 1, and k_zinit clears nfrag and bit 2; a frame
+// starts with k_frame_begin, which clears all three, and k_frame adds up
+// ntri.  The host writes nline before either.
 struct FrameHdr {
   uint64_t ntri;        // triangles in the mesh (or the frame)
   uint64_t nwork;       // raster work items (sum of the images' triangle ranges)
@@ -219,53 +225,47 @@ hipError_t launch_vertex_normals(const MeshView<R>& m, const ObjMeta* meta_dev, 
 // MeshView) for one object: out[0..4] as k_mesh_compare documents
 hipError_t launch_mesh_compare(const MeshView<double>& a, const ObjMeta* ma, const void* b, int b_fp32,
                                const ObjMeta* mb, uint64_t count, unsigned long long* out, hipStream_t st);
-// Frames without a stored mesh: tessellation fused with the raster.  Every
-// triangle is drawn from registers into each image that shows its object
-// (jimg: per-field-pass offsets [njobs + 1] into a list of the images that
-// show any of the pass's objects).  FP64 frames name triangles by
-// tri_id64 (id: uint64_t per pixel, frags: Frag64) and need no tile starts
-// (start, cell: null); their Append pass adds its triangles to hdr->ntri.
-// FP32 frames number them serially from the tile starts (id: uint32_t,
-// frags: Frag) and store each one's cell index (cell[cap]).  `mode` is a
-// raster mode.
+// A frame without a stored mesh.  launch_frame_begin clears the z-buffer
+// (key, id: uint64_t per pixel), the header and the brick counters (take:
+// 16 counters, 64 words apart) and lists the field passes' groups of bricks
+// by depth (order: one entry per group, TessJob::group0 on); launch_frame
+// then draws every triangle into each image that shows its object (jimg:
+// per-field-pass offsets [njobs + 1] into a list of the images that show any
+// of the pass's objects), with the fragments that may be nearest in frags,
+// and adds the triangles up in hdr->ntri.  Triangles are named by tri_id64.
+// Modes: kFrameDraw, and kFrameIds, the id pass over the geometry, which
+// runs only after the fragment list overflowed.
+enum { kFrameDraw = 0, kFrameIds = 1 };
 template <typename R>
-hipError_t launch_tess_raster(const TessJob* jobs, int njobs, uint32_t nitems, const uint64_t* start, uint32_t* cell,
-                              uint64_t cap, const RasterJob<R>* rjobs, const uint32_t* jimg, FrameHdr* hdr, int mode,
-                              uint64_t* key, void* id, void* frags, uint32_t fcap, uint32_t grid, hipStream_t st);
-// resolve of a fused frame: the nearest triangles and their neighbours'
-// smoothing weights are recomputed from the fields (id as launch_tess_raster)
+hipError_t launch_frame_begin(const TessJob* jobs, int njobs, const RasterJob<R>* rjobs, const uint32_t* jimg,
+                              uint2* order, uint32_t* take, uint64_t* key, uint64_t* id, uint64_t npx, FrameHdr* hdr,
+                              hipStream_t st);
 template <typename R>
-hipError_t launch_resolve_field(const TessJob* jobs, const uint32_t* cell, const RasterJob<R>* rjobs, int njobs,
-                                uint32_t ntiles, const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr,
-                                const uint64_t* key, const void* id, hipStream_t st);
+hipError_t launch_frame(const TessJob* jobs, const uint2* order, uint32_t ngroups, uint32_t shift, uint32_t* take,
+                        const RasterJob<R>* rjobs, const uint32_t* jimg, FrameHdr* hdr, int mode, uint64_t* key,
+                        uint64_t* id, Frag64* frags, uint32_t fcap, uint32_t grid, hipStream_t st);
+// resolve of a frame: the nearest triangles and their neighbours' smoothing
+// weights are recomputed from the fields; a frame of more than max_tri
+// triangles writes nothing
+template <typename R>
+hipError_t launch_resolve_field(const TessJob* jobs, const RasterJob<R>* rjobs, int njobs, uint32_t ntiles,
+                                const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr, const uint64_t* key,
+                                const uint64_t* id, uint64_t max_tri, hipStream_t st);
 // pixel tiles of a W x H image (the resolve's workgroups)
 uint32_t resolve_tiles(uint64_t W, uint64_t H);
-// clears the z-buffer (and the ids: uint64_t per pixel when wide, else
-// uint32_t), the header's fragment count and list-overflow bit, and with
-// fresh (FP64 frames) also its triangle count and capacity bit
-hipError_t launch_zinit(uint64_t* key, void* id, bool wide, uint64_t npx, int precision, bool fresh, FrameHdr* hdr,
-                        hipStream_t st);
-// raster modes:
+// a stored mesh's render: clears the z-buffer and ids (when not null) and
+// the header's fragment count and list-overflow bit
+hipError_t launch_zinit(uint64_t* key, uint32_t* id, uint64_t npx, int precision, FrameHdr* hdr, hipStream_t st);
+// raster modes of a stored mesh:
 //   kRasterFp32     FP32 z-test over packed (depth << 32 | id) keys
 //   kRasterDepth64  FP64 z-test keeping the fragments that may end up nearest
 //   kRasterId64     FP64 id pass over the geometry (runs only when the
 //                   fragment list overflowed)
-//   kRasterAppend   no z-test: every covered pixel goes to the fragment list
-//                   with its key (FP64: the depth's order key; FP32: the
-//                   packed key); launch_frag_keys then applies the list
-//   kRasterKey64    FP64 z-test without a list (runs only when the list
-//                   overflowed, before the geometry id pass)
-// The fused kernel takes kRasterAppend and, after an overflow, kRasterFp32
-// or kRasterKey64 + kRasterId64; the stored-mesh raster takes the first three.
-enum { kRasterFp32 = 0, kRasterDepth64 = 1, kRasterId64 = 2, kRasterAppend = 3, kRasterKey64 = 4 };
+enum { kRasterFp32 = 0, kRasterDepth64 = 1, kRasterId64 = 2 };
 template <typename R>
 hipError_t launch_raster(const MeshView<R>& m, const RasterJob<R>* rjobs, int njobs, FrameHdr* hdr, int mode,
                          uint64_t* key, uint32_t* id, Frag* frags, uint32_t cap, uint32_t grid, hipStream_t st);
-// z-buffer keys of every listed fragment (reads the count from hdr; does
-// nothing when the list overflowed); wide: Frag64, else Frag
-hipError_t launch_frag_keys(const void* frags, bool wide, uint32_t cap, const FrameHdr* hdr, uint64_t* key,
-                            uint32_t grid, hipStream_t st);
-// FP64 id pass over the fragment list (reads the count from hdr; does
+// id pass over the fragment list (reads the count from hdr; does
 // nothing when the list overflowed); wide: Frag64 and uint64_t ids
 hipError_t launch_frag_ids(const void* frags, bool wide, uint32_t cap, const FrameHdr* hdr, const uint64_t* key,
                            void* id, uint32_t grid, hipStream_t st);

@@ -56,6 +56,21 @@ __device__ __forceinline__ const C3D_GLOBAL T* gptr(const T* p) {
   return (const C3D_GLOBAL T*)p;
 }
 
+// a value that every lane holds, as a scalar
+__device__ __forceinline__ uint32_t uniform(uint32_t x) { return uint32_t(__builtin_amdgcn_readfirstlane(int(x))); }
+__device__ __forceinline__ uint64_t uniform(uint64_t x) {
+  return uint64_t(uniform(uint32_t(x >> 32))) << 32 | uniform(uint32_t(x));
+}
+__device__ __forceinline__ double uniform(double x) {
+  return __longlong_as_double(int64_t(uniform(uint64_t(__double_as_longlong(x)))));
+}
+
+// orders a wave's LDS accesses among its own lanes
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 struct CellLoc {
   uint32_t i, j, k;
   uint64_t p0;  // lattice index of corner 0
@@ -816,32 +831,10 @@ __device__ __forceinline__ int find_rjob(const RasterJob<R>* __restrict__ jobs, 
 //                   list holds every fragment whose key equals the final
 //                   value.  Overflow (LDS or global) sets bit 2 of
 //                   hdr->overflow.
-//   kRasterId64     FP64 id pass over the geometry: the latest id (serial,
-//                   or tri_id64 in the fused frames) at each pixel's final
-//                   depth; runs only when the fragment list overflowed
+//   kRasterId64     FP64 id pass over the geometry: the latest serial id at
+//                   each pixel's final depth; runs only when the fragment
+//                   list overflowed
 constexpr int kFragLds = 1024;
-
-// Appends fr to the workgroup's LDS fragment list (s_n entries, cap_lds
-// slots), one LDS atomic per wave; fragments that do not fit go straight to
-// the frame's list (gfrags, gcap entries, counted in hdr->nfrag).  Called
-// by any subset of a wave's lanes.
-template <typename FT>
-__device__ __forceinline__ void append_frag(const FT& fr, FT* s_frag, uint32_t* s_n, uint32_t cap_lds,
-                                            FT* __restrict__ gfrags, uint32_t gcap, FrameHdr* __restrict__ hdr) {
-  const uint64_t act = __ballot(1);
-  const int lane = int(__lane_id());
-  const int leader = __ffsll((long long)act) - 1;
-  uint32_t o0 = 0;
-  if (lane == leader) o0 = atomicAdd(s_n, uint32_t(__popcll(act)));
-  const uint32_t o = uint32_t(__shfl(int(o0), leader)) + uint32_t(__popcll(act & ((1ull << lane) - 1ull)));
-  if (o < cap_lds) {
-    s_frag[o] = fr;
-  } else {
-    const uint32_t g = atomicAdd(&hdr->nfrag, 1u);
-    if (g < gcap) gfrags[g] = fr;
-    else atomicOr(&hdr->overflow, 2u);
-  }
-}
 
 // Projection (project.c), the reference's box and area (render.c:60-89)
 // and the narrowed box of one triangle; returns its candidate pixels (0
@@ -862,28 +855,19 @@ __device__ __forceinline__ uint32_t setup_triangle(const ViewDev<R>& v, const V3
   return uint32_t(P.i1 - P.i0 + 1) * uint32_t(P.j1 - P.j0 + 1);
 }
 
-// The id type of a raster pass (uint32_t serial ids, or uint64_t
-// tri_id64 in the fused FP64 frames) and its fragment record.
-template <typename TId>
-using FragOf = typename std::conditional<sizeof(TId) == 8, Frag64, Frag>::type;
-
 __device__ __forceinline__ void atomic_max_id(uint32_t* p, uint32_t v) { atomicMax(p, v); }
 __device__ __forceinline__ void atomic_max_id(uint64_t* p, uint64_t v) {
   atomicMax(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
 }
 
-// One candidate pixel (i, j) of triangle P (id tid1): the reference's
+// One candidate pixel (i, j) of stored triangle P (id tid1): the reference's
 // barycentric test and harmonic depth (render.c:91-124), then the z-buffer
-// update of `MODE`.  Depth64 and Append put fragments in the workgroup list
-// s_frag (s_n entries, `cap_lds` slots); Append sends those that do not fit
-// straight to the frame's list (gfrags, gcap entries, counted in
-// hdr->nfrag).
-template <typename R, int MODE, typename TId>
+// update of `MODE`.  Depth64 puts fragments in the workgroup list s_frag
+// (s_n entries).
+template <typename R, int MODE>
 __device__ __forceinline__ void pixel_update(const ViewDev<R>& v, uint64_t row0, const Projected<R>& P, int32_t i,
-                                             int32_t j, TId tid1, uint64_t* __restrict__ key, TId* __restrict__ id,
-                                             FragOf<TId>* s_frag, uint32_t* s_n, uint32_t cap_lds,
-                                             FragOf<TId>* __restrict__ gfrags, uint32_t gcap,
-                                             FrameHdr* __restrict__ hdr) {
+                                             int32_t j, uint32_t tid1, uint64_t* __restrict__ key,
+                                             uint32_t* __restrict__ id, Frag* s_frag, uint32_t* s_n) {
   R w0, w1, w2;
   if (!pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2)) return;
   const R dep = pixel_depth(P, w0, w1, w2);
@@ -893,15 +877,6 @@ __device__ __forceinline__ void pixel_update(const ViewDev<R>& v, uint64_t row0,
     // never change it and skips the atomic
     const uint64_t k = uint64_t(ord32(float(dep))) << 32 | uint64_t(tid1);
     if (k > key[px]) atomicMax(reinterpret_cast<unsigned long long*>(key + px), (unsigned long long)k);
-  } else if constexpr (MODE == kRasterAppend) {
-    FragOf<TId> fr;
-    fr.px = uint32_t(px);
-    fr.id = tid1;
-    fr.key = sizeof(R) == 8 ? ord64(double(dep)) : (uint64_t(ord32(float(dep))) << 32 | uint64_t(tid1));
-    append_frag(fr, s_frag, s_n, cap_lds, gfrags, gcap, hdr);
-  } else if constexpr (MODE == kRasterKey64) {
-    const uint64_t k = ord64(double(dep));
-    if (k > key[px]) atomicMax(reinterpret_cast<unsigned long long*>(key + px), (unsigned long long)k);
   } else if constexpr (MODE == kRasterDepth64) {
     const uint64_t k = ord64(double(dep));
     if (k < key[px]) return;
@@ -909,8 +884,8 @@ __device__ __forceinline__ void pixel_update(const ViewDev<R>& v, uint64_t row0,
     // every fragment whose key equals the final value is kept: its key was
     // at least the value read before its own atomic
     const uint32_t o = atomicAdd(s_n, 1u);
-    if (o < cap_lds) {
-      FragOf<TId> fr;
+    if (o < uint32_t(kFragLds)) {
+      Frag fr;
       fr.px = uint32_t(px);
       fr.id = tid1;
       fr.key = k;
@@ -922,17 +897,15 @@ __device__ __forceinline__ void pixel_update(const ViewDev<R>& v, uint64_t row0,
 }
 
 // one triangle drawn by its own lane: every candidate of its box in turn
-template <typename R, int MODE, typename TId>
-__device__ __forceinline__ void draw_triangle(const ViewDev<R>& v, uint64_t row0, const V3<R> wpos[3], TId tid1,
-                                              uint64_t* __restrict__ key, TId* __restrict__ id,
-                                              FragOf<TId>* s_frag, uint32_t* s_n, uint32_t cap_lds,
-                                              FragOf<TId>* __restrict__ gfrags = nullptr, uint32_t gcap = 0,
-                                              FrameHdr* __restrict__ hdr = nullptr) {
+template <typename R, int MODE>
+__device__ __forceinline__ void draw_triangle(const ViewDev<R>& v, uint64_t row0, const V3<R> wpos[3], uint32_t tid1,
+                                              uint64_t* __restrict__ key, uint32_t* __restrict__ id, Frag* s_frag,
+                                              uint32_t* s_n) {
   Projected<R> P;
   if (!setup_triangle<R>(v, wpos, P)) return;
   for (int32_t j = P.j0; j <= P.j1; j++)
     for (int32_t i = P.i0; i <= P.i1; i++)
-      pixel_update<R, MODE, TId>(v, row0, P, i, j, tid1, key, id, s_frag, s_n, cap_lds, gfrags, gcap, hdr);
+      pixel_update<R, MODE>(v, row0, P, i, j, tid1, key, id, s_frag, s_n);
 }
 
 // registers of one raster work item, loaded a round ahead
@@ -989,7 +962,7 @@ __global__ __launch_bounds__(kThreads) void k_raster(MeshView<R> m, const Raster
       const V3<R> wp[3] = {{cur.p[0], cur.p[1], cur.p[2]}, {cur.p[3], cur.p[4], cur.p[5]},
                            {cur.p[6], cur.p[7], cur.p[8]}};
       const ViewDev<R> v = rjobs[cur.jb].v;
-      draw_triangle<R, MODE>(v, rjobs[cur.jb].px0, wp, uint32_t(cur.t + 1), key, id, s_frag, &s_n, kFragLds);
+      draw_triangle<R, MODE>(v, rjobs[cur.jb].px0, wp, uint32_t(cur.t + 1), key, id, s_frag, &s_n);
     }
     if constexpr (MODE == kRasterDepth64) {
       __syncthreads();
@@ -1012,45 +985,54 @@ __global__ __launch_bounds__(kThreads) void k_raster(MeshView<R> m, const Raster
 // ----------------------------------------------------------------------
 // frames without a stored mesh: tessellation fused with the raster
 //
-// Each tile is classified and scanned in chunks of 256 cells as in the emit
-// pass, but a chunk holds only about a third as many triangles as cells, so
-// its triangles are not drawn in place.  They are queued instead, as
-// compact items (serial position in FP32, cell, vertex corners,
-// threshold), in a per-workgroup LDS ring that carries them over chunk and
-// tile boundaries (within one field pass), and the ring is drained 256
-// items at a time:
-// every lane then computes, projects and draws one triangle.  A drained
-// triangle rereads the corner values its vertices need (they were loaded
-// moments earlier by the same workgroup, so they come from cache).  An FP32
-// frame stores only the cell index of each triangle (at its serial
-// position), an FP64 frame nothing (its ids name the cell and slot); the
-// resolve recomputes what it needs from the field.  Triangles are drawn
-// into every image of the field pass that shows their object (jimg:
-// offsets per field pass into a list of the images showing any of its
-// objects).  In Append mode every covered pixel collects in an LDS list
-// that is flushed to the frame's list once half full; the z-test modes run
-// only after that list overflowed.  A frame flagged by the plan as outgrowing `cap`
-// draws nothing (it is rendered again).
-constexpr uint32_t kFragLdsFused = 512;  // LDS fragment slots of a workgroup (about 20 per drain at 512^3)
-constexpr uint32_t kFragFlushAt = 256;   // flushed to the frame's list from this fill on
-constexpr uint32_t kRing = 512;          // a power of two, at least 2 * kThreads
+// Every wave works by itself, with no barrier between the waves of a
+// workgroup.  It takes bricks of a field (c3d_bricks.h: up to 8 x 8 x 8
+// cells, a lane per cell column), nearest groups first, from one counter per
+// XCD; classifies the brick's lattice points plane by plane; lists the cells
+// that a threshold cuts (about a fifth of a turbulent field's); and queues
+// the triangles of the listed cells of the rendered interior, 64 cells at a
+// time, as 8-byte items (cell; vertex corners, threshold, slot) in an LDS
+// ring that is drained 64 at a time: every lane then computes, projects and
+// draws one triangle into each image that shows its object (jimg: offsets
+// per field pass into a list of the images showing any of its objects).  The
+// ring carries items over rounds and bricks (within one field pass).
+// Nothing is stored per triangle: ids name the object, cell and slot
+// (tri_id64), and the resolve recomputes what it needs from the field.
+//
+// A brick that lies behind what the z-buffer holds is counted but not drawn,
+// except for cells whose triangles' projections may be too small for the
+// depth bound to hold (c3d_cull.h; FP64 only: in FP32 rounding leaves too
+// many such cells).  With the bricks taken front to back, most of a dense
+// field is behind its first surfaces: at 512^3, three thresholds and
+// 1920 x 1080, 42 M of 129 M triangles are drawn.
+//
+// What bounds it: vector-ALU issue and the latency of each brick's chain of
+// reads.  That FP64 frame's kernel took 4.50 ms as a tessellation of whole
+// rows with a queue and barriers per workgroup, no z-test and no order; 3.61
+// ms in bricks taken front to back by workgroups; and 2.2 ms by waves, with
+// the cut cells listed before anything is done with them (FP32, where every
+// triangle is drawn: 3.41 -> 2.8 ms, besides 0.28 ms of counting passes that
+// serial ids had needed).  Close-ups, where few triangles cover many pixels
+// each, gained most: 301 x 187 x 223 with five thresholds 8.15 -> 1.4 ms.
+//
+// Every covered pixel is tested against the z-buffer as it is drawn (key:
+// the depth's order key, larger is nearer); a fragment at or above the value
+// read goes through atomicMax into the z-buffer and, with its id, into the
+// frame's fragment list.  The list holds every fragment whose key equals the pixel's final key, and
+// k_frag_ids then gives each pixel the largest id among them: "largest
+// depth, then last in drawing order", the result of the reference's
+// sequential >= test (render.c:125-132).  If the frame's list overflows, a
+// second pass over the geometry (kFrameIds) finds the ids instead.
+constexpr uint32_t kFragChunk0 = 64, kFragChunk = 1024;  // entries of the frame's fragment list that a wave
+                                                         // reserves at a time: at first, and at most
+static_assert(kFragChunk0 >= 64, "a reservation holds a fragment of every lane");
+constexpr uint32_t kNoPixel = 0xffffffffu;               // a reserved entry that stayed empty
+constexpr uint32_t kWaveRing = 128;    // queued triangles of a wave (a power of two, at least 2 * 64)
+constexpr uint32_t kRing = 512;        // of a workgroup of the emit (at least 2 * kThreads)
 
 // a queued triangle names its threshold in 2 bits (ring item bits 18-19),
 // and the drains index ThrSet::thr and ::obj with it
 static_assert(kMaxThr == 4, "the ring's threshold field is 2 bits wide");
-
-struct FusedLds {
-  uint8_t code[kMaxThr][kThreads];
-  uint16_t pref[kMaxThr][kThreads];
-  uint16_t low[kTileChunks][kThreads];  // lower-plane codes of the tile's cells (cell p at [p / 256][p % 256])
-  uint64_t wave[kThreads / 64];
-  uint8_t ntri[256];
-  uint32_t rg[kRing];  // serial position of the queued triangle
-  uint32_t rc[kRing];  // its cell
-  uint32_t re[kRing];  // its vertices' (tail, head) corners (slot entry bits 0-17) | threshold << 18 |
-                       // slot << 20 | corner code << 24
-  uint32_t nfrag, fbase, fcnt;
-};
 
 // positions of the triangle whose vertices join the corners in `ent` (slot
 // entry bits 0-17) of cell L, reading the two corner values of each
@@ -1083,107 +1065,696 @@ __device__ __forceinline__ void slot_positions_mem(const FieldDev& f, const Cell
   }
 }
 
-// Ends a drain: in Append mode, moves the workgroup's LDS fragments to the
-// frame's list once they fill kFragFlushAt slots (every time with `all`).
-// One reservation on the frame's counter per flush keeps that shared atomic
-// rare.
-template <int MODE, typename FT>
-__device__ __forceinline__ void flush_frags(FusedLds& S, FT* s_frag, FrameHdr* __restrict__ hdr,
-                                            FT* __restrict__ frags, uint32_t fcap, bool all) {
-  __syncthreads();
-  if constexpr (MODE == kRasterAppend) {
-    if (threadIdx.x == 0) {
-      const uint32_t have = S.nfrag;
-      const uint32_t c = have < kFragLdsFused ? have : kFragLdsFused;
-      const bool go = c && (all || c >= kFragFlushAt);
-      uint32_t b = 0;
-      if (go) {
-        b = atomicAdd(&hdr->nfrag, c);
-        if (uint64_t(b) + c > fcap) atomicOr(&hdr->overflow, 2u);
-        S.nfrag = 0;
-      }
-      S.fbase = b;
-      S.fcnt = go ? c : 0u;
+// Images of a field pass for which triangles are told apart by whether they
+// can reach them; a pass shown in more draws every triangle into the others.
+constexpr uint32_t kMaskImages = 8;
+constexpr uint32_t kAllImages = (1u << kMaskImages) - 1u;
+
+struct FrameLds {
+  uint16_t pc[kBrickPlanes + 1][64];    // plane codes of each lane's cell column
+  uint16_t list[kBrickPlanes * 64];     // the brick's cut cells: plane << 6 | column
+  uint32_t rc[kWaveRing];  // cell of the queued triangle
+  uint32_t re[kWaveRing];  // its vertices' (tail, head) corners (slot entry bits 0-17) | threshold << 18 | slot << 20 |
+                           // the images it may reach, of the pass's first kMaskImages, << 24
+  // a round of 64 listed cells: their indices, codes, exclusive triangle
+  // counts and irregular thresholds (bit q)
+  uint32_t cell[64];
+  uint16_t pref[kMaxThr][64];
+  uint8_t code[kMaxThr][64];
+  uint8_t irr[64];
+  uint32_t fnext, fend, fchunk;  // the wave's entries of the fragment list: free ones, and the next reservation's size
+};
+
+// a lane's value, as a scalar
+__device__ __forceinline__ uint32_t lane_u32(uint32_t x, int l) { return uint32_t(__builtin_amdgcn_readlane(int(x), l)); }
+__device__ __forceinline__ float lane_of(float x, int l) { return __uint_as_float(lane_u32(__float_as_uint(x), l)); }
+__device__ __forceinline__ uint64_t lane_of(uint64_t x, int l) {
+  return uint64_t(lane_u32(uint32_t(x >> 32), l)) << 32 | lane_u32(uint32_t(x), l);
+}
+__device__ __forceinline__ double lane_of(double x, int l) {
+  return __longlong_as_double(int64_t(lane_of(uint64_t(__double_as_longlong(x)), l)));
+}
+
+// depth keys: larger is nearer; 32-bit depths in the upper half
+__device__ __forceinline__ uint64_t depth_key(double d) { return ord64(d); }
+__device__ __forceinline__ uint64_t depth_key(float d) { return uint64_t(ord32(d)) << 32; }
+
+// Appends fr to the frame's fragment list (called by any subset of the
+// wave's lanes).  A wave fills entries that it reserved, and reserves twice
+// as many as the last time when they run out, so the list's counter, which
+// all waves share, is touched rarely whether a wave finds three fragments or
+// a million.
+__device__ __forceinline__ void append_frag(const Frag64& fr, FrameLds& S, Frag64* __restrict__ gfrags, uint32_t gcap,
+                                            FrameHdr* __restrict__ hdr) {
+  const uint64_t act = __ballot(1);
+  const uint32_t lane = __lane_id(), n = uint32_t(__popcll(act));
+  const int leader = __builtin_ctzll(act);
+  const uint32_t rank = uint32_t(__popcll(act & ((1ull << lane) - 1ull)));
+  const uint32_t at = S.fnext, room = S.fend - at;
+  wave_lds_fence();
+  uint32_t more = 0;
+  if (n > room) {
+    // the rest go to a new reservation
+    const uint32_t size = S.fchunk;
+    if (lane == uint32_t(leader)) {
+      more = atomicAdd(&hdr->nfrag, size);
+      if (uint64_t(more) + size > gcap) atomicOr(&hdr->overflow, 2u);
+      S.fnext = more + (n - room);
+      S.fend = more + size;
+      S.fchunk = 2u * size < kFragChunk ? 2u * size : kFragChunk;
     }
-    __syncthreads();
-    const uint32_t b0 = S.fbase, c = S.fcnt;
-    if (c) {
-      for (uint32_t e = threadIdx.x; e < c; e += kThreads) {
-        if (uint64_t(b0) + e < fcap) frags[b0 + e] = s_frag[e];
-      }
-      __syncthreads();
-    }
+    more = lane_u32(more, leader);
+  } else if (lane == uint32_t(leader)) {
+    S.fnext = at + n;
+  }
+  wave_lds_fence();
+  const uint32_t g = rank < room ? at + rank : more + (rank - room);
+  if (g < gcap) gfrags[g] = fr;
+}
+
+// what a drawing lane needs beside its triangle
+struct DrawTo {
+  uint64_t* __restrict__ key;
+  uint64_t* __restrict__ id;
+  Frag64* __restrict__ frags;
+  uint32_t fcap;
+  FrameHdr* __restrict__ hdr;
+};
+
+// One candidate pixel (i, j) of triangle P (id tid): the reference's
+// barycentric test and harmonic depth (render.c:91-124), then the z-test.
+template <typename R, int MODE>
+__device__ __forceinline__ void frame_pixel(const ViewDev<R>& v, uint64_t row0, const Projected<R>& P, int32_t i,
+                                            int32_t j, uint64_t tid, FrameLds& S, const DrawTo& D) {
+  R w0, w1, w2;
+  if (!pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2)) return;
+  const uint64_t k = depth_key(pixel_depth(P, w0, w1, w2));
+  const uint64_t px = row0 + uint64_t(j) * uint64_t(v.W) + uint64_t(i);
+  // keys only grow, so a value read here, however stale, that is above k
+  // means the fragment cannot be the pixel's
+  const uint64_t was = D.key[px];
+  if constexpr (MODE == kFrameDraw) {
+    if (k < was) return;
+    if (k > was) atomicMax(reinterpret_cast<unsigned long long*>(D.key + px), (unsigned long long)k);
+    Frag64 fr;
+    fr.key = k;
+    fr.id = tid;
+    fr.px = uint32_t(px);
+    fr.pad = 0;
+    append_frag(fr, S, D.frags, D.fcap, D.hdr);
+  } else {
+    if (k == was) atomic_max_id(D.id + px, tid);
   }
 }
 
-// Draws the n (<= kThreads) oldest queued triangles of field pass jb, one
-// per thread: with 64-bit ids (FP64) as tri_id64, else as their serial
-// position + 1.
-template <typename R, int MODE, typename TId>
-__device__ __forceinline__ void drain_ring(FusedLds& S, FragOf<TId>* s_frag, uint32_t head, uint32_t n,
-                                           const TessJob* __restrict__ jobs, uint32_t jb,
-                                           const RasterJob<R>* __restrict__ rjobs, const uint32_t* __restrict__ jimg,
-                                           FrameHdr* __restrict__ hdr, uint64_t* __restrict__ key,
-                                           TId* __restrict__ id, FragOf<TId>* __restrict__ frags, uint32_t fcap) {
+// Draws the wave's triangles (one per lane with `here`).  Each lane walks
+// the box of its own triangle; a box much larger than the wave's average
+// (more than 64 pixels and four times the average) is walked by the whole
+// wave, 8 x 8 pixels at a time, so that one large triangle among small ones
+// does not hold the other 63 lanes.
+template <typename R, int MODE>
+__device__ __forceinline__ void draw_wave(const ViewDev<R>& v, uint64_t row0, bool here, const V3<R> wpos[3],
+                                          uint64_t tid, FrameLds& S, const DrawTo& D) {
+  constexpr uint32_t kLarge = 64;
+  Projected<R> P;
+  uint32_t n = 0;
+  if (here) n = setup_triangle<R>(v, wpos, P);
+  bool together = n > kLarge;
+  if (__ballot(together)) {
+    float sum = float(n);
+#pragma unroll
+    for (int d = 32; d; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    together = together && float(n) > sum * (4.0f / 64.0f);
+  }
+  if (n && !together)
+    for (int32_t j = P.j0; j <= P.j1; j++)
+      for (int32_t i = P.i0; i <= P.i1; i++) frame_pixel<R, MODE>(v, row0, P, i, j, tid, S, D);
+  for (uint64_t todo = __ballot(together); todo; todo &= todo - 1u) {
+    const int l = __builtin_ctzll(todo);
+    Projected<R> Q;
+#pragma unroll
+    for (int a = 0; a < 3; a++) Q.q[a] = {lane_of(P.q[a].x, l), lane_of(P.q[a].y, l), lane_of(P.q[a].z, l)};
+    Q.ainv = lane_of(P.ainv, l);
+    Q.i0 = int32_t(lane_u32(uint32_t(P.i0), l));
+    Q.i1 = int32_t(lane_u32(uint32_t(P.i1), l));
+    Q.j0 = int32_t(lane_u32(uint32_t(P.j0), l));
+    Q.j1 = int32_t(lane_u32(uint32_t(P.j1), l));
+    const uint64_t t = lane_of(tid, l);
+    const int32_t li = int32_t(__lane_id() & 7u), lj = int32_t(__lane_id() >> 3);
+    for (int32_t jb = Q.j0; jb <= Q.j1; jb += 8)
+      for (int32_t ib = Q.i0; ib <= Q.i1; ib += 8)
+        if (ib + li <= Q.i1 && jb + lj <= Q.j1) frame_pixel<R, MODE>(v, row0, Q, ib + li, jb + lj, t, S, D);
+  }
+}
+
+// Marks the entries that the wave reserved and did not fill.
+__device__ __forceinline__ void close_frags(FrameLds& S, Frag64* __restrict__ frags, uint32_t fcap) {
+  wave_lds_fence();
+  for (uint32_t g = S.fnext + __lane_id(); g < S.fend; g += 64u)
+    if (g < fcap) frags[g].px = kNoPixel;
+}
+
+// Draws the n (<= 64) oldest queued triangles of field pass jb, one per
+// lane.
+template <typename R, int MODE>
+__device__ __forceinline__ void drain_ring(FrameLds& S, uint32_t head, uint32_t n, const TessJob* __restrict__ jobs,
+                                           uint32_t jb, const RasterJob<R>* __restrict__ rjobs,
+                                           const uint32_t* __restrict__ jimg, const DrawTo& D) {
   V3<R> P[3];
-  bool drawn = false;
-  uint32_t obj = 0;
-  TId tid = 0;
-  if (threadIdx.x < n) {
+  uint32_t obj = 0, images = 0;
+  uint64_t tid = 0;
+  const uint32_t lane = __lane_id();
+  const bool drawn = lane < n;
+  if (drawn) {
     const FieldDev f = jobs[jb].f;
-    const uint32_t s = (head + threadIdx.x) & (kRing - 1u);
+    const uint32_t s = (head + lane) & (kWaveRing - 1u);
     const uint32_t cc = S.rc[s], x = S.re[s];
-    if constexpr (sizeof(TId) == 4) tid = S.rg[s] + 1u;
     const CellLoc L = locate(f, cc);
-    if (interior_cell(f, L)) {
-      const uint32_t q = (x >> 18) & 3u;
-      // one load per lane indexed by the threshold number: fewer vector
-      // instructions and spilled registers than selecting among kMaxThr
-      const double thr = jobs[jb].ts.thr[q];
-      obj = jobs[jb].ts.obj[q];
-      slot_positions_mem<R>(f, L, thr, x & 0x3ffffu, P);
-      if constexpr (sizeof(TId) == 8) tid = tri_id64(obj, cc, (x >> 20) & 15u);
-      drawn = true;
-    }
+    const uint32_t q = (x >> 18) & 3u;
+    // one load per lane indexed by the threshold number: fewer vector
+    // instructions and spilled registers than selecting among kMaxThr
+    const double thr = jobs[jb].ts.thr[q];
+    obj = jobs[jb].ts.obj[q];
+    slot_positions_mem<R>(f, L, thr, x & 0x3ffffu, P);
+    tid = tri_id64(obj, cc, (x >> 20) & 15u);
+    images = x >> 24;
   }
-  // the images of this field pass (the same for the whole workgroup)
-  for (uint32_t u = jimg[jb]; u < jimg[jb + 1]; u++) {
-    const uint32_t k = jimg[u];
-    const bool here = drawn && obj >= rjobs[k].obj0 && obj < rjobs[k].obj1;
+  // the images of this field pass (the same for every lane)
+  for (uint32_t u = uniform(jimg[jb]), end = uniform(jimg[jb + 1]); u < end; u++) {
+    const uint32_t k = uniform(jimg[u]);
+    const bool here = drawn && obj >= rjobs[k].obj0 && obj < rjobs[k].obj1 && (images & 1u);
+    images = images >> 1 | 1u << (kMaskImages - 1u);  // the images past the mask: always
+    if (!__ballot(here)) continue;
     const ViewDev<R> v = rjobs[k].v;
-    if (here)
-      draw_triangle<R, MODE, TId>(v, rjobs[k].px0, P, tid, key, id, s_frag, &S.nfrag, kFragLdsFused, frags, fcap,
-                                  hdr);
+    draw_wave<R, MODE>(v, rjobs[k].px0, here, P, tid, S, D);
   }
-  flush_frags<MODE>(S, s_frag, hdr, frags, fcap, false);
 }
 
-// The work-item loop shared by the queue kernels: marches each work item's
-// column up its planes, classifies each tile's cells in chunks of 256
-// (loading only the upper corners: the lower-plane codes carry over from the
-// plane below, in LDS), queues the chunk's triangles in the LDS ring in
-// serial order and calls drain(head, n, jb) for every full 256 items (and
-// for the rest when the field pass changes and at the end).  With kPlanes
-// each plane's upper codes are first computed for the whole tile by column
-// segments (classify_plane, into s_hi: the cells of a segment share their
-// rows of lattice points) and the chunks read them from LDS; the fused
-// kernel measured 3.6% (FP64) and 1.3% (FP32) faster so, the FP32 emit
-// 1.5%; the FP64 emit, which would lose a workgroup per CU to the extra
-// LDS, loads each cell's corners itself.  With
-// kStoreCell the cell index of each triangle is stored at its serial
-// position as it is queued; with kStoreCode every cell's corner code of
-// every threshold q is stored at codeout[code_off + q * ncells + cell]: by
-// each cell's thread as bytes (kStoreCode 1) or from LDS as 4-byte words
-// (kStoreCode 2; measured faster in the FP64 emit, slower in the FP32 one).
-// With kSerial each queued triangle carries its serial position (from the
-// tile starts `start`); without it (fused FP64 frames, whose ids come from
-// the cell and slot) start is not read.  Expects S.ntri loaded and a
-// barrier since.
-template <bool kStoreCell, int kStoreCode, bool kReload, bool kPlanes, bool kSerial, typename Drain>
-__device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const TessJob* __restrict__ jobs, int njobs,
+constexpr uint32_t kMaxBoxPixels = 1u << 14;  // pixels read for one brick's visibility at most
+
+// Whether every z-buffer key of the pixel box of an image (first pixel row0,
+// W pixels a row) is above `bound`: 256 pixels at a time until one is not.
+// The reads go to the device's coherent level, so that they see what other
+// XCDs have drawn (an older value would only be smaller).
+__device__ __forceinline__ bool box_above(const uint64_t* __restrict__ key, uint64_t row0, uint32_t W,
+                                          const BrickLimits& o, uint64_t bound) {
+  if (o.i1 < o.i0 || o.j1 < o.j0) return true;  // no fragment falls on the image
+  const uint32_t w = uint32_t(o.i1 - o.i0) + 1u, n = w * (uint32_t(o.j1 - o.j0) + 1u);
+  if (n > kMaxBoxPixels) return false;
+  const float rw = 1.0f / float(w);
+  for (uint32_t t0 = 0; t0 < n; t0 += 256u) {
+    bool below = false;
+#pragma unroll
+    for (uint32_t a = 0; a < 4u; a++) {
+      uint32_t t = t0 + a * 64u + __lane_id();
+      t = t < n ? t : n - 1u;
+      // t / w for t < 2^14: the quotient's error is far below 1 / w
+      const uint32_t r = uint32_t((float(t) + 0.5f) * rw);
+      const uint64_t px = row0 + uint64_t(uint32_t(o.j0) + r) * W + uint32_t(o.i0) + (t - r * w);
+      below = below || __hip_atomic_load(key + px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= bound;
+    }
+    if (__ballot(below)) return false;
+  }
+  return true;
+}
+
+// The images (of the pass's first kMaskImages, bit u for image jimg[u0 + u])
+// that regular cells of brick B may still reach; scale gets the others'
+// area scale (lane u holds image u's).  The corners' views are formed by
+// lanes 0-7 (and every other eight lanes alike).
+__device__ __forceinline__ uint32_t reachable_images(const FieldDev& f, const BrickBox& B,
+                                                     const RasterJob<double>* __restrict__ rjobs,
+                                                     const uint32_t* __restrict__ jimg, uint32_t u0, uint32_t u1,
+                                                     const uint64_t* __restrict__ key, float& scale) {
+  uint32_t seen = kAllImages;
+  const uint32_t c = __lane_id() & 7u;
+  const double px = gptr(f.gx)[c & 1u ? B.i1 : B.i0], py = gptr(f.gy)[c & 2u ? B.j1 : B.j0],
+               pz = gptr(f.gz)[c & 4u ? B.k1 : B.k0];
+  for (uint32_t u = u0; u < u1 && u - u0 < kMaskImages; u++) {
+    const RasterJob<double>& J = rjobs[uniform(jimg[u])];
+    CornerView cv;
+    const bool ok = corner_view(J.v, px, py, pz, cv);
+    if (__ballot(ok) != ~0ull) continue;
+    BrickRange r = {cv.x, cv.x, cv.y, cv.y, cv.nr, cv.nr, cv.size};
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) {
+      r.x0 = fmin(r.x0, __shfl_xor(r.x0, d, 64));
+      r.x1 = fmax(r.x1, __shfl_xor(r.x1, d, 64));
+      r.y0 = fmin(r.y0, __shfl_xor(r.y0, d, 64));
+      r.y1 = fmax(r.y1, __shfl_xor(r.y1, d, 64));
+      r.n0 = fmin(r.n0, __shfl_xor(r.n0, d, 64));
+      r.n1 = fmax(r.n1, __shfl_xor(r.n1, d, 64));
+      r.size = fmax(r.size, __shfl_xor(r.size, d, 64));
+    }
+    BrickLimits o;
+    if (!uniform(uint32_t(brick_limits(J.v, r, o)))) continue;
+    o.i0 = int32_t(uniform(uint32_t(o.i0)));
+    o.i1 = int32_t(uniform(uint32_t(o.i1)));
+    o.j0 = int32_t(uniform(uint32_t(o.j0)));
+    o.j1 = int32_t(uniform(uint32_t(o.j1)));
+    if (!box_above(key, J.px0, uint32_t(J.v.W), o, uniform(depth_key(o.bound)))) continue;
+    seen &= ~(1u << (u - u0));
+    scale = __lane_id() == u - u0 ? o.scale : scale;
+  }
+  return seen;
+}
+
+// The thresholds (bit q) at which cell (i, j, k) is cut (`cuts`) and not
+// regular in one of the images its brick is hidden in: there it is drawn all
+// the same.
+__device__ __forceinline__ uint32_t irregular_at(const TessJob& J, uint32_t i, uint32_t j, uint32_t k, uint32_t cuts,
+                                                 const RasterJob<double>* __restrict__ rjobs,
+                                                 const uint32_t* __restrict__ jimg, uint32_t u0, uint32_t seen,
+                                                 float scale, bool inner) {
+  const FieldDev& f = J.f;
+  double v[8], x0 = 0, y0 = 0, z0 = 0, hx = 1, hy = 1, hz = 1;
+  if (inner) {
+    const uint64_t nxy = uint64_t(f.nx) * f.ny;
+    const C3D_GLOBAL double* p = gptr(f.f) + k * nxy + uint64_t(j) * f.nx + i;
+    load_plane4(p, f.nx, v);
+    load_plane4(p + nxy, f.nx, v + 4);
+    x0 = gptr(f.gx)[i];
+    y0 = gptr(f.gy)[j];
+    z0 = gptr(f.gz)[k];
+    hx = gptr(f.gx)[i + 1u] - x0;
+    hy = gptr(f.gy)[j + 1u] - y0;
+    hz = gptr(f.gz)[k + 1u] - z0;
+  }
+  const float fx = float(hx), fy = float(hy), fz = float(hz);
+  const float cell = fabsf(fx * fy * fz) * 0.999999f;
+  uint32_t bad = 0;
+  for (uint32_t hid = ~seen & kAllImages; hid; hid &= hid - 1u) {
+    const uint32_t u = uint32_t(__builtin_ctz(hid));
+    const ViewDev<double>& vw = rjobs[uniform(jimg[u0 + u])].v;
+    const float volume = cell * lane_of(scale, int(u));
+    if (inner) {
+      CellValues cv;
+      cell_values(v, float(vw.cam[0] - x0) / fx, float(vw.cam[1] - y0) / fy, float(vw.cam[2] - z0) / fz, cv);
+#pragma unroll
+      for (int q = 0; q < kMaxThr; q++)
+        if (((cuts >> q) & 1u) && !cell_regular(cv, float(v[0] - J.ts.thr[q]), volume)) bad |= 1u << q;
+    }
+  }
+  return bad;
+}
+
+// Takes bricks for a wave, from XCD list x, and from another list once that
+// one is empty; each is asked for while the one before is worked on.  The
+// lists' counters are `take`, 64 words apart.
+struct Taker {
+  uint32_t* __restrict__ take;
+  uint32_t ngroups, shift;
+  uint32_t x;
+  uint32_t ahead;  // lane 0: the position asked for
+
+  __device__ __forceinline__ void ask() {
+    if (__lane_id() == 0) ahead = atomicAdd(take + 64u * x, 1u);
+  }
+  // the brick asked for, or one from the first other list that still has
+  // some; false when all are empty.  The next one is asked for at once.
+  __device__ __forceinline__ bool next(uint32_t& px, uint32_t& pp) {
+    pp = uniform(ahead);
+    for (uint32_t tried = 0; pp >= brick_positions(ngroups, shift, x); tried++) {
+      if (tried == 16u) return false;  // a list never fills again
+      const uint32_t lane = __lane_id();
+      bool some = false;
+      if (lane < 8u)
+        some = __hip_atomic_load(take + 64u * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+               brick_positions(ngroups, shift, lane);
+      const uint32_t left = uint32_t(__ballot(some));
+      if (!left) return false;
+      // the first after x
+      const uint32_t turned = (left >> x | left << (8u - x)) & 255u;
+      x = (x + uint32_t(__builtin_ctz(turned))) & 7u;
+      ask();
+      pp = uniform(ahead);
+    }
+    px = x;
+    ask();
+    return true;
+  }
+};
+
+// Occupancy: five waves per SIMD in FP64, six in FP32.
+template <typename R, int MODE>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 5 : 6))) void k_frame(
+    const TessJob* __restrict__ jobs, const uint2* __restrict__ order, uint32_t ngroups, uint32_t shift,
+    uint32_t* __restrict__ take, const RasterJob<R>* __restrict__ rjobs, const uint32_t* __restrict__ jimg,
+    FrameHdr* __restrict__ hdr, uint64_t* __restrict__ key, uint64_t* __restrict__ id, Frag64* __restrict__ frags,
+    uint32_t fcap) {
+  __shared__ FrameLds lds[kThreads / 64];
+  __shared__ uint8_t s_ntri[256];
+  // the id pass runs only after the fragment list overflowed
+  if (MODE == kFrameIds && !(hdr->overflow & 2u)) return;
+  const uint32_t lane = __lane_id(), wave = uniform(threadIdx.x >> 6);
+  FrameLds& S = lds[wave];
+  s_ntri[threadIdx.x] = c_ntri[threadIdx.x];
+  if (lane == 0) {
+    S.fnext = 0;
+    S.fend = 0;
+    S.fchunk = kFragChunk0;
+  }
+  __syncthreads();  // the only barrier
+  const DrawTo D = {key, id, frags, fcap, hdr};
+  Taker T = {take, ngroups, shift, uniform(blockIdx.x & 7u), 0u};
+  T.ask();
+  uint32_t ntri = 0;  // triangles of the cells this lane counted
+  // ring state: oldest item, items queued, and the field pass they belong to
+  // (the queue holds one pass at a time)
+  uint32_t head = 0, npend = 0, cur = 0;
+  for (bool more = true; more;) {
+    uint32_t tx = 0, tp = 0;
+    more = T.next(tx, tp);
+    uint32_t jb = cur, ncut = 0;  // the brick's field pass, and its cut cells
+    BrickBox B = {};
+    if (more) {
+      const uint2 og = order[tx + 8u * (tp >> (3u * shift))];
+      const uint32_t ogx = uniform(og.x), within = tp & ((1u << (3u * shift)) - 1u);
+      jb = ogx & 0x1fffffffu;
+      const FieldDev& f = jobs[jb].f;
+      if (brick_box(jobs[jb].bg, f.ncx, f.ncy, f.ncz, uniform(og.y), within, ogx >> 29, B)) {
+        const uint32_t row = fdiv(lane, jobs[jb].bg.div_bw), col = lane - row * jobs[jb].bg.bw;
+        const uint32_t ci = B.i0 + col, cj = B.j0 + row;
+        const bool valid = ci < B.i1 && cj < B.j1;
+        // plane codes of the lane's cell column, every load independent
+        const uint64_t nxy = uint64_t(f.nx) * f.ny;
+        const C3D_GLOBAL double* p = gptr(f.f) + B.k0 * nxy + uint64_t(cj) * f.nx + ci;
+        const uint32_t points = B.k1 - B.k0 + 1u;
+        if (valid) {
+          for (uint32_t z = 0; z < points; z += 3u) {
+            // three planes in flight; past the last one it is read again
+            double v[3][4];
+            uint32_t zz[3];
+#pragma unroll
+            for (uint32_t u = 0; u < 3u; u++) {
+              zz[u] = z + u < points ? z + u : points - 1u;
+              load_plane4(p + zz[u] * nxy, f.nx, v[u]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 3u; u++) S.pc[zz[u]][lane] = uint16_t(plane_codes(jobs[jb].ts, v[u]));
+          }
+        }
+        // the cells that a threshold cuts: some corner of either kind
+        uint32_t lo = valid ? S.pc[0][lane] : 0u;
+        for (uint32_t z = 0; z + 1u < points; z++) {
+          const uint32_t hi = valid ? S.pc[z + 1u][lane] : 0u;
+          const uint32_t some = lo | hi, all = lo & hi;
+          const uint32_t any = (some | some >> 1 | some >> 2 | some >> 3) & 0x1111u;
+          const bool is_cut = (any & ~(all & all >> 1 & all >> 2 & all >> 3)) != 0u;
+          const uint64_t m = __ballot(is_cut);
+          if (is_cut) S.list[ncut + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = uint16_t(z << 6 | lane);
+          ncut += uint32_t(__popcll(m));
+          lo = hi;
+        }
+        wave_lds_fence();
+      }
+    }
+    uint32_t seen = kAllImages;  // the images that the brick's regular cells may reach
+    bool unseen = false;         // none at all
+    float scale = 0.0f;
+    if constexpr (sizeof(R) == 8) {
+      if (ncut && jobs[jb].f.ordered) {
+        const uint32_t u0 = uniform(jimg[jb]), u1 = uniform(jimg[jb + 1u]);
+        seen = reachable_images(jobs[jb].f, B, rjobs, jimg, u0, u1, key, scale);
+        unseen = u1 - u0 <= kMaskImages && (seen & ((1u << (u1 - u0)) - 1u)) == 0;
+      }
+    }
+    // The pass's constants are read again around every drain, through an
+    // index made opaque: the compiler then loads them (scalar loads from the
+    // constant cache) instead of holding them in scalar registers across the
+    // drain, where the image constants need those registers.
+    const auto job = [&]() -> const TessJob& {
+      uint32_t again = jb;
+      asm volatile("" : "+v"(again));
+      return jobs[uniform(again)];
+    };
+    // round 0 draws what is left of an earlier pass; then 64 listed cells a
+    // round, drawing every full 64 triangles (one drain in the code: it is
+    // large)
+    const bool rest = npend && (!more || jb != cur);
+    const uint32_t rounds = (ncut + 63u) >> 6;
+    for (uint32_t round = rest ? 0u : 1u; round <= rounds; round++) {
+      uint32_t qoff[kMaxThr + 1] = {};
+      if (round) {
+        cur = jb;
+        const TessJob& J = job();
+        const uint32_t at = (round - 1u) * 64u + lane;
+        const bool has = at < ncut;
+        const uint32_t it = S.list[has ? at : 0u], z = it >> 6, c = it & 63u;
+        const uint32_t lo = S.pc[z][c], hi = S.pc[z + 1u][c];
+        const uint32_t row = fdiv(c, J.bg.div_bw);
+        const uint32_t i = B.i0 + c - row * J.bg.bw, j = B.j0 + row, k = B.k0 + z;
+        const bool inner = has && i >= 1u && i + 2u <= J.f.ncx && j >= 1u && j + 2u <= J.f.ncy && k >= 1u &&
+                           k + 2u <= J.f.ncz;
+        uint64_t packed = 0;
+        uint32_t cuts = 0;
+#pragma unroll
+        for (int q = 0; q < kMaxThr; q++) {
+          // codes of thresholds past the last are 0
+          const uint32_t cd = ((lo >> (4 * q)) & 15u) | ((hi >> (4 * q)) & 15u) << 4;
+          const uint32_t nt = has ? s_ntri[cd] : 0u;
+          S.code[q][lane] = uint8_t(cd);
+          ntri += nt;
+          cuts |= nt ? 1u << q : 0u;
+          packed |= uint64_t(nt) << (16 * q);
+        }
+        uint32_t irr = 0;
+        if constexpr (sizeof(R) == 8) {
+          if (seen != kAllImages) {
+            irr = irregular_at(J, i, j, k, cuts, rjobs, jimg, uniform(jimg[cur]), seen, scale, inner);
+            // a brick hidden in every image draws only its irregular cells
+            if (unseen)
+#pragma unroll
+              for (int q = 0; q < kMaxThr; q++)
+                if (!((irr >> q) & 1u)) packed &= ~(uint64_t(0xffffu) << (16 * q));
+          }
+        }
+        // cells outside the rendered interior are counted, not drawn
+        if (!inner) packed = 0;
+        if (!__ballot(packed != 0)) continue;
+        uint64_t end = packed;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const uint64_t y = __shfl_up((unsigned long long)end, d, 64);
+          if (lane >= uint32_t(d)) end += y;
+        }
+        const uint64_t tot = lane_of(end, 63), ex = end - packed;
+#pragma unroll
+        for (int q = 0; q < kMaxThr; q++) {
+          qoff[q + 1] = qoff[q] + (uint32_t(tot >> (16 * q)) & 0xffffu);
+          S.pref[q][lane] = uint16_t(ex >> (16 * q));
+        }
+        S.cell[lane] = (k * J.f.ncy + j) * J.f.ncx + i;
+        S.irr[lane] = uint8_t(irr);
+        wave_lds_fence();
+      }
+      const uint32_t total = qoff[kMaxThr];
+      uint32_t pos = 0;
+      do {
+        // queue as many of the round's triangles as the ring holds
+        const uint32_t room = kWaveRing - npend;
+        const uint32_t put = total - pos < room ? total - pos : room;
+        for (uint32_t e = lane; e < put; e += 64u) {
+          const uint32_t item = pos + e;
+          int q = 0;
+#pragma unroll
+          for (int z = 1; z < kMaxThr; z++) q += item >= qoff[z] ? 1 : 0;
+          uint32_t qsel = 0;
+#pragma unroll
+          for (int z = 1; z < kMaxThr; z++) qsel = q == z ? qoff[z] : qsel;
+          const uint32_t r = item - qsel;
+          uint32_t l = 0;
+#pragma unroll
+          for (uint32_t step = 32; step; step >>= 1) l += S.pref[q][l + step] <= r ? step : 0u;
+          const uint32_t sl = r - S.pref[q][l];
+          const uint32_t s = (head + npend + e) & (kWaveRing - 1u);
+          const uint32_t images = seen != kAllImages && !((S.irr[l] >> q) & 1u) ? seen : kAllImages;
+          S.rc[s] = S.cell[l];
+          S.re[s] = (uint32_t(c_cslot[S.code[q][l] * 12u + sl]) & 0x3ffffu) | uint32_t(q) << 18 | sl << 20 |
+                    images << 24;
+        }
+        pos += put;
+        npend += put;
+        wave_lds_fence();
+        while (npend >= 64u || (round == 0 && npend)) {
+          const uint32_t n = npend < 64u ? npend : 64u;
+          drain_ring<R, MODE>(S, head, n, jobs, uniform(cur), rjobs, jimg, D);
+          head = (head + n) & (kWaveRing - 1u);
+          npend -= n;
+        }
+      } while (pos < total);
+    }
+  }
+  if constexpr (MODE == kFrameDraw) {
+    close_frags(S, frags, fcap);
+    // the frame's triangle count, which no count pass gives it
+#pragma unroll
+    for (int d = 32; d; d >>= 1) ntri += __shfl_xor(ntri, d, 64);
+    if (lane == 0 && ntri)
+      atomicAdd(reinterpret_cast<unsigned long long*>(&hdr->ntri), (unsigned long long)ntri);
+  }
+}
+
+// Before a frame: clears its z-buffer, ids, header and brick counters, and
+// (workgroup b for field pass b) lists the pass's groups of bricks, nearest
+// first: a counting sort over 256 depth bins of the groups' centres, the
+// depth being the reference's z key direction (nrm . (p - cam), larger is
+// nearer) scaled to the lattice's range, the nearest of the images' where a
+// pass is shown in several.  The order decides only how soon the z-buffer
+// fills, never a result.
+constexpr uint32_t kBins = 256;
+
+template <typename R>
+__device__ void order_groups(const TessJob& J, uint32_t jb, const RasterJob<R>* __restrict__ rjobs,
+                             const uint32_t* __restrict__ jimg, uint2* __restrict__ order, uint32_t* s_bin,
+                             uint32_t* s_wave, float (*s_range)[2]) {
+  const FieldDev& f = J.f;
+  const BrickGeo& g = J.bg;
+  const uint32_t ng = brick_groups(g);
+  const auto point = [&](uint32_t i, uint32_t j, uint32_t k) -> V3<R> {
+    if (f.cx) {
+      const uint64_t p = (uint64_t(k) * f.ny + j) * f.nx + i;
+      return {R(gptr(f.cx)[p]), R(gptr(f.cy)[p]), R(gptr(f.cz)[p])};
+    }
+    return {R(gptr(f.gx)[i]), R(gptr(f.gy)[j]), R(gptr(f.gz)[k])};
+  };
+  const auto depth = [&](const ViewDev<R>& v, V3<R> p) {
+    return v.nrm[0] * (p.x - v.cam[0]) + v.nrm[1] * (p.y - v.cam[1]) + v.nrm[2] * (p.z - v.cam[2]);
+  };
+  const uint32_t u0 = jimg[jb], u1 = jimg[jb + 1];
+  // from which end each axis is taken inside a group: the nearer one in the
+  // first image
+  uint32_t flip = 0;
+  if (u0 < u1) {
+    const ViewDev<R>& v = rjobs[jimg[u0]].v;
+    const R d0 = depth(v, point(0, 0, 0));
+    flip = (depth(v, point(f.ncx, 0, 0)) > d0 ? 1u : 0u) | (depth(v, point(0, f.ncy, 0)) > d0 ? 2u : 0u) |
+           (depth(v, point(0, 0, f.ncz)) > d0 ? 4u : 0u);
+  }
+  // depth range of the lattice's corners in each of the first kMaskImages
+  // images (a pass shown in more is ordered for those)
+  const uint32_t nu = u1 - u0 < kMaskImages ? u1 - u0 : kMaskImages;
+  __syncthreads();
+  if (threadIdx.x < nu) {
+    const ViewDev<R>& v = rjobs[jimg[u0 + threadIdx.x]].v;
+    R lo = R(0), hi = R(0);
+    for (uint32_t c = 0; c < 8u; c++) {
+      const R d = depth(v, point(c & 1u ? f.ncx : 0u, c & 2u ? f.ncy : 0u, c & 4u ? f.ncz : 0u));
+      lo = c ? fmin(lo, d) : d;
+      hi = c ? fmax(hi, d) : d;
+    }
+    s_range[threadIdx.x][0] = float(lo);
+    s_range[threadIdx.x][1] = float(kBins) / float(hi - lo);
+  }
+  __syncthreads();
+  const auto bin_of = [&](uint32_t s) {
+    uint32_t x, y, z;
+    group_at(g, s, x, y, z);
+    const auto mid = [&](uint32_t a, uint32_t b, uint32_t n) {
+      const uint32_t m = ((2u * a + 1u) << g.shift) * b / 2u;
+      return m < n ? m : n;
+    };
+    const V3<R> p = point(mid(x, g.bw, f.ncx), mid(y, g.bh, f.ncy), mid(z, g.bz, f.ncz));
+    float best = 0.0f;
+    for (uint32_t u = 0; u < nu; u++)
+      best = fmaxf(best, (float(depth(rjobs[jimg[u0 + u]].v, p)) - s_range[u][0]) * s_range[u][1]);
+    // not a number, or outside the corners' range: an end bin
+    const float t = float(kBins) - best;
+    return t > 0.0f ? (t < float(kBins) ? uint32_t(t) : kBins - 1u) : 0u;
+  };
+  s_bin[threadIdx.x] = 0;
+  __syncthreads();
+  for (uint32_t s = threadIdx.x; s < ng; s += kThreads) atomicAdd(&s_bin[bin_of(s)], 1u);
+  __syncthreads();
+  uint32_t tot;
+  const uint32_t ex = block_excl_scan(s_bin[threadIdx.x], s_wave, tot);
+  s_bin[threadIdx.x] = ex;
+  __syncthreads();
+  for (uint32_t s = threadIdx.x; s < ng; s += kThreads)
+    order[J.group0 + atomicAdd(&s_bin[bin_of(s)], 1u)] = make_uint2(jb | flip << 29, s);
+}
+
+template <typename R>
+__global__ __launch_bounds__(kThreads) void k_frame_begin(const TessJob* __restrict__ jobs, uint32_t njobs,
+                                                          const RasterJob<R>* __restrict__ rjobs,
+                                                          const uint32_t* __restrict__ jimg,
+                                                          uint2* __restrict__ order, uint32_t* __restrict__ take,
+                                                          uint64_t* __restrict__ key, uint64_t* __restrict__ id,
+                                                          uint64_t npx, FrameHdr* __restrict__ hdr) {
+  static_assert(kBins == kThreads, "a bin per thread");
+  __shared__ uint32_t s_bin[kBins], s_wave[kThreads / 64];
+  __shared__ float s_range[kMaskImages][2];
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      hdr->ntri = 0;
+      hdr->nfrag = 0;
+      hdr->overflow = 0;
+    }
+    if (threadIdx.x < 16u) take[64u * threadIdx.x] = 0;
+  }
+  for (uint32_t jb = blockIdx.x; jb < njobs; jb += gridDim.x) {
+    order_groups<R>(jobs[jb], jb, rjobs, jimg, order, s_bin, s_wave, s_range);
+    __syncthreads();
+  }
+  const uint64_t k0 = sizeof(R) == 8 ? 0x0010000000000000ull /* ord64(-DBL_MAX) */ : 0ull;
+  for (uint64_t p = uint64_t(blockIdx.x) * kThreads + threadIdx.x; p < npx; p += uint64_t(gridDim.x) * kThreads) {
+    key[p] = k0;
+    id[p] = 0;
+  }
+}
+
+// ----------------------------------------------------------------------
+// tessellation: emit pass (the stored mesh)
+//
+// The work-item loop of the queue kernels; every drain computes up to 256
+// triangles, one per thread, into records in LDS (a position record and a
+// gather record each), and the workgroup then stores those records at
+// their serial positions as 8-byte words, thread q taking words q, q + 256,
+// ... of each array: the drain's triangles are a few runs of consecutive
+// positions (one per object in the drained chunks), so every store
+// instruction writes contiguous bytes and whole lines, where one store per
+// record field (14 streams) had written scattered 4- or 8-byte pieces.  The
+// stores are non-temporal: the mesh streams past the caches, and the field
+// planes the workgroups march through stay in L2.
+//
+// Every earlier vector memory operation is waited for once before the
+// drain's stores, so that nothing is in flight when they issue: the
+// compiler then issues the store sequence back to back, where otherwise it
+// waited between stores for loads still counted ahead of them.
+
+// The emit's triangle queue: an LDS ring of 12-byte items, drained 256 at a
+// time so that every lane holds a triangle.
+struct EmitLds {
+  uint8_t code[kMaxThr][kThreads];
+  uint16_t pref[kMaxThr][kThreads];
+  uint16_t low[kTileChunks][kThreads];  // lower-plane codes of the tile's cells (cell p at [p / 256][p % 256])
+  uint64_t wave[kThreads / 64];
+  uint8_t ntri[256];
+  uint32_t rg[kRing];  // serial position of the queued triangle
+  uint32_t rc[kRing];  // its cell
+  uint32_t re[kRing];  // its vertices' (tail, head) corners (slot entry bits 0-17) | threshold << 18 |
+                       // slot << 20 | corner code << 24
+};
+
+// The emit's work-item loop: marches each work item's column up its planes,
+// classifies each tile's cells in chunks of 256 (loading only the upper
+// corners: the lower-plane codes carry over from the plane below, in LDS),
+// queues the chunk's triangles in the LDS ring in serial order and calls
+// drain(head, n, jb) for every full 256 items (and for the rest when the
+// field pass changes and at the end).  With kPlanes each plane's upper codes
+// are first computed for the whole tile by column segments (classify_plane,
+// into s_hi: the cells of a segment share their rows of lattice points) and
+// the chunks read them from LDS; the FP32 emit measured 1.5% faster so; the
+// FP64 emit, which would lose a workgroup per CU to the extra LDS, loads
+// each cell's corners itself.  Every cell's corner code of every threshold q
+// is stored at codeout[code_off + q * ncells + cell]: by each cell's thread
+// as bytes (kStoreCode 1) or from LDS as 4-byte words (kStoreCode 2;
+// measured faster in the FP64 emit, slower in the FP32 one).  Expects S.ntri
+// loaded and a barrier since.
+template <int kStoreCode, bool kPlanes, typename Drain>
+__device__ __forceinline__ void ring_tiles(EmitLds& S, uint16_t* s_hi, const TessJob* __restrict__ jobs, int njobs,
                                            uint32_t nitems, const uint64_t* __restrict__ start,
-                                           uint32_t* __restrict__ cellout, uint64_t cap, uint8_t* __restrict__ codeout,
-                                           Drain&& drain) {
+                                           uint8_t* __restrict__ codeout, Drain&& drain) {
   // ring state, the same in every thread: oldest item, items queued, and
   // the field pass they belong to
   uint32_t head = 0, npend = 0, cur = 0;
@@ -1199,20 +1770,11 @@ __device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const Te
       npend -= n;
     }
     cur = jb;
-    // The pass's field and thresholds are read through jbx, which with
-    // kReload is made opaque after every drain: the compiler then reloads
-    // them (scalar loads from the constant cache) instead of holding them in
-    // scalar registers across the drain, where the fused kernel's image
-    // constants need those registers (it had spilled scalars to vector lanes
-    // at twice the rate; the frames got 2-3.5% faster, the emit, whose
-    // drains hold no image constants, 3% slower).
-    uint32_t jbx = jb;
-    const auto Fd = [&]() -> const FieldDev& { return jobs[jbx].f; };
-    const auto Ts = [&]() -> const ThrSet& { return jobs[jbx].ts; };
+    const auto Fd = [&]() -> const FieldDev& { return jobs[jb].f; };
+    const auto Ts = [&]() -> const ThrSet& { return jobs[jb].ts; };
     uint32_t col, k0, k1;
     item_range(Fd(), item, col, k0, k1);
-    // the tile's span and plane strides, recomputed from the pass (and so
-    // after a drain) rather than held
+    // the tile's span and plane strides, recomputed from the pass
     const auto Tsp = [&]() { return tile_span(Fd(), k0, col); };
     const uint32_t nch = (Tsp().n + kThreads - 1) / kThreads;
     const auto nxy = [&]() { return uint64_t(Fd().nx) * Fd().ny; };
@@ -1244,7 +1806,7 @@ __device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const Te
       }
       uint64_t base[kMaxThr];
 #pragma unroll
-      for (int q = 0; q < kMaxThr; q++) base[q] = kSerial && q < Ts().n ? start[Ts().boff[q] + tile] : 0;
+      for (int q = 0; q < kMaxThr; q++) base[q] = q < Ts().n ? start[Ts().boff[q] + tile] : 0;
       for (uint32_t ch = 0; ch < nch; ch++) {
         const uint32_t c0 = ctile + ch * kThreads;
         const uint32_t p = ch * kThreads + threadIdx.x;
@@ -1333,14 +1895,10 @@ __device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const Te
             const uint32_t cc = c0 + l;
             const uint32_t cd = S.code[q][l];
             const uint32_t s = (head + npend + e) & (kRing - 1u);
-            if constexpr (kSerial) {
-              uint64_t bq = base[0];
+            uint64_t bq = base[0];
 #pragma unroll
-              for (int z = 1; z < kMaxThr; z++) bq = q == z ? base[z] : bq;
-              const uint64_t g = bq + r;
-              if (kStoreCell && g < cap) cellout[g] = cc;
-              S.rg[s] = uint32_t(g);
-            }
+            for (int z = 1; z < kMaxThr; z++) bq = q == z ? base[z] : bq;
+            S.rg[s] = uint32_t(bq + r);
             S.rc[s] = cc;
             S.re[s] = (uint32_t(c_cslot[cd * 12u + sl]) & 0x3ffffu) | uint32_t(q) << 18 | sl << 20 | cd << 24;
           }
@@ -1349,7 +1907,6 @@ __device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const Te
           __syncthreads();
           while (npend >= kThreads) {
             drain(head, kThreads, jb);
-            if constexpr (kReload) asm volatile("" : "+s"(jbx));
             head = (head + kThreads) & (kRing - 1u);
             npend -= kThreads;
           }
@@ -1368,66 +1925,9 @@ __device__ __forceinline__ void ring_tiles(FusedLds& S, uint16_t* s_hi, const Te
   }
 }
 
-// Occupancy: the FP64 form runs five waves per SIMD (its LDS allows no
-// more), the FP32 form seven (72 VGPRs, no spill; 3% faster than six).
-template <typename R, int MODE>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 || MODE == kRasterAppend ? 5 : 7))) void
-k_tess_raster(const TessJob* __restrict__ jobs, int njobs, uint32_t nitems, const uint64_t* __restrict__ start,
-              uint32_t* __restrict__ cellout, uint64_t cap, const RasterJob<R>* __restrict__ rjobs,
-              const uint32_t* __restrict__ jimg, FrameHdr* __restrict__ hdr, uint64_t* __restrict__ key,
-              void* __restrict__ idv, void* __restrict__ fragv, uint32_t fcap) {
-  static_assert(MODE != kRasterDepth64, "the fused kernel keeps every fragment (kRasterAppend)");
-  // FP64 frames name triangles by tri_id64, FP32 ones by serial position
-  using TId = typename std::conditional<sizeof(R) == 8, uint64_t, uint32_t>::type;
-  constexpr bool kSerial = sizeof(R) == 4;
-  TId* id = static_cast<TId*>(idv);
-  FragOf<TId>* frags = static_cast<FragOf<TId>*>(fragv);
-  constexpr bool kPlanes = true;
-  __shared__ FusedLds S;
-  __shared__ uint16_t s_hi[kPlanes ? kTileCells : 1];
-  __shared__ FragOf<TId> s_frag[MODE == kRasterAppend ? kFragLdsFused : 1];
-  if (hdr->overflow & 1u) return;
-  // the FP64 z-test passes run only after the fragment list overflowed
-  if ((MODE == kRasterKey64 || MODE == kRasterId64) && !(hdr->overflow & 2u)) return;
-  S.ntri[threadIdx.x] = c_ntri[threadIdx.x];
-  if (threadIdx.x == 0) S.nfrag = 0;
-  __syncthreads();
-  uint64_t ndrawn = 0;  // triangles drained (the same in every thread)
-  // the first pass of an FP32 frame stores the cell indices
-  ring_tiles<kSerial && (MODE == kRasterAppend || MODE == kRasterFp32), 0, true, kPlanes, kSerial>(
-      S, s_hi, jobs, njobs, nitems, start, cellout, cap, nullptr, [&](uint32_t head, uint32_t n, uint32_t jb) {
-        ndrawn += n;
-        drain_ring<R, MODE, TId>(S, s_frag, head, n, jobs, jb, rjobs, jimg, hdr, key, id, frags, fcap);
-      });
-  flush_frags<MODE>(S, s_frag, hdr, frags, fcap, true);
-  // an FP64 frame's triangle count, which no count pass gives it
-  if (!kSerial && MODE == kRasterAppend && threadIdx.x == 0 && ndrawn)
-    atomicAdd(reinterpret_cast<unsigned long long*>(&hdr->ntri), (unsigned long long)ndrawn);
-}
-
-// ----------------------------------------------------------------------
-// tessellation: emit pass (the stored mesh)
-//
-// The work-item loop of the queue kernels; every drain computes up to 256
-// triangles, one per thread, into records in LDS (a position record and a
-// gather record each), and the workgroup then stores those records at
-// their serial positions as 8-byte words, thread q taking words q, q + 256,
-// ... of each array: the drain's triangles are a few runs of consecutive
-// positions (one per object in the drained chunks), so every store
-// instruction writes contiguous bytes and whole lines, where one store per
-// record field (14 streams) had written scattered 4- or 8-byte pieces.  The
-// stores are non-temporal: the mesh streams past the caches, and the field
-// planes the workgroups march through stay in L2.
-//
-// Every earlier vector memory operation is waited for once before the
-// drain's stores, so that nothing is in flight when they issue: the
-// compiler then issues the store sequence back to back, where otherwise it
-// waited between stores for loads still counted ahead of them.
-
 // stores n records of type Rec from LDS at the drain's serial positions
 template <typename Rec>
-__device__ __forceinline__ void store_drain(const FusedLds& S, const Rec* s_src, uint32_t head, uint32_t n,
+__device__ __forceinline__ void store_drain(const EmitLds& S, const Rec* s_src, uint32_t head, uint32_t n,
                                             Rec* out, uint64_t cap) {
   constexpr uint32_t kWords = sizeof(Rec) / 8u;
   const uint64_t* src = reinterpret_cast<const uint64_t*>(s_src);
@@ -1442,7 +1942,7 @@ __device__ __forceinline__ void store_drain(const FusedLds& S, const Rec* s_src,
 }
 
 template <typename R>
-__device__ __forceinline__ void emit_ring(FusedLds& S, MeshPos<R>* s_pos, MeshAux<R>* s_aux, uint32_t head,
+__device__ __forceinline__ void emit_ring(EmitLds& S, MeshPos<R>* s_pos, MeshAux<R>* s_aux, uint32_t head,
                                           uint32_t n, const TessJob* __restrict__ jobs, uint32_t jb,
                                           const MeshView<R>& m, FrameHdr* __restrict__ hdr) {
   if (threadIdx.x < n) {
@@ -1484,55 +1984,38 @@ template <typename R>
 __global__ __launch_bounds__(kThreads) void k_emit(const TessJob* __restrict__ jobs, int njobs, uint32_t nitems,
                                                    const uint64_t* __restrict__ start, MeshView<R> m,
                                                    FrameHdr* __restrict__ hdr) {
-  __shared__ FusedLds S;
+  __shared__ EmitLds S;
   __shared__ MeshPos<R> s_pos[kThreads];
   __shared__ MeshAux<R> s_aux[kThreads];
   constexpr bool kPl = sizeof(R) == 4;  // the FP64 build would lose a workgroup per CU to the LDS
   __shared__ uint16_t s_hi[kPl ? kTileCells : 1];
   S.ntri[threadIdx.x] = c_ntri[threadIdx.x];
   __syncthreads();
-  ring_tiles<false, sizeof(R) == 8 ? 2 : 1, false, kPl, true>(S, s_hi, jobs, njobs, nitems, start, nullptr, 0, m.code,
-                                                          [&](uint32_t head, uint32_t n, uint32_t jb) {
+  ring_tiles<sizeof(R) == 8 ? 2 : 1, kPl>(S, s_hi, jobs, njobs, nitems, start, m.code, [&](uint32_t head, uint32_t n, uint32_t jb) {
     emit_ring<R>(S, s_pos, s_aux, head, n, jobs, jb, m, hdr);
   });
 }
 
 // the latest triangle among the kept fragments at each pixel's final depth
-template <typename TId>
-__global__ void k_frag_ids(const FragOf<TId>* __restrict__ frags, uint32_t cap, const FrameHdr* __restrict__ hdr,
+template <typename FT, typename TId>
+__global__ void k_frag_ids(const FT* __restrict__ frags, uint32_t cap, const FrameHdr* __restrict__ hdr,
                            const uint64_t* __restrict__ key, TId* __restrict__ id) {
   if (hdr->overflow & 2u) return;
   const uint32_t n = min(hdr->nfrag, cap);
   for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < n; f += gridDim.x * blockDim.x) {
-    const FragOf<TId> fr = frags[f];
+    const FT fr = frags[f];
+    if (sizeof(TId) == 8 && fr.px == kNoPixel) continue;
     if (fr.key == key[fr.px]) atomic_max_id(id + fr.px, fr.id);
   }
 }
 
-// the z-buffer keys of every listed fragment
-template <typename FT>
-__global__ void k_frag_keys(const FT* __restrict__ frags, uint32_t cap, const FrameHdr* __restrict__ hdr,
-                            uint64_t* __restrict__ key) {
-  if (hdr->overflow & 2u) return;
-  const uint32_t n = min(hdr->nfrag, cap);
-  for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < n; f += gridDim.x * blockDim.x) {
-    const uint64_t fkey = frags[f].key;
-    const uint32_t fpx = frags[f].px;
-    // keys only grow, so a value read here (however stale) that is at least
-    // this key means the atomic could not change the pixel: skip it
-    if (fkey > key[fpx]) atomicMax(reinterpret_cast<unsigned long long*>(key + fpx), (unsigned long long)fkey);
-  }
-}
-
-// also clears the frame header's raster state (fragment count, list
-// overflow) and, fresh, its triangle count and capacity bit
-template <typename TId>
-__global__ void k_zinit(uint64_t* __restrict__ key, TId* __restrict__ id, uint64_t npx, uint64_t k0, bool fresh,
+// Before a stored mesh is rendered: clears the z-buffer, the ids and the
+// frame header's raster state.
+__global__ void k_zinit(uint64_t* __restrict__ key, uint32_t* __restrict__ id, uint64_t npx, uint64_t k0,
                         FrameHdr* __restrict__ hdr) {
-  if (hdr && blockIdx.x == 0 && threadIdx.x == 0) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     hdr->nfrag = 0;
-    hdr->overflow &= fresh ? 0u : 1u;
-    if (fresh) hdr->ntri = 0;
+    hdr->overflow &= 1u;
   }
   for (uint64_t p = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; p < npx; p += uint64_t(gridDim.x) * blockDim.x) {
     key[p] = k0;
@@ -1551,12 +2034,13 @@ __global__ void k_line_frags(const uint32_t* __restrict__ pix, const double* __r
   if (f >= hdr->nline) return;
   const uint32_t px = pix[f];
   const TId lid = sizeof(TId) == 8 ? TId(kLineObj << 40 | f) : TId(hdr->ntri + 1 + f);
-  if (fp32) {
+  if (sizeof(TId) == 4 && fp32) {
+    // a stored FP32 mesh: one pass, the key carries the id
     const uint64_t k = uint64_t(ord32(float(depth[f]))) << 32 | uint64_t(lid);
     atomicMax(reinterpret_cast<unsigned long long*>(key + px), (unsigned long long)k);
     return;
   }
-  const uint64_t k = ord64(depth[f]);
+  const uint64_t k = fp32 ? depth_key(float(depth[f])) : depth_key(depth[f]);
   if (pass == 0) {
     atomicMax(reinterpret_cast<unsigned long long*>(key + px), (unsigned long long)k);
   } else if (k == __hip_atomic_load(key + px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
@@ -1689,11 +2173,6 @@ struct WaveHits {
   R w[64][3];
 };
 
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // The winning triangle of one pixel, as phase 1 leaves it for phase 3.
 template <typename R>
 struct PixelTri {
@@ -1713,63 +2192,30 @@ __device__ __forceinline__ void weights_at(const ViewDev<R>& v, const V3<R> p[3]
   pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), X.w0, X.w1, X.w2);
 }
 
-// A frame without a stored mesh: triangles are found from their ids (FP64:
-// the object, cell and slot fields of tri_id64; FP32, a serial id: the
-// object among the image's objects by base, the cell from the stored cell
-// index, the slot from the cell store's neighbouring entries) and
-// recomputed from the field.
+// A frame without a stored mesh: triangles are found from their ids (the
+// object, cell and slot fields of tri_id64) and recomputed from the field.
 template <typename R>
 struct FieldSource {
   const TessJob* __restrict__ jobs;
-  const uint32_t* __restrict__ cell;
   const ObjMeta* __restrict__ meta;
-  const void* __restrict__ idv;
+  const uint64_t* __restrict__ ids;
 
   // the winner at pixel p with key k: a triangle (obj, cell c, slot sl), a
   // line fragment (fi) or neither
-  __device__ __forceinline__ void winner(const RasterJob<R>& J, uint64_t ntri, uint64_t p, uint64_t k, bool& tri,
+  __device__ __forceinline__ void winner(const RasterJob<R>& J, uint64_t, uint64_t p, uint64_t k, bool& tri,
                                          bool& line, uint32_t& obj, uint32_t& c, uint32_t& sl, uint64_t& fi,
                                          double& dep) const {
-    if constexpr (sizeof(R) == 8) {
-      // tri_id64: (object + 1) << 40 | cell << 4 | slot
-      const uint64_t id = static_cast<const uint64_t*>(idv)[p];
-      dep = unord64(k);
-      const uint64_t ob = id >> 40;
-      line = ob == kLineObj;
-      fi = id & ((uint64_t(1) << 40) - 1u);
-      tri = id != 0 && !line && ob - 1u >= J.obj0 && ob - 1u < J.obj1;
-      obj = uint32_t(ob - 1u);
-      c = uint32_t(id >> 4);
-      sl = uint32_t(id & 15u);
-    } else {
-      const uint32_t id = uint32_t(k);
-      dep = id ? double(unord32(uint32_t(k >> 32))) : -DBL_MAX;
-      line = id > ntri;
-      fi = id - ntri - 1;
-      if (id != 0 && id <= ntri && J.obj0 < J.obj1) {
-        const uint64_t t = id - 1;
-        // the winner is one of the image's own objects
-        int lo = int(J.obj0), hi = int(J.obj1) - 1;
-        while (lo < hi) {
-          const int mid = (lo + hi + 1) >> 1;
-          if (meta[mid].base <= t) lo = mid;
-          else hi = mid - 1;
-        }
-        obj = uint32_t(lo);
-        const uint64_t base = meta[lo].base;
-        c = cell[t];
-        // Within an object the cells ascend with the serial position and
-        // a cell has at most 12 triangles, so the slot of t is the number
-        // of the 11 positions before it, inside the object, that hold the
-        // same cell.  The 11 loads are independent and share one or two
-        // lines.
-#pragma unroll
-        for (uint32_t d = 1; d < 12; d++) sl += t >= base + d && cell[t - d] == c ? 1u : 0u;
-        // a position outside the object can only come from a damaged cell
-        // store: such a pixel keeps the background
-        tri = t >= base && t - base < meta[lo].count;
-      }
-    }
+    // tri_id64: (object + 1) << 40 | cell << 4 | slot
+    const uint64_t id = ids[p];
+    if constexpr (sizeof(R) == 8) dep = unord64(k);
+    else dep = id ? double(unord32(uint32_t(k >> 32))) : -DBL_MAX;
+    const uint64_t ob = id >> 40;
+    line = ob == kLineObj;
+    fi = id & ((uint64_t(1) << 40) - 1u);
+    tri = id != 0 && !line && ob - 1u >= J.obj0 && ob - 1u < J.obj1;
+    obj = uint32_t(ob - 1u);
+    c = uint32_t(id >> 4);
+    sl = uint32_t(id & 15u);
   }
 
   // phase 1 of the wave's pixels with a winning triangle (have)
@@ -1784,7 +2230,7 @@ struct FieldSource {
       todo &= ~__ballot(mine);
       const FieldDev& f = jobs[jb].f;
       // a cell index outside the object's field or its interior, or a slot
-      // outside its cell, can only come from a damaged id or cell store:
+      // outside its cell, can only come from a damaged id buffer:
       // such a pixel keeps the background rather than read out of bounds
       if (!mine || c >= f.ncells) continue;
       const double thr = jobs[jb].ts.thr[meta[obj].q & 3u];
@@ -2021,9 +2467,10 @@ __device__ __forceinline__ void resolve_tile(const Source& src, VtxTable<R>& T, 
 template <typename R, typename Source>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_resolve(
     Source src, const RasterJob<R>* __restrict__ rjobs, int njobs, uint32_t ntiles,
-    const uint8_t* __restrict__ frag_rgb, const FrameHdr* __restrict__ hdr, const uint64_t* __restrict__ key) {
-  // a frame whose triangles outgrew the cell store is rendered again: skip it
-  if (hdr->overflow & 1u) return;
+    const uint8_t* __restrict__ frag_rgb, const FrameHdr* __restrict__ hdr, const uint64_t* __restrict__ key,
+    uint64_t max_tri) {
+  // a frame of more triangles than it may hold is refused: write nothing
+  if ((hdr->overflow & 1u) || hdr->ntri > max_tri) return;
   __shared__ VtxTable<R> T;
   __shared__ WaveHits<R> hits[kThreads / 64];
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
@@ -2103,14 +2550,9 @@ hipError_t launch_vertex_normals(const MeshView<R>& m, const ObjMeta* meta_dev, 
   return hipGetLastError();
 }
 
-hipError_t launch_zinit(uint64_t* key, void* id, bool wide, uint64_t npx, int precision, bool fresh, FrameHdr* hdr,
-                        hipStream_t st) {
+hipError_t launch_zinit(uint64_t* key, uint32_t* id, uint64_t npx, int precision, FrameHdr* hdr, hipStream_t st) {
   const uint64_t k0 = precision == 0 ? 0x0010000000000000ull /* ord64(-DBL_MAX) */ : 0ull;
-  const dim3 g(grid8((npx + 255) / 256, 4096));
-  if (wide)
-    hipLaunchKernelGGL(k_zinit<uint64_t>, g, dim3(256), 0, st, key, static_cast<uint64_t*>(id), npx, k0, fresh, hdr);
-  else
-    hipLaunchKernelGGL(k_zinit<uint32_t>, g, dim3(256), 0, st, key, static_cast<uint32_t*>(id), npx, k0, fresh, hdr);
+  hipLaunchKernelGGL(k_zinit, dim3(grid8((npx + 255) / 256, 4096)), dim3(256), 0, st, key, id, npx, k0, hdr);
   return hipGetLastError();
 }
 
@@ -2131,25 +2573,14 @@ hipError_t launch_raster(const MeshView<R>& m, const RasterJob<R>* rjobs, int nj
   return hipGetLastError();
 }
 
-hipError_t launch_frag_keys(const void* frags, bool wide, uint32_t cap, const FrameHdr* hdr, uint64_t* key,
-                            uint32_t grid, hipStream_t st) {
-  if (wide)
-    hipLaunchKernelGGL(k_frag_keys<Frag64>, dim3(grid), dim3(256), 0, st, static_cast<const Frag64*>(frags), cap, hdr,
-                       key);
-  else
-    hipLaunchKernelGGL(k_frag_keys<Frag>, dim3(grid), dim3(256), 0, st, static_cast<const Frag*>(frags), cap, hdr,
-                       key);
-  return hipGetLastError();
-}
-
 hipError_t launch_frag_ids(const void* frags, bool wide, uint32_t cap, const FrameHdr* hdr, const uint64_t* key,
                            void* id, uint32_t grid, hipStream_t st) {
   if (wide)
-    hipLaunchKernelGGL(k_frag_ids<uint64_t>, dim3(grid), dim3(256), 0, st, static_cast<const Frag64*>(frags), cap,
-                       hdr, key, static_cast<uint64_t*>(id));
+    hipLaunchKernelGGL((k_frag_ids<Frag64, uint64_t>), dim3(grid), dim3(256), 0, st, static_cast<const Frag64*>(frags),
+                       cap, hdr, key, static_cast<uint64_t*>(id));
   else
-    hipLaunchKernelGGL(k_frag_ids<uint32_t>, dim3(grid), dim3(256), 0, st, static_cast<const Frag*>(frags), cap, hdr,
-                       key, static_cast<uint32_t*>(id));
+    hipLaunchKernelGGL((k_frag_ids<Frag, uint32_t>), dim3(grid), dim3(256), 0, st, static_cast<const Frag*>(frags), cap,
+                       hdr, key, static_cast<uint32_t*>(id));
   return hipGetLastError();
 }
 
@@ -2179,7 +2610,7 @@ hipError_t launch_resolve(const MeshView<R>& m, const RasterJob<R>* rjobs, int n
                           const uint64_t* key, const uint32_t* id, hipStream_t st) {
   const MeshSource<R> src = {m, meta, nobj, id};
   hipLaunchKernelGGL((k_resolve<R, MeshSource<R>>), resolve_grid(ntiles), dim3(kThreads), 0, st, src, rjobs, njobs,
-                     ntiles, frag_rgb, hdr, key);
+                     ntiles, frag_rgb, hdr, key, ~uint64_t(0));
   return hipGetLastError();
 }
 
@@ -2197,53 +2628,57 @@ hipError_t launch_mesh_compare(const MeshView<double>& a, const ObjMeta* ma, con
 }
 
 template <typename R>
-hipError_t launch_tess_raster(const TessJob* jobs, int njobs, uint32_t nitems, const uint64_t* start, uint32_t* cell,
-                              uint64_t cap, const RasterJob<R>* rjobs, const uint32_t* jimg, FrameHdr* hdr, int mode,
-                              uint64_t* key, void* id, void* frags, uint32_t fcap, uint32_t grid, hipStream_t st) {
-  if (nitems == 0) return hipSuccess;
-  const dim3 g(grid8(nitems, grid));
-  if (mode == kRasterAppend) {
-    hipLaunchKernelGGL((k_tess_raster<R, kRasterAppend>), g, dim3(kThreads), 0, st, jobs, njobs, nitems, start, cell,
-                       cap, rjobs, jimg, hdr, key, id, frags, fcap);
-  } else if constexpr (sizeof(R) == 4) {
-    if (mode != kRasterFp32) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_tess_raster<R, kRasterFp32>), g, dim3(kThreads), 0, st, jobs, njobs, nitems, start, cell, cap,
-                       rjobs, jimg, hdr, key, id, frags, fcap);
-  } else {
-    if (mode == kRasterKey64)
-      hipLaunchKernelGGL((k_tess_raster<R, kRasterKey64>), g, dim3(kThreads), 0, st, jobs, njobs, nitems, start, cell,
-                         cap, rjobs, jimg, hdr, key, id, frags, fcap);
-    else if (mode == kRasterId64)
-      hipLaunchKernelGGL((k_tess_raster<R, kRasterId64>), g, dim3(kThreads), 0, st, jobs, njobs, nitems, start, cell,
-                         cap, rjobs, jimg, hdr, key, id, frags, fcap);
-    else
-      return hipErrorInvalidValue;
-  }
+hipError_t launch_frame_begin(const TessJob* jobs, int njobs, const RasterJob<R>* rjobs, const uint32_t* jimg,
+                              uint2* order, uint32_t* take, uint64_t* key, uint64_t* id, uint64_t npx, FrameHdr* hdr,
+                              hipStream_t st) {
+  const uint64_t want = (npx + kThreads - 1) / kThreads;
+  hipLaunchKernelGGL(k_frame_begin<R>, dim3(grid8(want > uint64_t(njobs) ? want : uint64_t(njobs), 4096)),
+                     dim3(kThreads), 0, st, jobs, uint32_t(njobs), rjobs, jimg, order, take, key, id, npx, hdr);
   return hipGetLastError();
 }
 
 template <typename R>
-hipError_t launch_resolve_field(const TessJob* jobs, const uint32_t* cell, const RasterJob<R>* rjobs, int njobs,
-                                uint32_t ntiles, const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr,
-                                const uint64_t* key, const void* id, hipStream_t st) {
-  const FieldSource<R> src = {jobs, cell, meta, id};
-  hipLaunchKernelGGL((k_resolve<R, FieldSource<R>>), resolve_grid(ntiles), dim3(kThreads), 0, st, src, rjobs, njobs,
-                     ntiles, frag_rgb, hdr, key);
+hipError_t launch_frame(const TessJob* jobs, const uint2* order, uint32_t ngroups, uint32_t shift, uint32_t* take,
+                        const RasterJob<R>* rjobs, const uint32_t* jimg, FrameHdr* hdr, int mode, uint64_t* key,
+                        uint64_t* id, Frag64* frags, uint32_t fcap, uint32_t grid, hipStream_t st) {
+  if (ngroups == 0) return hipSuccess;
+  const uint64_t bricks = uint64_t(ngroups) << (3 * shift);
+  const dim3 g(grid8((bricks + kThreads / 64 - 1) / (kThreads / 64), grid));
+  if (mode == kFrameDraw)
+    hipLaunchKernelGGL((k_frame<R, kFrameDraw>), g, dim3(kThreads), 0, st, jobs, order, ngroups, shift, take, rjobs,
+                       jimg, hdr, key, id, frags, fcap);
+  else
+    hipLaunchKernelGGL((k_frame<R, kFrameIds>), g, dim3(kThreads), 0, st, jobs, order, ngroups, shift,
+                       take + 64 * 8, rjobs, jimg, hdr, key, id, frags, fcap);
   return hipGetLastError();
 }
 
-template hipError_t launch_tess_raster<double>(const TessJob*, int, uint32_t, const uint64_t*, uint32_t*, uint64_t,
-                                               const RasterJob<double>*, const uint32_t*, FrameHdr*, int, uint64_t*,
-                                               void*, void*, uint32_t, uint32_t, hipStream_t);
-template hipError_t launch_tess_raster<float>(const TessJob*, int, uint32_t, const uint64_t*, uint32_t*, uint64_t,
-                                              const RasterJob<float>*, const uint32_t*, FrameHdr*, int, uint64_t*,
-                                              void*, void*, uint32_t, uint32_t, hipStream_t);
-template hipError_t launch_resolve_field<double>(const TessJob*, const uint32_t*, const RasterJob<double>*, int, uint32_t,
-                                                 const ObjMeta*, const uint8_t*, const FrameHdr*, const uint64_t*,
-                                                 const void*, hipStream_t);
-template hipError_t launch_resolve_field<float>(const TessJob*, const uint32_t*, const RasterJob<float>*, int, uint32_t,
-                                                 const ObjMeta*, const uint8_t*, const FrameHdr*, const uint64_t*,
-                                                 const void*, hipStream_t);
+template <typename R>
+hipError_t launch_resolve_field(const TessJob* jobs, const RasterJob<R>* rjobs, int njobs, uint32_t ntiles,
+                                const ObjMeta* meta, const uint8_t* frag_rgb, const FrameHdr* hdr, const uint64_t* key,
+                                const uint64_t* id, uint64_t max_tri, hipStream_t st) {
+  const FieldSource<R> src = {jobs, meta, id};
+  hipLaunchKernelGGL((k_resolve<R, FieldSource<R>>), resolve_grid(ntiles), dim3(kThreads), 0, st, src, rjobs, njobs,
+                     ntiles, frag_rgb, hdr, key, max_tri);
+  return hipGetLastError();
+}
+
+template hipError_t launch_frame_begin<double>(const TessJob*, int, const RasterJob<double>*, const uint32_t*, uint2*,
+                                               uint32_t*, uint64_t*, uint64_t*, uint64_t, FrameHdr*, hipStream_t);
+template hipError_t launch_frame<double>(const TessJob*, const uint2*, uint32_t, uint32_t, uint32_t*,
+                                         const RasterJob<double>*, const uint32_t*, FrameHdr*, int, uint64_t*, uint64_t*,
+                                         Frag64*, uint32_t, uint32_t, hipStream_t);
+template hipError_t launch_resolve_field<double>(const TessJob*, const RasterJob<double>*, int, uint32_t, const ObjMeta*,
+                                                 const uint8_t*, const FrameHdr*, const uint64_t*, const uint64_t*,
+                                                 uint64_t, hipStream_t);
+template hipError_t launch_frame_begin<float>(const TessJob*, int, const RasterJob<float>*, const uint32_t*, uint2*,
+                                               uint32_t*, uint64_t*, uint64_t*, uint64_t, FrameHdr*, hipStream_t);
+template hipError_t launch_frame<float>(const TessJob*, const uint2*, uint32_t, uint32_t, uint32_t*,
+                                         const RasterJob<float>*, const uint32_t*, FrameHdr*, int, uint64_t*, uint64_t*,
+                                         Frag64*, uint32_t, uint32_t, hipStream_t);
+template hipError_t launch_resolve_field<float>(const TessJob*, const RasterJob<float>*, int, uint32_t, const ObjMeta*,
+                                                 const uint8_t*, const FrameHdr*, const uint64_t*, const uint64_t*,
+                                                 uint64_t, hipStream_t);
 template hipError_t launch_plan<double>(const uint64_t*, uint64_t, ObjMeta*, int, RasterJob<double>*, int, FrameHdr*,
                                         uint64_t, hipStream_t);
 template hipError_t launch_plan<float>(const uint64_t*, uint64_t, ObjMeta*, int, RasterJob<float>*, int, FrameHdr*,
