@@ -1282,14 +1282,14 @@ __device__ __forceinline__ bool box_above(const uint64_t* __restrict__ key, uint
 // that regular cells of brick B may still reach; scale gets the others'
 // area scale (lane u holds image u's).  The corners' views are formed by
 // lanes 0-7 (and every other eight lanes alike).
-__device__ __forceinline__ uint32_t reachable_images(const FieldDev& f, const BrickBox& B,
+__device__ __forceinline__ uint32_t reachable_images(const FieldDev& f, BrickBox B,
                                                      const RasterJob<double>* __restrict__ rjobs,
                                                      const uint32_t* __restrict__ jimg, uint32_t u0, uint32_t u1,
                                                      const uint64_t* __restrict__ key, float& scale) {
   uint32_t seen = kAllImages;
   const uint32_t c = __lane_id() & 7u;
-  const double px = gptr(f.gx)[c & 1u ? B.i1 : B.i0], py = gptr(f.gy)[c & 2u ? B.j1 : B.j0],
-               pz = gptr(f.gz)[c & 4u ? B.k1 : B.k0];
+  const double px = gptr(f.gx)[B.i0 + (c & 1u) * (B.i1 - B.i0)], py = gptr(f.gy)[B.j0 + (c >> 1 & 1u) * (B.j1 - B.j0)],
+               pz = gptr(f.gz)[B.k0 + (c >> 2) * (B.k1 - B.k0)];
   for (uint32_t u = u0; u < u1 && u - u0 < kMaskImages; u++) {
     const RasterJob<double>& J = rjobs[uniform(jimg[u])];
     CornerView cv;
@@ -1358,46 +1358,45 @@ __device__ __forceinline__ uint32_t irregular_at(const TessJob& J, uint32_t i, u
   return bad;
 }
 
-// Takes bricks for a wave, from XCD list x, and from another list once that
-// one is empty; each is asked for while the one before is worked on.  The
-// lists' counters are `take`, 64 words apart.
-struct Taker {
-  uint32_t* __restrict__ take;
-  uint32_t ngroups, shift;
-  uint32_t x;
-  uint32_t ahead;  // lane 0: the position asked for
+// Bricks are taken one by one from XCD list x, and from another list once
+// that one is empty; each is asked for while the one before is worked on.
+// The lists' counters are `take`, 64 words apart.  ask_brick gives lane 0 a
+// position of list x; next_brick gives the wave the position asked for
+// (`ahead`), or one of the first other list that still has some, in p, and
+// asks for the next; false when every list is empty.
+__device__ __forceinline__ uint32_t ask_brick(uint32_t* __restrict__ take, uint32_t x) {
+  uint32_t p = 0;
+  if (__lane_id() == 0) p = atomicAdd(take + 64u * x, 1u);
+  return p;
+}
 
-  __device__ __forceinline__ void ask() {
-    if (__lane_id() == 0) ahead = atomicAdd(take + 64u * x, 1u);
+__device__ __forceinline__ bool next_brick(uint32_t* __restrict__ take, uint32_t ngroups, uint32_t shift, uint32_t& x,
+                                           uint32_t& ahead, uint32_t& from, uint32_t& p) {
+  p = uniform(ahead);
+  for (uint32_t tried = 0; p >= brick_positions(ngroups, shift, x); tried++) {
+    if (tried == 16u) return false;  // a list never fills again
+    const uint32_t lane = __lane_id();
+    bool some = false;
+    if (lane < 8u)
+      some = __hip_atomic_load(take + 64u * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+             brick_positions(ngroups, shift, lane);
+    const uint32_t left = uint32_t(__ballot(some));
+    if (!left) return false;
+    // the first after x
+    const uint32_t turned = (left >> x | left << (8u - x)) & 255u;
+    x = uniform((x + uint32_t(__builtin_ctz(turned))) & 7u);
+    p = uniform(ask_brick(take, x));
   }
-  // the brick asked for, or one from the first other list that still has
-  // some; false when all are empty.  The next one is asked for at once.
-  __device__ __forceinline__ bool next(uint32_t& px, uint32_t& pp) {
-    pp = uniform(ahead);
-    for (uint32_t tried = 0; pp >= brick_positions(ngroups, shift, x); tried++) {
-      if (tried == 16u) return false;  // a list never fills again
-      const uint32_t lane = __lane_id();
-      bool some = false;
-      if (lane < 8u)
-        some = __hip_atomic_load(take + 64u * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-               brick_positions(ngroups, shift, lane);
-      const uint32_t left = uint32_t(__ballot(some));
-      if (!left) return false;
-      // the first after x
-      const uint32_t turned = (left >> x | left << (8u - x)) & 255u;
-      x = (x + uint32_t(__builtin_ctz(turned))) & 7u;
-      ask();
-      pp = uniform(ahead);
-    }
-    px = x;
-    ask();
-    return true;
-  }
-};
+  from = x;
+  ahead = ask_brick(take, x);
+  return true;
+}
 
-// Occupancy: five waves per SIMD in FP64, six in FP32.
+// Occupancy: four waves per SIMD in FP64 (128 VGPRs, no spill; five spill 120
+// bytes a lane and take 2.71 ms instead of 2.34 for the 512^3 frame), six in
+// FP32.
 template <typename R, int MODE>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 5 : 6))) void k_frame(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 8 ? 4 : 6))) void k_frame(
     const TessJob* __restrict__ jobs, const uint2* __restrict__ order, uint32_t ngroups, uint32_t shift,
     uint32_t* __restrict__ take, const RasterJob<R>* __restrict__ rjobs, const uint32_t* __restrict__ jimg,
     FrameHdr* __restrict__ hdr, uint64_t* __restrict__ key, uint64_t* __restrict__ id, Frag64* __restrict__ frags,
@@ -1416,15 +1415,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof
   }
   __syncthreads();  // the only barrier
   const DrawTo D = {key, id, frags, fcap, hdr};
-  Taker T = {take, ngroups, shift, uniform(blockIdx.x & 7u), 0u};
-  T.ask();
+  uint32_t list = uniform(blockIdx.x & 7u), ahead = ask_brick(take, list);
   uint32_t ntri = 0;  // triangles of the cells this lane counted
   // ring state: oldest item, items queued, and the field pass they belong to
   // (the queue holds one pass at a time)
   uint32_t head = 0, npend = 0, cur = 0;
   for (bool more = true; more;) {
     uint32_t tx = 0, tp = 0;
-    more = T.next(tx, tp);
+    more = next_brick(take, ngroups, shift, list, ahead, tx, tp);
     uint32_t jb = cur, ncut = 0;  // the brick's field pass, and its cut cells
     BrickBox B = {};
     if (more) {
