@@ -883,6 +883,7 @@ ViewDev<R> dev_view(const HostView& h) {
   v.fw = R(double(h.W));
   v.fh = R(double(h.H));
   set_pitch(v);
+  set_recips(v);
   set_cv(v);
   v.W = int32_t(h.W);
   v.H = int32_t(h.H);

@@ -72,6 +72,9 @@ struct ViewDev {
   R nc, d, lxx, lyy;
   R fw, fh;   // width, height as reals
   R pitch;    // max(1 / fw, 1 / fh): the larger pixel spacing (set_pitch)
+  R fine;     // 0.4 min(1 / fw, 1 / fh), or 0 where a pixel number may not be exact in R (set_pitch)
+  R ux, uy;   // the rounding slack of a pixel number, 4 eps (fw + 2) (set_pitch)
+  double rlxx, rlyy, rfw, rfh;  // 1 / lxx, 1 / lyy, 1 / fw, 1 / fh, rounded once (set_recips)
   R cv;       // (d - nc)^2 |lx x ly| / (lxx lyy): projected area per volume (set_cv)
   int32_t W, H;
 };
@@ -80,6 +83,19 @@ struct ViewDev {
 template <typename R>
 C3D_HD void set_pitch(ViewDev<R>& v) {
   v.pitch = fmax(R(1) / v.fw, R(1) / v.fh);
+  const R eps = sizeof(R) == 8 ? R(2.220446049250313e-16) : R(1.1920929e-7);
+  v.ux = R(4) * eps * (v.fw + R(2));
+  v.uy = R(4) * eps * (v.fh + R(2));
+  v.fine = fmax(v.fw, v.fh) < R(8388608) ? R(0.4) * fmin(R(1) / v.fw, R(1) / v.fh) : R(0);
+}
+
+// fills the reciprocals of a view whose lxx, lyy, fw and fh are set
+template <typename R>
+C3D_HD void set_recips(ViewDev<R>& v) {
+  v.rlxx = 1.0 / double(v.lxx);
+  v.rlyy = 1.0 / double(v.lyy);
+  v.rfw = 1.0 / double(v.fw);
+  v.rfh = 1.0 / double(v.fh);
 }
 
 // fills the area constant of a view whose lx, ly, lxx, lyy, nc and d are set
@@ -94,11 +110,13 @@ C3D_HD void set_cv(ViewDev<R>& v) {
 // constant).  The compiler's IEEE division is v_div_scale of the
 // denominator, v_rcp and two Newton steps on it, then v_div_scale of the
 // numerator, a product, an FMA, v_div_fmas and v_div_fixup.  Here the
-// denominator half is recip_shared(b), computed once for all numerators,
-// and the rest is the same instructions.  The denominator's v_div_scale
-// depends on a too: it leaves b unchanged except at extreme exponent
-// ratios, which is checked per numerator, and any other case takes the
-// plain division.  Every result therefore equals a / b bit for bit.
+// denominator half is rb, computed once for all numerators (recip_shared, or
+// 1 / b rounded once), and the rest is the same instructions: with such an
+// rb the quotient before the last FMA is within a unit in the last place,
+// and the FMA rounds it correctly (Markstein).  The denominator's
+// v_div_scale depends on a too: it leaves b unchanged except at extreme
+// exponent ratios, which is checked per numerator, and any other case takes
+// the plain division.  Every result therefore equals a / b bit for bit.
 __device__ __forceinline__ double recip_shared(double b) {
   const double r0 = __builtin_amdgcn_rcp(b);
   const double e0 = __builtin_fma(-b, r0, 1.0);
@@ -117,13 +135,32 @@ __device__ __forceinline__ double div_shared(double a, double b, double rb) {
 }
 #endif
 
-// a / b, b a view constant (see div_shared)
-template <typename R>
-C3D_HD R div_view(R a, R b) {
+// a / b for a constant b of the view, rb = 1 / b rounded once to FP64, equal
+// to the division bit for bit.  FP32: the FP64 product a rb is within
+// 2^-52 of a / b, and the quotient of two 24-bit significands is never
+// nearer than 2^-49 to the middle of two floats, so rounding the product
+// gives the rounded quotient; below the smallest normal float the middles
+// lie elsewhere, and the plain division is taken.  With plain divisions here
+// and in the pixel centres the 512^3 frame took 2.93 ms in FP32 instead of
+// 2.81, and the close-up of 301 x 187 x 223 in FP64 1.60 ms instead of 1.48.
+C3D_HD float div_const(float a, float b, double rb) {
+  float q = float(double(a) * rb);
+  if (fabs(q) < 1.1754943508222875e-38f) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (sizeof(R) == 8) return div_shared(a, b, recip_shared(b));
+    // (keeps the compiler from dividing every time and selecting)
+    asm volatile("" : "+v"(a));
 #endif
+    q = a / b;
+  }
+  return q;
+}
+C3D_HD double div_const(double a, double b, double rb) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return div_shared(a, b, rb);
+#else
+  (void)rb;
   return a / b;
+#endif
 }
 
 // perspective projection (project.c:9-67); false when rejected
@@ -140,8 +177,8 @@ C3D_HD bool project(const ViewDev<R>& v, V3<R> p, V3<R>& q) {
                        v.cam[2] + t * ray.z - v.ctr[2]};
   const V3<R> lx = {v.lx[0], v.lx[1], v.lx[2]};
   const V3<R> ly = {v.ly[0], v.ly[1], v.ly[2]};
-  q.x = div_view(vdot(delta, lx), v.lxx);
-  q.y = div_view(vdot(delta, ly), v.lyy);
+  q.x = div_const(vdot(delta, lx), v.lxx, v.rlxx);
+  q.y = div_const(vdot(delta, ly), v.lyy, v.rlyy);
   q.z = nr;
   return true;
 }
@@ -166,6 +203,28 @@ C3D_HD int32_t clampi(int32_t lo, int32_t x, int32_t hi) { return x < lo ? lo : 
 template <typename R>
 C3D_HD R pixel_centre(int32_t i, R extent) {
   return R(1) * (R(i) + R(0.5)) / extent - R(0.5);
+}
+
+// (i + 1/2) / extent for 0 <= i <= 2^31 and a whole extent of at most 2^31,
+// rb = 1 / extent rounded once to FP64, equal to the division bit for bit.
+// FP64: the quotient after the correction is within 2^-104 of the exact one
+// before it is rounded, and a quotient of whole numbers of 32 bits is either
+// a double or farther than 2^-87 from the middle of two.  FP32: as
+// div_const; the quotients are normal numbers.
+C3D_HD double centre_quotient(double a, double extent, double rb) {
+  const double q = a * rb;
+  return __builtin_fma(__builtin_fma(-extent, q, a), rb, q);
+}
+C3D_HD float centre_quotient(float a, float, double rb) { return float(double(a) * rb); }
+
+// pixel_centre of a view's column i and row j
+template <typename R>
+C3D_HD R column_centre(const ViewDev<R>& v, int32_t i) {
+  return centre_quotient(R(i) + R(0.5), v.fw, v.rfw) - R(0.5);
+}
+template <typename R>
+C3D_HD R row_centre(const ViewDev<R>& v, int32_t j) {
+  return centre_quotient(R(j) + R(0.5), v.fh, v.rfh) - R(0.5);
 }
 
 // A projected triangle: vertices, 1 / (clamped) doubled area and the pixel
@@ -271,6 +330,38 @@ C3D_HD void tight_box(const ViewDev<R>& v, R area, Projected<R>& P) {
   P.i1 = b;
   P.j0 = c;
   P.j1 = d;
+}
+
+// raster_box and tight_box at once for the usual triangle.  Where M (see
+// tight_box) is below v.fine, 0.4 pixels of either axis, the narrowed box
+// lies inside the reference's, whose bounds are a pixel and more outside the
+// vertices' box and cut off at the image alike: the reference's box need not
+// be formed, and the bounds are cut off as reals.  emax is the larger side of
+// the vertices' box: the vertices that span a side are joined by an edge.
+template <typename R>
+C3D_HD void pixel_box(const ViewDev<R>& v, Projected<R>& P) {
+  const R eps = sizeof(R) == 8 ? R(2.220446049250313e-16) : R(1.1920929e-7);
+  const R g = R(2.25) * eps;
+  const V3<R>* q = P.q;
+  const R area = edge_fn(q[0], q[1], q[2].x, q[2].y);
+  const R ainv = R(1) / (area < R(0) ? fmin(area, R(-1.e-16)) : fmax(area, R(1.e-16)));
+  const R minx = fmin(q[0].x, fmin(q[1].x, q[2].x)), maxx = fmax(q[0].x, fmax(q[1].x, q[2].x));
+  const R miny = fmin(q[0].y, fmin(q[1].y, q[2].y)), maxy = fmax(q[0].y, fmax(q[1].y, q[2].y));
+  const R emax = fmax(maxx - minx, maxy - miny), A = fabs(area), e2 = emax * emax;
+  const R D = emax + R(4) * v.pitch;
+  const R qmax = fmax(fmax(fmax(fabs(minx), fabs(maxx)), fmax(fabs(miny), fabs(maxy))), R(1));
+  const R M = (R(5.8e-8) * emax + R(12) * g * D * e2 * fabs(ainv)) * R(1.00000095367431640625) + R(16) * eps * qmax;
+  if (!(A > R(1.e-14) && emax > R(0) && A > R(4.1) * g * e2 && M < v.fine)) {
+    tight_box(v, raster_box(v, P), P);
+    return;
+  }
+  P.ainv = ainv;
+  const R ulo = (minx - M + R(0.5)) * v.fw - R(0.5), uhi = (maxx + M + R(0.5)) * v.fw - R(0.5);
+  const R vlo = (miny - M + R(0.5)) * v.fh - R(0.5), vhi = (maxy + M + R(0.5)) * v.fh - R(0.5);
+  P.i0 = int32_t(fmin(fmax(ceil(ulo - (v.ux + R(4) * eps * fabs(ulo))), R(0)), v.fw));
+  P.i1 = int32_t(fmin(fmax(floor(uhi + (v.ux + R(4) * eps * fabs(uhi))), R(-1)), v.fw - R(1)));
+  P.j0 = int32_t(fmin(fmax(ceil(vlo - (v.uy + R(4) * eps * fabs(vlo))), R(0)), v.fh));
+  P.j1 = int32_t(fmin(fmax(floor(vhi + (v.uy + R(4) * eps * fabs(vhi))), R(-1)), v.fh - R(1)));
 }
 
 }  // namespace c3d

@@ -846,10 +846,10 @@ __device__ __forceinline__ uint32_t setup_triangle(const ViewDev<R>& v, const V3
 #pragma unroll
   for (int n = 0; n < 3; n++) vis = vis && project(v, wpos[n], P.q[n]);
   if (!vis) return 0;
-  const R area = raster_box(v, P);
-  if (sizeof(R) == 4 && area == R(0)) return 0;
+  if (sizeof(R) == 4 && edge_fn(P.q[0], P.q[1], P.q[2].x, P.q[2].y) == R(0)) return 0;
   // about 12 reference-box candidates of a pixel-sized triangle narrow to 3
-  tight_box(v, area, P);
+  // (by way of the reference's box: 512^3 FP32 frame 2.89 ms instead of 2.81)
+  pixel_box(v, P);
   if (P.i1 < P.i0 || P.j1 < P.j0) return 0;
   // a box lies inside one image: fewer than 2^31 pixels
   return uint32_t(P.i1 - P.i0 + 1) * uint32_t(P.j1 - P.j0 + 1);
@@ -869,7 +869,7 @@ __device__ __forceinline__ void pixel_update(const ViewDev<R>& v, uint64_t row0,
                                              int32_t j, uint32_t tid1, uint64_t* __restrict__ key,
                                              uint32_t* __restrict__ id, Frag* s_frag, uint32_t* s_n) {
   R w0, w1, w2;
-  if (!pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2)) return;
+  if (!pixel_weights(P, column_centre(v, i), row_centre(v, j), w0, w1, w2)) return;
   const R dep = pixel_depth(P, w0, w1, w2);
   const uint64_t px = row0 + uint64_t(j) * uint64_t(v.W) + uint64_t(i);
   if constexpr (MODE == kRasterFp32) {
@@ -1006,8 +1006,13 @@ __global__ __launch_bounds__(kThreads) void k_raster(MeshView<R> m, const Raster
 // field is behind its first surfaces: at 512^3, three thresholds and
 // 1920 x 1080, 42 M of 129 M triangles are drawn.
 //
-// What bounds it: vector-ALU issue and the latency of each brick's chain of
-// reads.  That FP64 frame's kernel took 4.50 ms as a tessellation of whole
+// What bounds it: vector-ALU issue (1000 instructions per 64 triangles in
+// FP32 before the pixel box was formed directly, divisions by view constants
+// became products and corners were selected by masks: 512^3 FP32 frame 3.15
+// -> 2.81 ms, 1024^3 19.1 -> 16.9 ms), and the latency of each brick's chain
+// of reads.  Letting every lane walk to its next covered pixel before any of
+// them forms a depth was no faster on small triangles and slower on large
+// ones (close-up 1.65 -> 2.51 ms).  That FP64 frame's kernel took 4.50 ms as a tessellation of whole
 // rows with a queue and barriers per workgroup, no z-test and no order; 3.61
 // ms in bricks taken front to back by workgroups; and 2.2 ms by waves, with
 // the cut cells listed before anything is done with them (FP32, where every
@@ -1034,11 +1039,27 @@ constexpr uint32_t kRing = 512;        // of a workgroup of the emit (at least 2
 // and the drains index ThrSet::thr and ::obj with it
 static_assert(kMaxThr == 4, "the ring's threshold field is 2 bits wide");
 
+// bit b of x as a mask, and a where the mask is set, else b
+__device__ __forceinline__ uint32_t bit_mask(uint32_t x, int b) { return uint32_t(int32_t(x << (31 - b)) >> 31); }
+__device__ __forceinline__ uint32_t pick(uint32_t m, uint32_t a, uint32_t b) { return (m & a) | (~m & b); }
+__device__ __forceinline__ float pick(uint32_t m, float a, float b) {
+  return __uint_as_float(pick(m, __float_as_uint(a), __float_as_uint(b)));
+}
+__device__ __forceinline__ uint64_t pick(uint32_t m, uint64_t a, uint64_t b) {
+  return uint64_t(pick(m, uint32_t(a >> 32), uint32_t(b >> 32))) << 32 | pick(m, uint32_t(a), uint32_t(b));
+}
+__device__ __forceinline__ double pick(uint32_t m, double a, double b) {
+  return __hiloint2double(int(pick(m, uint32_t(__double2hiint(a)), uint32_t(__double2hiint(b)))),
+                          int(pick(m, uint32_t(__double2loint(a)), uint32_t(__double2loint(b)))));
+}
+
 // positions of the triangle whose vertices join the corners in `ent` (slot
 // entry bits 0-17) of cell L, reading the two corner values of each
 // vertex's lattice edge from the field; on a grid lattice the cell's six
 // coordinates are read once.  Every load depends only on L and ent, so they
-// are in flight together.
+// are in flight together.  The corners' bits select by masks (v_bfi), which
+// is half the instructions of compares and selects: a frame at 512^3 in FP32
+// took 2.92 ms with those instead of 2.81.
 template <typename R>
 __device__ __forceinline__ void slot_positions_mem(const FieldDev& f, const CellLoc& L, double thr, uint32_t ent,
                                                    V3<R> P[3]) {
@@ -1053,15 +1074,20 @@ __device__ __forceinline__ void slot_positions_mem(const FieldDev& f, const Cell
     }
     return;
   }
-  const double x0 = gptr(f.gx)[L.i], x1 = gptr(f.gx)[L.i + 1], y0 = gptr(f.gy)[L.j], y1 = gptr(f.gy)[L.j + 1];
-  const double z0 = gptr(f.gz)[L.k], z1 = gptr(f.gz)[L.k + 1];
+  const R x0 = R(gptr(f.gx)[L.i]), x1 = R(gptr(f.gx)[L.i + 1]), y0 = R(gptr(f.gy)[L.j]),
+          y1 = R(gptr(f.gy)[L.j + 1]), z0 = R(gptr(f.gz)[L.k]), z1 = R(gptr(f.gz)[L.k + 1]);
+  const uint64_t below = uint64_t(p), above = uint64_t(p + uint64_t(f.nx) * f.ny);  // the cell's two planes
+  const auto load_at = [](uint64_t plane, uint32_t off) { return reinterpret_cast<const C3D_GLOBAL double*>(plane)[off]; };
 #pragma unroll
   for (int vv = 0; vv < 3; vv++) {
-    const uint32_t tail = (ent >> (6 * vv)) & 7u;
-    const uint32_t head = (ent >> (6 * vv + 3)) & 7u;
-    const V3<R> pt = {R(tail & 1u ? x1 : x0), R(tail & 2u ? y1 : y0), R(tail & 4u ? z1 : z0)};
-    const V3<R> ph = {R(head & 1u ? x1 : x0), R(head & 2u ? y1 : y0), R(head & 4u ? z1 : z0)};
-    P[vv] = interp<R>(thr, pt, p[corner_offset(f, tail)], ph, p[corner_offset(f, head)]);
+    uint32_t m[6];  // the corners' bits as masks: tail x, y, z, head x, y, z
+#pragma unroll
+    for (int b = 0; b < 6; b++) m[b] = bit_mask(ent, 6 * vv + b);
+    const V3<R> pt = {pick(m[0], x1, x0), pick(m[1], y1, y0), pick(m[2], z1, z0)};
+    const V3<R> ph = {pick(m[3], x1, x0), pick(m[4], y1, y0), pick(m[5], z1, z0)};
+    // a plane may hold 2^32 points and more, a row holds at most 2^30
+    const uint64_t at = pick(m[2], above, below), ah = pick(m[5], above, below);
+    P[vv] = interp<R>(thr, pt, load_at(at, (m[0] & 1u) + (m[1] & f.nx)), ph, load_at(ah, (m[3] & 1u) + (m[4] & f.nx)));
   }
 }
 
@@ -1147,7 +1173,7 @@ template <typename R, int MODE>
 __device__ __forceinline__ void frame_pixel(const ViewDev<R>& v, uint64_t row0, const Projected<R>& P, int32_t i,
                                             int32_t j, uint64_t tid, FrameLds& S, const DrawTo& D) {
   R w0, w1, w2;
-  if (!pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), w0, w1, w2)) return;
+  if (!pixel_weights(P, column_centre(v, i), row_centre(v, j), w0, w1, w2)) return;
   const uint64_t k = depth_key(pixel_depth(P, w0, w1, w2));
   const uint64_t px = row0 + uint64_t(j) * uint64_t(v.W) + uint64_t(i);
   // keys only grow, so a value read here, however stale, that is above k
@@ -2187,7 +2213,7 @@ __device__ __forceinline__ void weights_at(const ViewDev<R>& v, const V3<R> p[3]
 #pragma unroll
   for (int n = 0; n < 3; n++) project(v, p[n], P.q[n]);
   raster_box(v, P);
-  pixel_weights(P, pixel_centre<R>(i, v.fw), pixel_centre<R>(j, v.fh), X.w0, X.w1, X.w2);
+  pixel_weights(P, column_centre(v, i), row_centre(v, j), X.w0, X.w1, X.w2);
 }
 
 // A frame without a stored mesh: triangles are found from their ids (the
