@@ -229,6 +229,13 @@ struct HostBuf {
 constexpr size_t kMaxGeoms = 1024;
 constexpr size_t kGeomTableBytes = size_t(16) << 30;
 
+// Where a lattice lies: its middle point, and for each axis the two ends of
+// the grid line through it.
+struct LatticeMid {
+  bool known = false;
+  double centre[3] = {}, lo[3][3] = {}, hi[3][3] = {};
+};
+
 struct Geom {
   void* conv = nullptr;
   const double* g[3] = {nullptr, nullptr, nullptr};
@@ -237,6 +244,7 @@ struct Geom {
   std::vector<double> host;  // the grid values (nx + ny + nz), compared on a hash match
   bool identity = true;
   bool ordered = false;  // every grid finite and monotonic: a range of cells lies between its ends
+  LatticeMid mid;
   DevBuf grids;  // nx + ny + nz doubles
   DevBuf table;  // 3 * npts doubles when not the identity
   uint64_t stamp = 0;
@@ -677,6 +685,28 @@ bool ordered_grid(const double* g, size_t n) {
   return fin && (up || down);
 }
 
+// from the grids, or from a table of points (x, y and z of all of them)
+LatticeMid lattice_mid(const double* const g[3], const size_t n[3], const double* tab) {
+  LatticeMid m;
+  const size_t c[3] = {n[0] / 2, n[1] / 2, n[2] / 2}, npts = n[0] * n[1] * n[2];
+  const auto point = [&](size_t i, size_t j, size_t k, double out[3]) {
+    const size_t p = (k * n[1] + j) * n[0] + i;
+    out[0] = tab ? tab[p] : g[0][i];
+    out[1] = tab ? tab[npts + p] : g[1][j];
+    out[2] = tab ? tab[2 * npts + p] : g[2][k];
+  };
+  point(c[0], c[1], c[2], m.centre);
+  for (int d = 0; d < 3; d++) {
+    size_t a[3] = {c[0], c[1], c[2]};
+    a[d] = 0;
+    point(a[0], a[1], a[2], m.lo[d]);
+    a[d] = n[d] - 1;
+    point(a[0], a[1], a[2], m.hi[d]);
+  }
+  m.known = true;
+  return m;
+}
+
 int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
   const size_t nx = o.glsizes[0], ny = o.glsizes[1], nz = o.glsizes[2];
   std::vector<double> hg[3];
@@ -730,10 +760,10 @@ int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
   C3D_HIP(hipMemcpy(g->grids.as<double>() + nx + ny, gp[2], nz * sizeof(double), hipMemcpyHostToDevice));
   g->identity = true;
   g->ordered = ordered_grid(gp[0], nx) && ordered_grid(gp[1], ny) && ordered_grid(gp[2], nz);
+  std::vector<double> tab;
   if (o.converter != contour3d_amd_identity) {
     const ConvFn conv = o.converter;
     const size_t npts = nx * ny * nz;
-    std::vector<double> tab;
     size_t p = 0;
     for (size_t k = 0; k < nz; k++) {
       for (size_t j = 0; j < ny; j++) {
@@ -765,6 +795,7 @@ int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
       C3D_HIP(hipMemcpy(g->table.p, tab.data(), 3 * npts * sizeof(double), hipMemcpyHostToDevice));
     }
   }
+  g->mid = lattice_mid(gp, o.glsizes, g->identity ? nullptr : tab.data());
   unbuilt.g = nullptr;
   g->stamp = ++L.stamp;
   // Keep up to kMaxGeoms geometries and kGeomTableBytes of coordinate
@@ -1029,12 +1060,103 @@ int ensure_capacity(contour3d_amd_mesh& M) {
   return 0;
 }
 
-// Cells from which a frame's bricks get `planes` planes: fewer planes make
-// more bricks, and a small lattice needs them to fill the device.
-uint32_t brick_planes(uint64_t cells) {
-  uint32_t planes = kBrickPlanes;
-  while (planes > 1 && cells / (uint64_t(kBrickColumns) * planes) < 5120) planes /= 2;
-  return planes;
+// The pixels that a cell of the lattice (n cells per axis) covers in view v,
+// by the lattice's middle; 0 where that does not project.
+template <typename R>
+double cell_pixels(const ViewDev<R>& v, const LatticeMid& m, const uint32_t n[3]) {
+  if (!m.known) return 0;
+  V3<R> q0, q;
+  if (!project(v, V3<R>{R(m.centre[0]), R(m.centre[1]), R(m.centre[2])}, q0)) return 0;
+  double e[3][2];  // the image of a cell's edges, from an eighth of each axis
+  for (int d = 0; d < 3; d++) {
+    R p[3];
+    for (int c = 0; c < 3; c++) p[c] = R(m.centre[c] + (m.hi[d][c] - m.lo[d][c]) / 8);
+    if (!project(v, V3<R>{p[0], p[1], p[2]}, q)) return 0;
+    e[d][0] = double(q.x - q0.x) * v.W * 8 / n[d];
+    e[d][1] = double(q.y - q0.y) * v.H * 8 / n[d];
+  }
+  double sum = 0;
+  for (int d = 0; d < 3; d++) {
+    const int a = (d + 1) % 3, b = (d + 2) % 3;
+    sum += fabs(e[a][0] * e[b][1] - e[a][1] * e[b][0]);
+  }
+  return std::isfinite(sum) ? sum : 0;
+}
+
+// Chooses the shape of each field pass's bricks (an index of kBrickShapes)
+// for a device that holds `waves` waves of the frame kernel.
+//
+// A brick is worked on by one wave, so a frame ends no sooner than its
+// longest brick: that grows with the brick's cells times the work of one,
+// which is counted as one for each image and threshold (the triangles'
+// setup) and one more per kSetupPixels pixels that it covers there.  And
+// every brick, empty or not, has its turn at a counter, so the turns' time
+// grows with the frame's cells over the brick's.  The sum is least at
+// kVolume sqrt(cells / work).  Two limits besides: where that is just more
+// bricks than waves, with cells of at most kLightPixels pixels, the larger
+// bricks that are all worked on at once are better by the latency of a brick
+// (23 us); and there are at most kMostBricks, unless the largest are more.
+//
+// Where the lines lie: frame times in us with halving planes of 64-column
+// bricks until there are 5120 of them, and with this rule (turbulence unless
+// said otherwise, FP64 unless said otherwise).
+//   24^3, 640 x 480                    320 ->  175    (2 x 2 x 1)
+//   33 x 29 x 31, a close-up           638 ->  239    (2 x 2 x 1)
+//   96^3, a close-up, FP32             729 ->  576    (4 x 4 x 2)
+//   128^3 blobs, 800 x 600             238 ->  212    (8 x 8 x 8)
+//   180^3, a close-up                  916 ->  720    (8 x 8 x 2)
+//   301 x 187 x 223, a close-up       1468 -> 1379    (8 x 8 x 2)
+//   24 fields of 48^3 to 256^3, FP32  4959 -> 4151
+//   100^3, 1920 x 1080, a deep close-up 41756 -> 11998  (2 x 2 x 1)
+//   256^3, 1920 x 1080                 776 ->  776    (8 x 8 x 8)
+// kVolume of 0.2 costs 128^3 blobs 248 and the 24 fields 4400, 0.45 costs the
+// 33 x 29 x 31 close-up 294 and 180^3 770; kSetupPixels of 15 costs the 24
+// fields 4563 and 33 x 29 x 31 291; kMostPixels of 256 costs 100^3 19559.
+constexpr double kVolume = 0.3, kSetupPixels = 5, kLightPixels = 100, kMostPixels = 4096, kMostBricks = 131072;
+
+template <typename R>
+void choose_bricks(const std::vector<TessJob>& tj, const std::vector<const LatticeMid*>& mids,
+                   const std::vector<RasterJob<R>>& rj, bool by_view, uint32_t waves, std::vector<uint32_t>& shape) {
+  const size_t n = tj.size();
+  // (a batch of very many views: one image, of no size, stands for them)
+  by_view = by_view && n * rj.size() <= 65536;
+  double cells = 0, most = 0;
+  for (const TessJob& j : tj) cells += double(j.f.ncells);
+  const auto bricks = [&] {
+    double sum = 0;
+    for (size_t j = 0; j < n; j++) sum += double(tj[j].f.ncells) / brick_volume(shape[j]);
+    return sum;
+  };
+  const auto coarser = [&] {
+    bool any = false;
+    for (size_t j = 0; j < n; j++) {
+      any = any || shape[j];
+      shape[j] -= shape[j] ? 1 : 0;
+    }
+    return any;
+  };
+  shape.assign(n, 0);
+  for (size_t j = 0; j < n; j++) {
+    const FieldDev& f = tj[j].f;
+    const uint32_t nc[3] = {f.ncx, f.ncy, f.ncz};
+    double work = by_view ? 0 : tj[j].ts.n;
+    for (size_t q = 0; by_view && q < rj.size(); q++) {
+      uint32_t shown = 0;
+      for (uint32_t t = 0; t < tj[j].ts.n; t++)
+        shown += tj[j].ts.obj[t] >= rj[q].obj0 && tj[j].ts.obj[t] < rj[q].obj1 ? 1u : 0u;
+      if (!shown) continue;
+      const double pixels = std::min(cell_pixels(rj[q].v, *mids[j], nc), kMostPixels);
+      most = std::max(most, pixels);
+      work += shown * (1 + pixels / kSetupPixels);
+    }
+    // the shape nearest to the best volume by ratio: they go down by halves
+    const double best = kVolume * std::sqrt(cells / std::max(work, 1.0));
+    while (shape[j] + 1 < kNumBrickShapes && brick_volume(shape[j]) > best * 1.4142135623730951) shape[j]++;
+  }
+  const double b = bricks();
+  if (most <= kLightPixels && b > waves && b <= 2.0 * waves) (void)coarser();
+  while (bricks() > kMostBricks && coarser()) {
+  }
 }
 
 // Host half of a frame's tessellation (or, with `stored`, a mesh's): validates the objects, resolves
@@ -1043,7 +1165,7 @@ uint32_t brick_planes(uint64_t cells) {
 // of the pass and object tables.  The layout goes to F.tl.
 template <typename R>
 int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<const contour3d_contour_obj_t*>& objs,
-                 bool stored) {
+                 bool stored, bool by_view = true) {
   const size_t n = objs.size();
   if (F.noalloc && n > F.tjobs.bytes / sizeof(TessJob) - 1) {
     log_error("the allocation-free call takes at most %zu contour objects", F.tjobs.bytes / sizeof(TessJob) - 1);
@@ -1068,6 +1190,7 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
   // usually share one field and lattice)
   std::vector<char> on_dev(n, 0);
   std::vector<Geom*> geo(n, nullptr);
+  std::vector<LatticeMid> mids(n);
   for (size_t o = 0; o < n; o++) {
     const contour3d_contour_obj_t& ob = *objs[o];
     if (validate_obj(ob, o)) return 1;
@@ -1129,8 +1252,12 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
       f.gz = f.gy + f.ny;
       f.cx = f.cy = f.cz = nullptr;
       f.ordered = 1;
-      for (int d = 0; d < 3; d++)
-        if (is_device_ptr(ob.grids[d]) || !ordered_grid(ob.grids[d], ob.glsizes[d])) f.ordered = 0;
+      bool on_host = true;
+      for (int d = 0; d < 3; d++) {
+        if (is_device_ptr(ob.grids[d])) on_host = false;
+        if (!on_host || !ordered_grid(ob.grids[d], ob.glsizes[d])) f.ordered = 0;
+      }
+      if (on_host) mids[o] = lattice_mid(ob.grids, ob.glsizes, nullptr);
     } else if (on_dev[o]) {
       f.f = ob.array;
     } else {
@@ -1158,6 +1285,7 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
       f.gx = g->grids.as<double>();
       f.gy = f.gx + f.nx;
       f.gz = f.gy + f.ny;
+      mids[o] = g->mid;
       if (g->identity) {
         f.ordered = g->ordered;
         f.cx = f.cy = f.cz = nullptr;
@@ -1257,13 +1385,24 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
     // share out, of 2^3 below
     uint64_t cells = 0;
     for (const TessJob& j : tj) cells += uint64_t(j.f.ncx) * j.f.ncy * j.f.ncz;
-    uint32_t rows = L.tess_rows, planes = L.tess_zc ? L.tess_zc : brick_planes(cells);
+    uint32_t rows = L.tess_rows;
+    std::vector<uint32_t> shape;
+    std::vector<const LatticeMid*> pass_mid;
+    for (const TessJob& j : tj) pass_mid.push_back(&mids[j.ts.obj[0]]);
+    choose_bricks<R>(tj, pass_mid, F.rjobs_host<R>(), by_view,
+                     uint32_t(persistent_blocks()) / 8u * (sizeof(R) == 8 ? 4u : 6u) * 4u, shape);
+    // a knob holds for every pass
+    if (L.tess_rows || L.tess_zc) shape.assign(tj.size(), 0);
+    bool chosen = true;
     F.tl.shift = cells / (uint64_t(kBrickColumns) * kBrickPlanes) >= 65536 ? 2 : 1;
     uint64_t ng = 0;
     for (int attempt = 0; attempt < 2; attempt++) {
       ng = 0;
-      for (TessJob& j : tj) {
-        j.bg = make_brick_geo(j.f.ncx, j.f.ncy, j.f.ncz, rows, planes, F.tl.shift);
+      for (size_t q = 0; q < tj.size(); q++) {
+        TessJob& j = tj[q];
+        const BrickShape b = kBrickShapes[chosen ? shape[q] : 0];
+        j.bg = make_brick_geo(j.f.ncx, j.f.ncy, j.f.ncz, rows, chosen && L.tess_zc ? L.tess_zc : b.planes, F.tl.shift,
+                              b.side);
         j.group0 = uint32_t(ng);
         ng += brick_groups(j.bg);
       }
@@ -1271,7 +1410,7 @@ int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<cons
       // takes, but not in any shape that the knobs ask for
       if (!F.noalloc || ng <= F.order.bytes / sizeof(uint2)) break;
       rows = 0;
-      planes = kBrickPlanes;
+      chosen = false;
       F.tl.shift = 2;
     }
     if (ng >= (uint64_t(1) << 31) >> (3 * F.tl.shift) || (F.noalloc && ng > F.order.bytes / sizeof(uint2))) {
@@ -1801,7 +1940,9 @@ int run_frame_t(Lib& L, Frame& F, std::vector<Image>& imgs, bool graph) {
     log_error("%zu contour objects exceed a frame's %llu", objs.size(), (unsigned long long)(kLineObj - 2));
     return 1;
   }
-  if (tess_prepare<R>(L, F, F.mesh, objs, false)) return 1;
+  // (a replayed graph holds for one set of bricks: there they do not depend
+  // on the view)
+  if (tess_prepare<R>(L, F, F.mesh, objs, false, !graph)) return 1;
   if (upload_pass_images(F, imgs)) return 1;
   if (raster_prepare<R>(F, npx, false)) return 1;
   if (graph ? graph_frame<R>(L, F, rjd, njobs, npx) : frame_launch<R>(L, F, rjd, njobs, npx, F.h_nline)) return 1;

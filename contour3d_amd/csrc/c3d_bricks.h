@@ -21,6 +21,14 @@ constexpr uint32_t kBrickColumns = 64;  // cell columns of a brick at most (a wa
 constexpr uint32_t kBrickSide = 8;      // cells per axis of a brick's plane, where the lattice has them
 constexpr uint32_t kBrickPlanes = 8;    // planes of a brick at most
 
+// The shapes a frame chooses from: columns per side of a brick, and planes.
+struct BrickShape {
+  uint32_t side, planes;
+};
+constexpr BrickShape kBrickShapes[] = {{8, 8}, {8, 4}, {8, 2}, {4, 4}, {4, 2}, {4, 1}, {2, 2}, {2, 1}};
+constexpr uint32_t kNumBrickShapes = sizeof(kBrickShapes) / sizeof(kBrickShapes[0]);
+constexpr uint32_t brick_volume(uint32_t s) { return kBrickShapes[s].side * kBrickShapes[s].side * kBrickShapes[s].planes; }
+
 struct BrickGeo {
   uint32_t bw, bh, bz;     // cells per brick
   uint32_t nbx, nby, nbz;  // bricks per axis
@@ -29,18 +37,19 @@ struct BrickGeo {
   FastDiv div_bw, div_nsx, div_nsy;
 };
 
-// Bricks of an ncx x ncy x ncz cell lattice: balanced, at most max_rows rows
-// (0: as many as fit) and `planes` planes each.
+// Bricks of an ncx x ncy x ncz cell lattice: balanced, at most side^2 columns,
+// max_rows rows (0: as many as fit) and `planes` planes each.
 inline BrickGeo make_brick_geo(uint32_t ncx, uint32_t ncy, uint32_t ncz, uint32_t max_rows, uint32_t planes,
-                               uint32_t shift) {
+                               uint32_t shift, uint32_t side = kBrickSide) {
   auto parts = [](uint32_t n, uint32_t of) { return (n + of - 1) / of; };
   BrickGeo g{};
-  uint32_t rows = ncy < kBrickSide ? ncy : kBrickSide;
+  const uint32_t columns = side * side;
+  uint32_t rows = ncy < side ? ncy : side;
   if (max_rows && rows > max_rows) rows = max_rows;
-  g.nbx = parts(ncx, kBrickColumns / rows);
+  g.nbx = parts(ncx, columns / rows);
   g.bw = parts(ncx, g.nbx);
   g.nbx = parts(ncx, g.bw);
-  rows = kBrickColumns / g.bw;
+  rows = columns / g.bw;
   if (max_rows && rows > max_rows) rows = max_rows;
   g.nby = parts(ncy, rows);
   g.bh = parts(ncy, g.nby);

@@ -1,11 +1,12 @@
 // Brute-force check of the brick arithmetic of c3d_bricks.h (the header the
 // device kernels use).  For each lattice given as "ncx ncy ncz max_rows
-// planes shift" on the command line, walks every position of every XCD list
-// and every lane of every brick as the kernel does, for all eight flips, and
-// checks that every cell is visited exactly once, that a brick holds at most
-// 64 columns and kBrickPlanes planes inside the lattice, and that every
-// position lies inside the ordered list.  Prints one line per lattice; exits
-// 1 on the first failure.
+// planes shift" on the command line, and bricks of 8, 4 and 2 columns a
+// side, walks every position of every XCD list and every lane of every brick
+// as the kernel does, for all eight flips, and checks that every cell is
+// visited exactly once, that a brick holds at most side^2 columns and
+// kBrickPlanes planes inside the lattice, and that every position lies inside
+// the ordered list.  Prints one line per lattice and side; exits 1 on the
+// first failure.
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -19,10 +20,11 @@ static int fail(const char* what, unsigned long long a, unsigned long long b) {
   return 1;
 }
 
-static int check(uint32_t ncx, uint32_t ncy, uint32_t ncz, uint32_t rows, uint32_t planes, uint32_t shift) {
-  const BrickGeo g = make_brick_geo(ncx, ncy, ncz, rows, planes, shift);
+static int check(uint32_t ncx, uint32_t ncy, uint32_t ncz, uint32_t rows, uint32_t planes, uint32_t shift,
+                 uint32_t side) {
+  const BrickGeo g = make_brick_geo(ncx, ncy, ncz, rows, planes, shift, side);
   const uint32_t ng = brick_groups(g), per = 1u << (3 * shift);
-  if (g.bw * g.bh > kBrickColumns || g.bz > kBrickPlanes || !g.bw || !g.bh || !g.bz) return fail("size", g.bw, g.bh);
+  if (g.bw * g.bh > side * side || g.bz > kBrickPlanes || !g.bw || !g.bh || !g.bz) return fail("size", g.bw, g.bh);
   if (rows && g.bh > rows) return fail("rows", g.bh, rows);
   for (uint32_t flip = 0; flip < 8; flip++) {
     std::vector<uint8_t> seen(uint64_t(ncx) * ncy * ncz, 0), taken(ng, 0);
@@ -58,7 +60,8 @@ int main(int argc, char** argv) {
   for (int a = 1; a + 5 < argc; a += 6) {
     uint32_t v[6];
     for (int q = 0; q < 6; q++) v[q] = uint32_t(std::atoi(argv[a + q]));
-    if (check(v[0], v[1], v[2], v[3], v[4], v[5])) return 1;
+    for (uint32_t side = kBrickSide; side >= 2; side /= 2)
+      if (check(v[0], v[1], v[2], v[3], v[4], v[5], side)) return 1;
   }
   return 0;
 }
