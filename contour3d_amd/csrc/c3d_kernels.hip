@@ -648,87 +648,6 @@ __global__ __launch_bounds__(kThreads) void k_cell_starts(const uint8_t* __restr
   }
 }
 
-// Vertex normals of every triangle of one object, a thread per (triangle,
-// vertex): the sum of vertex_normal -- cells sharing the vertex's lattice
-// edge in the neighbour table's increasing order, in each the triangles
-// with a vertex on the edge in slot order (c_emask of the cell's stored
-// corner code), from +0 -- gathered directly: a neighbour cell's triangles
-// start at bstart[its tile] + cstart[cell].  A thread's (at most four)
-// neighbour cells are fetched together.  Rows of triangles outside the
-// rendered interior are NaN.
-//
-// (Measured against this: one 32-bit cell word of code and start, the masks
-// in LDS and a persistent grid were 5% slower; a workgroup per tile, tiles
-// z-fastest along each column and one contiguous run per XCD (to keep the
-// planes above and below in L2), 1.55-1.66x slower: the serial order streams
-// the records and the normals in address order; a workgroup per tile
-// gathering a window of cells into LDS 3-4x slower.)
-template <typename R>
-__global__ __launch_bounds__(kThreads) void k_smooth(MeshView<R> m, const ObjMeta* __restrict__ meta,
-                                                     const uint16_t* __restrict__ cstart, R* __restrict__ out) {
-  const ObjMeta om = *meta;
-  const uint64_t n3 = 3 * om.count;
-  const uint8_t* cd = m.code + om.code_off;
-  const uint16_t* cs = cstart + om.code_off;
-  const int64_t sy = om.ncx, sz = int64_t(om.ncx) * om.ncy;
-  const R nan = R(__longlong_as_double(0x7ff8000000000000ll));
-  for (uint64_t it = uint64_t(blockIdx.x) * kThreads + threadIdx.x; it < n3; it += uint64_t(gridDim.x) * kThreads) {
-    const uint64_t t = it / 3u;
-    const uint32_t vv = uint32_t(it - 3u * t);
-    const uint64_t u = om.base + t;
-    const uint32_t c = m.aux[u].cell, ed = edges_of(m, u);
-    R* o = out + 9u * t + 3u * vv;
-    if (!((ed >> 15) & 1u)) {
-      o[0] = nan;
-      o[1] = nan;
-      o[2] = nan;
-      continue;
-    }
-    const uint32_t e = (ed >> (5u * vv)) & 31u;
-    const int nn = c_nbr.n[e];
-    uint32_t mask[4];
-    uint64_t s2[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      mask[q] = 0;
-      s2[q] = 0;
-      if (q < nn) {
-        // an interior cell's neighbours lie inside the lattice
-        const uint32_t c2 = uint32_t(int64_t(c) + c_nbr.v[e][q][0] * sz + c_nbr.v[e][q][1] * sy + c_nbr.v[e][q][2]);
-        mask[q] = c_emask[uint32_t(cd[c2]) * 19u + uint32_t(c_nbr.v[e][q][3])];
-        s2[q] = om.bstart[tile_of_cell(om, c2)] + cs[c2];
-      }
-    }
-    // each neighbour's first four hits are loaded together, then added in
-    // slot order (more hits, rare, follow one at a time)
-    V3<R> sum = {R(0), R(0), R(0)};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      uint32_t h = mask[q];
-      V3<R> wv[4];
-      bool hv[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const uint64_t u2 = s2[q] + uint32_t(__builtin_ctz(h | 0x80000000u));
-        hv[r] = h != 0 && u2 < m.cap;
-        wv[r] = hv[r] ? V3<R>{m.aux[u2].w[0], m.aux[u2].w[1], m.aux[u2].w[2]} : V3<R>{R(0), R(0), R(0)};
-        h &= h - 1u;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (hv[r]) sum = vadd(sum, wv[r]);
-      for (; h; h &= h - 1u) {
-        const uint64_t u2 = s2[q] + uint32_t(__builtin_ctz(h));
-        if (u2 < m.cap) sum = vadd(sum, V3<R>{m.aux[u2].w[0], m.aux[u2].w[1], m.aux[u2].w[2]});
-      }
-    }
-    const V3<R> nv = vunit(sum);
-    o[0] = nv.x;
-    o[1] = nv.y;
-    o[2] = nv.z;
-  }
-}
-
 // Compares object meshes built in two arithmetic forms, triangle by
 // triangle (the topology is the same by construction, which this checks):
 // out[0] topology mismatches (cell or edge ids), out[1] max |vertex
@@ -2188,6 +2107,125 @@ __device__ __forceinline__ uint32_t edge_id_at(uint32_t lo, uint32_t dir) {
   return dir == 1u || dir == 2u || dir == 4u ? by_axis : by_diag;
 }
 
+// Vertex normals of every triangle of one object: rows of nine reals, NaN
+// for triangles outside the rendered interior.  A workgroup takes 256
+// consecutive triangles, enters their vertices in a table of lattice edges in
+// LDS, forms each distinct vertex's normal once, a thread each, and writes
+// the rows as contiguous words.
+//
+// A normal is the sum of vertex_normal -- cells sharing the vertex's lattice
+// edge in the neighbour table's increasing order, in each the triangles with
+// a vertex on the edge in slot order (c_emask of the cell's stored corner
+// code), from +0 -- gathered directly: a neighbour cell's triangles start at
+// bstart[its tile] + cstart[cell].  A thread's (at most four) neighbour cells
+// are fetched together.  The sum depends on the edge alone, so it serves
+// every triangle with a vertex there.
+//
+// What bounds it: the gather of each vertex's code, start and weight records
+// through L1 and L2, 4 to 16 records a vertex.
+// With a thread per (triangle, vertex), each vertex of a cell's triangles was
+// gathered two or three times: 256^3 and two thresholds, FP64, 2 x 517 us
+// then, 2 x 308 now, and 1.38 ms for the mesh built and smoothed, 1.34 with
+// the rows stored non-temporally.
+//
+// (Measured against a thread per (triangle, vertex), the form before: one
+// 32-bit cell word of code and start, the masks in LDS and a persistent grid
+// were 5% slower; a workgroup per tile, tiles z-fastest along each column and
+// one contiguous run per XCD (to keep the planes above and below in L2),
+// 1.55-1.66x slower: the serial order streams the records and the normals in
+// address order; a workgroup per tile gathering a window of cells into LDS
+// 3-4x slower.)
+template <typename R>
+__device__ __forceinline__ V3<R> gathered_normal(const MeshView<R>& m, const ObjMeta& om, const uint8_t* cd,
+                                                 const uint16_t* cs, uint32_t c, uint32_t e) {
+  const int64_t sy = om.ncx, sz = int64_t(om.ncx) * om.ncy;
+  const int nn = c_nbr.n[e];
+  uint32_t mask[4];
+  uint64_t s2[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    mask[q] = 0;
+    s2[q] = 0;
+    if (q < nn) {
+      // an interior cell's neighbours lie inside the lattice
+      const uint32_t c2 = uint32_t(int64_t(c) + c_nbr.v[e][q][0] * sz + c_nbr.v[e][q][1] * sy + c_nbr.v[e][q][2]);
+      mask[q] = c_emask[uint32_t(cd[c2]) * 19u + uint32_t(c_nbr.v[e][q][3])];
+      s2[q] = om.bstart[tile_of_cell(om, c2)] + cs[c2];
+    }
+  }
+  // each neighbour's first four hits are loaded together, then added in
+  // slot order (more hits, rare, follow one at a time)
+  V3<R> sum = {R(0), R(0), R(0)};
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    uint32_t h = mask[q];
+    V3<R> wv[4];
+    bool hv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const uint64_t u2 = s2[q] + uint32_t(__builtin_ctz(h | 0x80000000u));
+      hv[r] = h != 0 && u2 < m.cap;
+      wv[r] = hv[r] ? V3<R>{m.aux[u2].w[0], m.aux[u2].w[1], m.aux[u2].w[2]} : V3<R>{R(0), R(0), R(0)};
+      h &= h - 1u;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (hv[r]) sum = vadd(sum, wv[r]);
+    for (; h; h &= h - 1u) {
+      const uint64_t u2 = s2[q] + uint32_t(__builtin_ctz(h));
+      if (u2 < m.cap) sum = vadd(sum, V3<R>{m.aux[u2].w[0], m.aux[u2].w[1], m.aux[u2].w[2]});
+    }
+  }
+  return vunit(sum);
+}
+
+template <typename R>
+__global__ __launch_bounds__(kThreads) void k_smooth(MeshView<R> m, const ObjMeta* __restrict__ meta,
+                                                     const uint16_t* __restrict__ cstart, R* __restrict__ out) {
+  __shared__ VtxTable<R> T;
+  __shared__ uint16_t s_vtx[3 * kThreads];  // the slots of the triangles' vertices
+  constexpr uint16_t kOutside = 0xffff;
+  const ObjMeta om = *meta;
+  const uint8_t* cd = m.code + om.code_off;
+  const uint16_t* cs = cstart + om.code_off;
+  const R nan = R(__longlong_as_double(0x7ff8000000000000ll));
+  for (uint64_t t0 = uint64_t(blockIdx.x) * kThreads; t0 < om.count; t0 += uint64_t(gridDim.x) * kThreads) {
+    for (uint32_t s = threadIdx.x; s < kVtxSlots; s += kThreads) T.key[s] = kNoVtx;
+    if (threadIdx.x == 0) T.count = 0;
+    __syncthreads();
+    const uint32_t nt = om.count - t0 < kThreads ? uint32_t(om.count - t0) : kThreads;
+    if (threadIdx.x < nt) {
+      const uint64_t u = om.base + t0 + threadIdx.x;
+      const uint32_t c = m.aux[u].cell, ed = edges_of(m, u);
+#pragma unroll
+      for (int n = 0; n < 3; n++) {
+        uint32_t s = kOutside;
+        if ((ed >> 15) & 1u) {
+          uint32_t lo, dir;
+          edge_lo_dir((ed >> (5 * n)) & 31u, lo, dir);
+          s = vtx_enter(T, vtx_key(0u, corner_cell(c, lo, om.ncx, om.ncy), dir));
+        }
+        s_vtx[3u * threadIdx.x + n] = uint16_t(s);
+      }
+    }
+    __syncthreads();
+    for (uint32_t u = threadIdx.x; u < T.count; u += kThreads) {
+      const unsigned long long key = T.key[T.slot[u]];
+      const V3<R> n = gathered_normal<R>(m, om, cd, cs, uint32_t(key >> 4), edge_id_at(0u, uint32_t(key) & 7u));
+      T.n[u][0] = n.x;
+      T.n[u][1] = n.y;
+      T.n[u][2] = n.z;
+    }
+    __syncthreads();
+    for (uint32_t w = threadIdx.x; w < 9u * nt; w += kThreads) {
+      const uint32_t v = w / 3u, s = s_vtx[v];
+      // (the rows stream past the caches, which hold the records)
+      __builtin_nontemporal_store(s == kOutside ? nan : T.n[T.idx[s]][w - 3u * v], out + 9u * t0 + w);
+    }
+    __syncthreads();  // the next triangles reuse the table
+  }
+}
+
 // Scratch of one wave forming vertex normals: the triangles found around
 // its 16 vertices (owner lane | slot << 6; an axis edge has at most 16, and
 // the diagonals fewer) and the smoothing weights of 64 of them.
@@ -2567,8 +2605,8 @@ template <typename R>
 hipError_t launch_vertex_normals(const MeshView<R>& m, const ObjMeta* meta_dev, const uint16_t* cstart,
                                  uint64_t count, R* out, hipStream_t st) {
   if (count == 0) return hipSuccess;
-  // one item per thread (the kernel strides past 2^24 workgroups)
-  const uint64_t blocks = (3 * count + kThreads - 1) / kThreads;
+  // one triangle per thread (the kernel strides past 2^24 workgroups)
+  const uint64_t blocks = (count + kThreads - 1) / kThreads;
   const uint32_t grid = uint32_t(blocks < (uint64_t(1) << 24) ? blocks : (uint64_t(1) << 24));
   hipLaunchKernelGGL(k_smooth<R>, dim3(grid), dim3(kThreads), 0, st, m, meta_dev, cstart, out);
   return hipGetLastError();
