@@ -2435,6 +2435,58 @@ int smooth_object(Frame& F, const contour3d_amd_mesh& M, size_t obj, void* out) 
   return prof_collect(F);
 }
 
+// Object obj's triangles in the caller's arrays (null: not wanted).  What is
+// already laid out as the caller wants it (an FP64 mesh's positions and
+// normals) is copied as it is; the rest is unpacked on the device,
+// kUnpackTriangles at a time, and copied from there.
+template <typename R>
+int mesh_copy_t(Frame& F, const contour3d_amd_mesh& M, size_t obj, double* pos, double* wfn, double* vn,
+                uint32_t* cell, uint32_t* edges) {
+  constexpr bool same = sizeof(R) == sizeof(double);
+  const uint64_t n = M.count[obj];
+  const MeshPos<R>* dp = M.pos.as<MeshPos<R>>() + M.base[obj];
+  const MeshAux<R>* da = M.aux.as<MeshAux<R>>() + M.base[obj];
+  // the mesh keeps no per-triangle vertex normals; they are gathered now
+  // with the same sums the resolve pass uses for nearest triangles.  They
+  // come first in the scratch, then a part's arrays.
+  const size_t chunk = size_t(std::min<uint64_t>(n, kUnpackTriangles));
+  const size_t vn_bytes = vn ? (size_t(n) * 9 * sizeof(R) + 255) / 256 * 256 : 0;
+  const bool parts = wfn || cell || edges || (!same && (pos || vn));
+  const size_t part = parts ? chunk * ((same ? 0 : 18) + 3) * sizeof(double) + 2 * chunk * sizeof(uint32_t) : 0;
+  if (F.vntmp.ensure(vn_bytes + part) != hipSuccess) {
+    log_error("mesh_copy: allocation failed");
+    return 1;
+  }
+  if (vn && smooth_object(F, M, obj, F.vntmp.p)) return 1;
+  const R* dn = F.vntmp.as<R>();
+  hipError_t e = hipSuccess;
+  const auto to_host = [&](void* dst, const void* src, size_t bytes) {
+    if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, F.st);
+  };
+  if (same && pos) to_host(pos, dp, size_t(n) * sizeof(MeshPos<R>));
+  if (same && vn) to_host(vn, dn, size_t(n) * 9 * sizeof(R));
+  double* const w = reinterpret_cast<double*>(F.vntmp.as<unsigned char>() + vn_bytes);
+  double *p64 = w + 3 * chunk, *n64 = p64 + (same ? 0 : 9 * chunk);
+  uint32_t *cells = reinterpret_cast<uint32_t*>(n64 + (same ? 0 : 9 * chunk)), *ed = cells + chunk;
+  const bool conv_pos = !same && pos, conv_vn = !same && vn;
+  for (uint64_t t = 0; parts && t < n && e == hipSuccess; t += chunk) {
+    const size_t k = size_t(std::min<uint64_t>(chunk, n - t));
+    e = launch_unpack<R>(dp + t, da + t, dn + 9 * t, uint32_t(k), conv_pos ? p64 : nullptr, wfn ? w : nullptr,
+                         conv_vn ? n64 : nullptr, cell ? cells : nullptr, edges ? ed : nullptr, F.st);
+    if (conv_pos) to_host(pos + 9 * t, p64, k * 9 * sizeof(double));
+    if (wfn) to_host(wfn + 3 * t, w, k * 3 * sizeof(double));
+    if (conv_vn) to_host(vn + 9 * t, n64, k * 9 * sizeof(double));
+    if (cell) to_host(cell + t, cells, k * sizeof(uint32_t));
+    if (edges) to_host(edges + t, ed, k * sizeof(uint32_t));
+  }
+  const hipError_t es = hipStreamSynchronize(F.st);
+  if (e != hipSuccess || es != hipSuccess) {
+    log_error("mesh_copy: device copy failed: %s", hipGetErrorString(e != hipSuccess ? e : es));
+    return 1;
+  }
+  return 0;
+}
+
 // The reference runs one pencil per MPI rank and reads each rank's local
 // extent from SimpleDecomp (extend.c:158-181); this library renders every
 // contour object's array as the whole field.  Under an MPI launch of more
@@ -2712,62 +2764,11 @@ int contour3d_amd_mesh_copy(const contour3d_amd_mesh_t* mesh, size_t obj, double
   }
   auto& L = lib();
   std::lock_guard<std::mutex> g(L.mu);
-  const uint64_t n = mesh->count[obj], b = mesh->base[obj];
-  if (n == 0) return 0;
-  const bool fp64 = mesh->precision == CONTOUR3D_AMD_FP64;
-  const size_t rs = fp64 ? 8 : 4;
-  // record sizes and the byte offset of the edge word in its record (the
-  // gather record in FP64, the position record in FP32)
-  const size_t PS = fp64 ? sizeof(c3d::MeshPos<double>) : sizeof(c3d::MeshPos<float>);
-  const size_t AS = fp64 ? sizeof(c3d::MeshAux<double>) : sizeof(c3d::MeshAux<float>);
-  auto real_at = [&](const unsigned char* q) {
-    if (rs == 8) {
-      double x;
-      std::memcpy(&x, q, 8);
-      return x;
-    }
-    float y;
-    std::memcpy(&y, q, 4);
-    return double(y);
-  };
-  // the object's records, unpacked field by field
-  std::vector<unsigned char> prec, arec;
-  if (pos || edges) prec.resize(n * PS);
-  if (wfn || cell || edges) arec.resize(n * AS);
-  if ((!prec.empty() && hipMemcpy(prec.data(), static_cast<const unsigned char*>(mesh->pos.p) + b * PS, n * PS,
-                                  hipMemcpyDeviceToHost) != hipSuccess) ||
-      (!arec.empty() && hipMemcpy(arec.data(), static_cast<const unsigned char*>(mesh->aux.p) + b * AS, n * AS,
-                                  hipMemcpyDeviceToHost) != hipSuccess)) {
-    c3d::log_error("mesh_copy: device copy failed");
-    return 1;
-  }
-  for (uint64_t t = 0; t < n; t++) {
-    const unsigned char* rp = prec.empty() ? nullptr : prec.data() + t * PS;
-    const unsigned char* ra = arec.empty() ? nullptr : arec.data() + t * AS;
-    if (pos)
-      for (int c = 0; c < 9; c++) pos[9 * t + c] = real_at(rp + c * rs);
-    if (wfn)
-      for (int c = 0; c < 3; c++) wfn[3 * t + c] = real_at(ra + c * rs);
-    if (cell) std::memcpy(cell + t, ra + 3 * rs, 4);
-    if (edges) std::memcpy(edges + t, fp64 ? ra + 3 * rs + 4 : rp + 9 * rs, 4);
-  }
-  if (vn) {
-    // the mesh keeps no per-triangle vertex normals; they are gathered now
-    // with the same sums the resolve pass uses for nearest triangles
-    if (c3d::ensure_init(L, 0)) return 1;
-    if (L.main.vntmp.ensure(n * 9 * rs) != hipSuccess) {
-      c3d::log_error("mesh_copy: allocation failed");
-      return 1;
-    }
-    if (c3d::smooth_object(L.main, *mesh, obj, L.main.vntmp.p)) return 1;
-    std::vector<unsigned char> raw(n * 9 * rs);
-    if (hipMemcpy(raw.data(), L.main.vntmp.p, n * 9 * rs, hipMemcpyDeviceToHost) != hipSuccess) {
-      c3d::log_error("mesh_copy: device copy failed");
-      return 1;
-    }
-    for (uint64_t q = 0; q < n * 9; q++) vn[q] = real_at(raw.data() + q * rs);
-  }
-  return 0;
+  if (mesh->count[obj] == 0 || !(pos || wfn || vn || cell || edges)) return 0;
+  if (c3d::ensure_init(L, 0)) return 1;
+  return mesh->precision == CONTOUR3D_AMD_FP64
+             ? c3d::mesh_copy_t<double>(L.main, *mesh, obj, pos, wfn, vn, cell, edges)
+             : c3d::mesh_copy_t<float>(L.main, *mesh, obj, pos, wfn, vn, cell, edges);
 }
 
 int contour3d_amd_mesh_normals(const contour3d_amd_mesh_t* mesh, size_t obj, void* vn) {

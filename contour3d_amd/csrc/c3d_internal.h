@@ -221,6 +221,12 @@ hipError_t launch_cell_starts(const uint8_t* code, const ObjMeta* meta_dev, uint
 template <typename R>
 hipError_t launch_vertex_normals(const MeshView<R>& m, const ObjMeta* meta_dev, const uint16_t* cstart,
                                  uint64_t count, R* out, hipStream_t st);
+// n (at most kUnpackTriangles) triangles' records, and rows of normals, as
+// the arrays of doubles that a host caller takes; null: not wanted
+constexpr uint32_t kUnpackTriangles = 1u << 18;
+template <typename R>
+hipError_t launch_unpack(const MeshPos<R>* pos, const MeshAux<R>* aux, const R* vn, uint32_t n, double* opos,
+                         double* owfn, double* ovn, uint32_t* ocell, uint32_t* oedges, hipStream_t st);
 // FP64 mesh a against mesh b (FP64, or FP32 when b_fp32; b points to its
 // MeshView) for one object: out[0..4] as k_mesh_compare documents
 hipError_t launch_mesh_compare(const MeshView<double>& a, const ObjMeta* ma, const void* b, int b_fp32,
