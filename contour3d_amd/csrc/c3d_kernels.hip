@@ -526,25 +526,6 @@ __device__ __forceinline__ V3<R> interp(double thr, V3<R> p0, double v0, V3<R> p
   return vadd(p0, vscale(fct, vsub(p1, p0)));
 }
 
-// positions of the triangle in slot entry `ent` of cell L from its corner
-// values v (the arithmetic of the emit pass, from registers)
-template <typename R>
-__device__ __forceinline__ void slot_positions(const FieldDev& f, const CellLoc& L, double thr, uint64_t ent,
-                                               const double v[8], V3<R> P[3]) {
-#pragma unroll
-  for (int vv = 0; vv < 3; vv++) {
-    const uint32_t tail = uint32_t(ent >> (6 * vv)) & 7u;
-    const uint32_t head = uint32_t(ent >> (6 * vv + 3)) & 7u;
-    double vt = v[0], vh = v[0];
-#pragma unroll
-    for (int q = 1; q < 8; q++) {
-      vt = tail == uint32_t(q) ? v[q] : vt;
-      vh = head == uint32_t(q) ? v[q] : vh;
-    }
-    P[vv] = interp<R>(thr, corner_pos<R>(f, L, tail), vt, corner_pos<R>(f, L, head), vh);
-  }
-}
-
 // The smoothing weight of a triangle: area * unit face normal
 // (triangulate.c:75-93), formed as normal.c:39-40 forms it.  The FP32 form
 // takes the cross product itself (the same vector): a triangle whose
@@ -2230,7 +2211,7 @@ __global__ __launch_bounds__(kThreads) void k_smooth(MeshView<R> m, const ObjMet
 // takes (null: not wanted), as doubles: positions, weights, vertex normals
 // (vn: n rows of the mesh's precision), cells and edges.
 //
-// Bound by the copies to the host that follow it: 90 bytes a triangle over
+// Bound by the copies to the host that follow it: 176 bytes a triangle over
 // the bus.  Records unpacked by the host after a copy of them took 3.5 to 9
 // ms for 61 x 57 x 50 turbulence built, copied and freed, by the state of the
 // host allocator (8.2 beside the 1.98 this takes).
@@ -2333,7 +2314,10 @@ struct FieldSource {
       if (sl >= c_ntri[code]) continue;
       const uint32_t ent = uint32_t(c_cslot[code * 12u + sl]);
       V3<R> wpos[3];
-      slot_positions<R>(f, L, thr, ent, cv, wpos);
+      // (the vertices' six values are read again, from L1: choosing them from
+      // the eight in registers took 126 selects; four 1280 x 720 cameras 1.90
+      // ms instead of 1.885, other frames within 0.5 %)
+      slot_positions_mem<R>(f, L, thr, ent & 0x3ffffu, wpos);
       weights_at(v, wpos, i, j, X);
 #pragma unroll
       for (int n = 0; n < 3; n++) {
