@@ -5,16 +5,20 @@ turbulence field (modes 1 <= |k| <= 64, k^-5/3 shell spectrum, seeded
 phases, mean 0 / variance 1) resident in HBM, thresholds {-1, 0, 1} as three
 contour objects, one 1920x1080 image written to HBM.  A step is one
 contour3d_amd_execute_rgb call; Gcells/s counts 3 * 511^3 cell-thresholds
-per frame.  `value` is the FP64 form (bit-identical to the reference).
+per frame: every cell is classified against every threshold in every frame,
+while triangles behind what the frame has drawn are not drawn (the image and
+its depths are the same).  `value` is the FP64 form (bit-identical to the
+reference).
 
 Beside it, in the same JSON line:
   fp32        the FP32-geometry form of the same frame
   roofline    the dominant kernel of the FP64 frame, the fused tessellation
-              + raster kernel (k_tess_raster), timed alone with HIP events
-              on its stream, charged with the graded tessellation bytes
-              B_tess = 8 N + 96 T (the field once, the FP64 triangles); its
-              measured HBM traffic and VALU figures come from the rocprofv3
-              summary under profiles/
+              + raster kernel (k_frame), timed alone with HIP events on its
+              stream, charged with the bytes it cannot do without: the field
+              once and a z-buffer key per pixel (it stores no triangles and
+              leaves out hidden ones, so bytes per triangle would charge it
+              with traffic it does not have); its measured HBM traffic and
+              VALU figures come from the rocprofv3 summary under profiles/
   tessellation  the stored-mesh tessellation (count + scan + emit of
               contour3d_amd_mesh_build) on the same field, FP32 and FP64,
               against B_tess (48 B per FP32 triangle, 96 B per FP64 one),
@@ -72,9 +76,9 @@ def algorithmic_bytes(stage, T, npts, npx, fp64):
     count    the field, read once for all thresholds (8 B per lattice point)
     emit     B_tess: the field once + per triangle 3 positions and the
              weighted face normal (96 B in FP64, 48 B in FP32)
-    fused    the fused tessellation + raster kernel, charged with the
-             graded tessellation bytes B_tess of the same triangles (it
-             tessellates them and draws them without storing them)
+    fused    the fused tessellation + raster kernel: the field once and a
+             z-buffer key per pixel (triangles are drawn, or left out as
+             hidden, without being stored)
     smooth   B_smooth: per triangle 3 edge keys (24 B), the face normal and
              area (12 + 4 B) in and 3 vertex normals (36 B) out in FP32
              (76 B); the same in FP64 is 24 + 32 + 72 = 128 B
@@ -85,8 +89,10 @@ def algorithmic_bytes(stage, T, npts, npx, fp64):
     r = 8 if fp64 else 4
     if stage == "count":
         return 8 * npts
-    if stage in ("emit", "fused"):
+    if stage == "emit":
         return 8 * npts + 12 * r * T
+    if stage == "fused":
+        return 8 * npts + 8 * npx
     if stage == "smooth":
         return (128 if fp64 else 76) * T
     if stage == "resolve":
@@ -766,7 +772,7 @@ def main():
     dom_b = algorithmic_bytes("fused", r["T"], npts, npx, True)
     achieved = dom_b / (fused_ms * 1e-3) / 1e9
     prof = profile_summary() if n == 512 else {}
-    kprof = prof.get("kernels", {}).get("k_tess_raster<double,3>", {})
+    kprof = prof.get("kernels", {}).get("k_frame<double,0>", {})
     copy_gbs = copy_bandwidth()
     log("stored-mesh tessellation (mesh build) and smoothing, FP64 and FP32")
     tess = {}
@@ -801,12 +807,12 @@ def main():
                                f"thresholds {{-1,0,1}}, {W}x{H} image in HBM",
                    "lattice": [n, n, n], "thresholds": list(THRESHOLDS), "image": [W, H],
                    "triangles_per_frame": int(r["T"])},
-        "roofline": {"bound": "hbm", "kernel": "k_tess_raster<double> (fused tessellation + raster, FP64 frame)",
+        "roofline": {"bound": "hbm", "kernel": "k_frame<double> (fused tessellation + raster, FP64 frame)",
                      "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": kprof.get("hbm_bytes"),
                      "copy_gbs": round(copy_gbs, 1), "frac_of_copy": round(achieved / copy_gbs, 4),
                      "algorithmic_bytes": round(dom_b), "kernel_ms": fused_ms,
-                     "algorithmic": "B_tess = 8 B x lattice points + 96 B x triangles",
+                     "algorithmic": "8 B x lattice points + 8 B x pixels",
                      "limiter": kprof.get("limiter"), "valu": kprof.get("valu"),
                      "profile": os.path.relpath(PROFILE_MD, ROOT) if kprof else None},
         "tessellation": tess,
