@@ -82,7 +82,7 @@ uint64_t next_buf_gen() {
 // Device blocks of freed meshes, kept for the next mesh: a mesh is built,
 // read and freed again and again (a surface per time step), and at 256^3 and
 // two thresholds the driver took 42 ms to allocate and free what the kernels
-// fill in 1.8 ms.  At most kPoolBytes are held (one FP64 mesh of 512^3 and
+// fill in 1.3 ms.  At most kPoolBytes are held (one FP64 mesh of 512^3 and
 // three thresholds takes 18 GB); the oldest go first, an allocation that
 // fails empties the pool and tries again, and contour3d_amd_finalize gives
 // everything back.  Blocks come here only after the device is done with

@@ -912,13 +912,14 @@ __global__ __launch_bounds__(kThreads) void k_raster(MeshView<R> m, const Raster
 // -> 2.81 ms, 1024^3 19.1 -> 16.9 ms), and the latency of each brick's chain
 // of reads.  Letting every lane walk to its next covered pixel before any of
 // them forms a depth was no faster on small triangles and slower on large
-// ones (close-up 1.65 -> 2.51 ms).  That FP64 frame's kernel took 4.50 ms as a tessellation of whole
-// rows with a queue and barriers per workgroup, no z-test and no order; 3.61
-// ms in bricks taken front to back by workgroups; and 2.2 ms by waves, with
-// the cut cells listed before anything is done with them (FP32, where every
-// triangle is drawn: 3.41 -> 2.8 ms, besides 0.28 ms of counting passes that
-// serial ids had needed).  Close-ups, where few triangles cover many pixels
-// each, gained most: 301 x 187 x 223 with five thresholds 8.15 -> 1.4 ms.
+// ones (close-up 1.65 -> 2.51 ms).  The 512^3 FP64 frame's kernel took 4.50
+// ms as a tessellation of whole rows with a queue and barriers per workgroup,
+// no z-test and no order; 3.61 ms in bricks taken front to back by
+// workgroups; 2.2 ms by waves, with the cut cells listed before anything is
+// done with them; and 1.86 ms since (FP32, where every triangle is drawn:
+// 3.41 -> 2.56 ms, besides 0.28 ms of counting passes that serial ids had
+// needed).  Close-ups, where few triangles cover many pixels each, gained
+// most: 301 x 187 x 223 with five thresholds 8.15 -> 1.19 ms.
 //
 // Every covered pixel is tested against the z-buffer as it is drawn (key:
 // the depth's order key, larger is nearer); a fragment at or above the value

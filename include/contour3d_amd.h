@@ -76,8 +76,8 @@ extern int contour3d_amd_execute_rgb(
  * reference.  For callers that cannot allocate device memory -- code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc --
  * this variant calls no hipMalloc, hipFree or other allocating routine.  Its
- * intermediate buffers (tile counts and starts, job tables, the cell store,
- * z-buffer, fragment list, line fragments, lattice grids) are regions of one
+ * intermediate buffers (brick order, job tables, z-buffer, fragment list,
+ * line fragments, lattice grids) are regions of one
  * static device array of 128 MiB that each GPU the library runs on holds
  * until the process ends; contour3d_amd_init (or the first call of any
  * other entry point) sets it up, and this call returns 1 before that.
@@ -87,10 +87,11 @@ extern int contour3d_amd_execute_rgb(
  *   rgb        device, W*H*3 bytes in PPM row order
  *   depth      device W*H doubles, or NULL
  * Limits (1 with an error line beyond them): 2^21 pixels (1920x1080 fits),
- * 2^24 triangles in FP32 (FP64 frames store nothing per triangle), 64
- * contour objects, 2^20 tessellation tiles (about 2^31 cells), 2^18 line
- * fragments, 65536 lattice coordinates; an FP64 frame with more than 2^19
- * covered pixel centres takes the slower z-test passes.  Results are
+ * 2^24 triangles in FP32 (frames store nothing per triangle; the limit is
+ * kept), 64 contour objects, 2^20 tessellation tiles (about 2^31 cells), 2^18
+ * line fragments, 65536 lattice coordinates; a frame with more than 3 * 2^20
+ * fragments that may be nearest takes the slower id pass over the geometry.
+ * Results are
  * bit-identical to contour3d_amd_execute_rgb.  Every call on a GPU shares
  * that GPU's array and keeps the last call's contents; calls are serialised
  * by the library mutex, and calls that overlapped on one GPU would race.
@@ -281,13 +282,14 @@ extern int contour3d_amd_mesh_free(contour3d_amd_mesh_t * mesh);
 /* Launch-shape and capacity parameters.  None changes a result: every
  * setting renders the same bits. */
 enum {
-  CONTOUR3D_AMD_TUNE_TESS_GRID = 0,     /* max workgroups of the tessellation kernels (count, the fused
-                                           tessellation + raster, emit); each walks several tiles
-                                           (0: the defaults, 128 per CU, and one per tile for emit) */
+  CONTOUR3D_AMD_TUNE_TESS_GRID = 0,     /* max workgroups of the tessellation kernels (a frame's fused
+                                           tessellation + raster, a mesh's count and emit); each takes
+                                           several bricks or tiles (0: the defaults, 6 per CU for frames,
+                                           128 per CU for count, and one per tile for emit) */
   CONTOUR3D_AMD_TUNE_RASTER_GRID = 1,   /* max workgroups of the raster passes (0 = one per 256 triangles) */
-  CONTOUR3D_AMD_TUNE_FRAG_CAPACITY = 2, /* FP64 fragment list entries, 24 B each (0: the default, 2^24; grows by
+  CONTOUR3D_AMD_TUNE_FRAG_CAPACITY = 2, /* fragment list entries, 24 B each (0: the default, 2^24; grows by
                                            itself after an overflow; an overflowing frame takes the slower
-                                           z-test passes over the geometry) */
+                                           id pass over the geometry) */
   CONTOUR3D_AMD_TUNE_GRAPHS = 3,        /* 1: contour3d_execute, _execute_rgb and _execute_batch capture
                                            their launch sequence as a HIP graph and replay it while the
                                            frame layout (image sizes, objects' fields and lattices,
@@ -297,10 +299,12 @@ enum {
                                            the n-th device or pinned allocation from now fail as an
                                            out-of-memory would (once); the call that needed it returns 1
                                            with the error line, and the library stays usable.  0 disarms. */
-  CONTOUR3D_AMD_TUNE_TESS_ROWS = 5,     /* tessellation brick: rows of cells per tile, at most 2048 cells
-                                           (0: as many rows as fit) */
-  CONTOUR3D_AMD_TUNE_TESS_ZPLANES = 6   /* tessellation brick: z-planes one workgroup marches through per
-                                           work item (0: the default, 4) */
+  CONTOUR3D_AMD_TUNE_TESS_ROWS = 5,     /* rows of cells of a frame's brick (up to 8, of at most 64 columns) and
+                                           of a mesh's tile (of at most 2048 cells); 0: a brick by the work of
+                                           the view, a tile of as many rows as fit */
+  CONTOUR3D_AMD_TUNE_TESS_ZPLANES = 6   /* planes of a frame's brick (up to 8), and z-planes that one workgroup
+                                           of a mesh's tessellation marches through per work item; 0: by the
+                                           work of the view, and 4 */
 };
 
 extern int contour3d_amd_tune(int param, int64_t value);
@@ -312,8 +316,8 @@ extern int contour3d_amd_tune(int param, int64_t value);
  * nearest to each pixel; they are gathered inside the RESOLVE stage, so the
  * SMOOTH stage stays at zero for frames. */
 enum {
-  CONTOUR3D_AMD_STAGE_COUNT = 0,   /* classify + per-tile triangle counts */
-  CONTOUR3D_AMD_STAGE_SCAN = 1,    /* tile scan + totals */
+  CONTOUR3D_AMD_STAGE_COUNT = 0,   /* classify + per-tile triangle counts (stored meshes) */
+  CONTOUR3D_AMD_STAGE_SCAN = 1,    /* tile scan + totals (stored meshes) */
   CONTOUR3D_AMD_STAGE_EMIT = 2,    /* triangle emission */
   CONTOUR3D_AMD_STAGE_SMOOTH = 3,  /* vertex normals of every triangle (contour3d_amd_mesh_normals; not used
                                       by frames) */
