@@ -1107,11 +1107,11 @@ double cell_pixels(const ViewDev<R>& v, const LatticeMid& m, const uint32_t n[3]
 //   180^3, a close-up                  916 ->  720    (8 x 8 x 2)
 //   301 x 187 x 223, a close-up       1468 -> 1379    (8 x 8 x 2)
 //   24 fields of 48^3 to 256^3, FP32  4959 -> 4151
-//   100^3, 1920 x 1080, a deep close-up 41756 -> 11998  (2 x 2 x 1)
+//   100^3, 1920 x 1080, a deep close-up 41756 -> 11998  (2 x 2 x 1; since then 2.3 ms, see draw_wave)
 //   256^3, 1920 x 1080                 776 ->  776    (8 x 8 x 8)
 // kVolume of 0.2 costs 128^3 blobs 248 and the 24 fields 4400, 0.45 costs the
 // 33 x 29 x 31 close-up 294 and 180^3 770; kSetupPixels of 15 costs the 24
-// fields 4563 and 33 x 29 x 31 291; kMostPixels of 256 costs 100^3 19559.
+// fields 4563 and 33 x 29 x 31 291; kMostPixels of 256 cost 100^3 19559 then.
 constexpr double kVolume = 0.3, kSetupPixels = 5, kLightPixels = 100, kMostPixels = 4096, kMostBricks = 131072;
 
 template <typename R>
