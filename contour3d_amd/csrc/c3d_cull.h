@@ -35,17 +35,23 @@
 //
 // What the area has to be.  Let u be the unit roundoff, g = 4.5 u, L a bound
 // on the projected extent of the brick (x and y ranges added), p the larger
-// pixel spacing and E a bound on the error of a projected vertex.  A
-// candidate pixel lies within L + 6 p of every vertex, so each computed edge
-// function is within g (L + 6 p) L of its exact value for the computed
-// vertices, their sum is the exact area of the computed vertices, and that is
-// within 6 E L of A.  Hence with
+// and s the smaller pixel spacing and E a bound on the error of a projected
+// vertex.  A candidate pixel lies within L + 6 p of every vertex, so each
+// computed edge function is within g (L + 6 p) L of its exact value for the
+// computed vertices, their sum is the exact area of the computed vertices, and
+// that is within 6 E L of A.  Hence with
 //   need = 2 (3 g (L + 6 p) L / kSlack + 6 E L),
 // and at least 4e-16 (above the reference's clamp of the area at 1e-16),
-// every A >= need gives weights whose sum is within kSlack of one.  Pixels
-// farther than the widened box (the reference clamps boxes to the image)
-// lie outside the triangle by more than a pixel spacing, where some exact
-// weight is below -p / (3 L); with L < 2000 p that is beyond rounding.
+// every A >= need gives weights whose sum is within kSlack of one, each within
+// kSlack / 6 of its exact value.  Pixels farther than the widened box (the
+// reference clamps boxes to the image) lie outside the triangle by more than
+// s, where some exact weight is below -s / (3 L); with L < 10000 s that is
+// beyond rounding.
+// All of it needs vertices that are near where they should be: 24 E < L, so
+// that L holds and the area's error is 6 E L at most, and E < s / 4, so that
+// the widened box holds.  Where a lattice's spacing nears the last place of
+// its coordinates neither is true, down to bricks whose corners all round
+// onto one screen point (L = 0, with which any area would do).
 #pragma once
 
 #include "c3d_geom.h"
@@ -90,8 +96,9 @@ struct BrickLimits {
 C3D_HD bool brick_limits(const ViewDev<double>& v, const BrickRange& r, BrickLimits& o) {
   const double u = 1.1102230246251565e-16, g = 4.5 * u;
   const double p = v.pitch;
+  const double s = 1.0 / fmax(v.fw, v.fh);
   const double L = (r.x1 - r.x0) + (r.y1 - r.y0);
-  if (!(L < 2000.0 * p)) return false;
+  if (!(L < fmin(2000.0 * p, 10000.0 * s))) return false;
   // one sign of depth, and not too wide a range of it
   if (!(r.n0 * r.n1 > 0.0)) return false;
   const double nmin = fmin(fabs(r.n0), fabs(r.n1)), nmax = fmax(fabs(r.n0), fabs(r.n1));
@@ -103,6 +110,8 @@ C3D_HD bool brick_limits(const ViewDev<double>& v, const BrickRange& r, BrickLim
   const double l = sqrt(fmin(v.lxx, v.lyy));
   const double q = fmax(fmax(fabs(r.x0), fabs(r.x1)), fmax(fabs(r.y0), fabs(r.y1)));
   const double E = 64.0 * u * (S * (1.0 + r.size / nmin) / l + 1.0 + q);
+  // (false also where E is not a number)
+  if (!(E < 0.25 * s && 24.0 * E < L)) return false;
   const double need = fmax(2.0 * (3.0 * g * (L + 6.0 * p) * L / kSlack + 6.0 * E * L), 4.0e-16);
   const double scale = v.cv / (need * nmax * nmax * nmax);
   if (!(scale > 0.0 && scale < 1.0e30)) return false;
