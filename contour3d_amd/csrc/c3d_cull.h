@@ -89,7 +89,7 @@ struct BrickRange {
 struct BrickLimits {
   int32_t i0, i1, j0, j1;  // pixels its regular cells' fragments fall on (empty: i1 < i0 or j1 < j0)
   double bound;            // no fragment of a regular cell has a larger depth
-  float scale;             // cell_regular's: cv / (need |nr|^3), per unit of cell volume
+  double scale;            // cell_volume's: cv / (need |nr|^3), per unit of cell volume
 };
 
 // false: nothing can be said of the brick
@@ -115,7 +115,7 @@ C3D_HD bool brick_limits(const ViewDev<double>& v, const BrickRange& r, BrickLim
   const double need = fmax(2.0 * (3.0 * g * (L + 6.0 * p) * L / kSlack + 6.0 * E * L), 4.0e-16);
   const double scale = v.cv / (need * nmax * nmax * nmax);
   if (!(scale > 0.0 && scale < 1.0e30)) return false;
-  o.scale = float(scale) * 0.999999f;
+  o.scale = scale;
   o.bound = r.n1 + kNearBy * fabs(r.n1);
   // boxes of pixel indices, widened by three; far off the image they are
   // clamped to a few pixels outside it
@@ -164,14 +164,27 @@ C3D_HD void cell_values(const double v[8], float X, float Y, float Z, CellValues
   c.at[4] = y2 + (c.e[6] - c.e[2]) * Z + (c.e[7] - c.e[6]) * X;
   c.at[5] = y2 + (c.e[3] - c.e[2]) * X + (c.e[7] - c.e[3]) * Z;
   // coordinates and differences are rounded once or twice each, products and
-  // sums once: under 8 units of 2^-24 per term
-  c.err = 1.0e-6f * (fabsf(X) + fabsf(Y) + fabsf(Z) + 1.0f);
+  // sums once: under 8 units of 2^-24 per term.  A camera so far off, in
+  // cells, that a product could leave float's range (which a minimum passes
+  // over once it is not a number) makes the bound one that nothing meets.
+  const float far = fabsf(X) + fabsf(Y) + fabsf(Z);
+  c.err = far < 1.0e15f ? 1.0e-6f * (far + 1.0f) : HUGE_VALF;
+}
+
+// scale * |hx hy hz| for cell_regular, from edges and a scale of any size: the
+// product is formed in FP64 and cut off at 1e20 (a smaller volume makes fewer
+// cells regular), and it is 0 where an edge, which the camera's place in cells
+// is divided by in FP32, comes near the ends of that range.
+C3D_HD float cell_volume(double hx, double hy, double hz, double scale) {
+  const double x = fabs(hx), y = fabs(hy), z = fabs(hz), v = x * y * z * scale;
+  if (!(fmin(fmin(x, y), z) > 1.0e-30 && fmax(fmax(x, y), z) < 1.0e30)) return 0.0f;
+  return v < 1.0e20 ? float(v) * 0.999999f : 1.0e20f;
 }
 
 // Whether every triangle of the cell at a threshold is regular; d0: value of
-// corner 0 minus the threshold; volume: scale * hx hy hz.  False for values
-// that are not finite, and below 1e-8 (where the interpolation keeps a
-// corner instead of a point between two).
+// corner 0 minus the threshold; volume: cell_volume.  False for values that
+// are not finite, and below 1e-8 (where the interpolation keeps a corner
+// instead of a point between two).
 C3D_HD bool cell_regular(const CellValues& c, float d0, float volume) {
   float m = fabsf(d0), f = fabsf(c.at[0] + d0);
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -1221,7 +1221,7 @@ __device__ __forceinline__ bool box_above(const uint64_t* __restrict__ key, uint
 __device__ __forceinline__ uint32_t reachable_images(const FieldDev& f, BrickBox B,
                                                      const RasterJob<double>* __restrict__ rjobs,
                                                      const uint32_t* __restrict__ jimg, uint32_t u0, uint32_t u1,
-                                                     const uint64_t* __restrict__ key, float& scale) {
+                                                     const uint64_t* __restrict__ key, double& scale) {
   uint32_t seen = kAllImages;
   const uint32_t c = __lane_id() & 7u;
   const double px = gptr(f.gx)[B.i0 + (c & 1u) * (B.i1 - B.i0)], py = gptr(f.gy)[B.j0 + (c >> 1 & 1u) * (B.j1 - B.j0)],
@@ -1261,7 +1261,7 @@ __device__ __forceinline__ uint32_t reachable_images(const FieldDev& f, BrickBox
 __device__ __forceinline__ uint32_t irregular_at(const TessJob& J, uint32_t i, uint32_t j, uint32_t k, uint32_t cuts,
                                                  const RasterJob<double>* __restrict__ rjobs,
                                                  const uint32_t* __restrict__ jimg, uint32_t u0, uint32_t seen,
-                                                 float scale, bool inner) {
+                                                 double scale, bool inner) {
   const FieldDev& f = J.f;
   double v[8], x0 = 0, y0 = 0, z0 = 0, hx = 1, hy = 1, hz = 1;
   if (inner) {
@@ -1277,12 +1277,11 @@ __device__ __forceinline__ uint32_t irregular_at(const TessJob& J, uint32_t i, u
     hz = gptr(f.gz)[k + 1u] - z0;
   }
   const float fx = float(hx), fy = float(hy), fz = float(hz);
-  const float cell = fabsf(fx * fy * fz) * 0.999999f;
   uint32_t bad = 0;
   for (uint32_t hid = ~seen & kAllImages; hid; hid &= hid - 1u) {
     const uint32_t u = uint32_t(__builtin_ctz(hid));
     const ViewDev<double>& vw = rjobs[uniform(jimg[u0 + u])].v;
-    const float volume = cell * lane_of(scale, int(u));
+    const float volume = cell_volume(hx, hy, hz, lane_of(scale, int(u)));
     if (inner) {
       CellValues cv;
       cell_values(v, float(vw.cam[0] - x0) / fx, float(vw.cam[1] - y0) / fy, float(vw.cam[2] - z0) / fz, cv);
@@ -1405,7 +1404,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(sizeof
     }
     uint32_t seen = kAllImages;  // the images that the brick's regular cells may reach
     bool unseen = false;         // none at all
-    float scale = 0.0f;
+    double scale = 0.0;
     if constexpr (sizeof(R) == 8) {
       if (ncut && jobs[jb].f.ordered) {
         const uint32_t u0 = uniform(jimg[jb]), u1 = uniform(jimg[jb + 1u]);

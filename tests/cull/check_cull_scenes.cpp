@@ -114,7 +114,7 @@ static void one_scene(const Scene& S, int kind, Stats& st) {
         CellValues cv;
         cell_values(w, float(v.cam[0] - g[0][i]) / fx, float(v.cam[1] - g[1][j]) / fy, float(v.cam[2] - g[2][k]) / fz,
                     cv);
-        if (!cell_regular(cv, float(w[0] - thr), fabsf(fx * fy * fz) * 0.999999f * lim.scale)) continue;
+        if (!cell_regular(cv, float(w[0] - thr), cell_volume(hx, hy, hz, lim.scale))) continue;
         st.regular++;
         for (int t = 0; t < 6; t++) {
           int m = 0;

@@ -1,5 +1,5 @@
 """CPU: the rule of contour3d_amd/csrc/c3d_cull.h on whole scenes moved away
-from the origin and on images of extreme proportions
+from the origin, scaled and stretched, and on images of extreme proportions
 (tests/cull/check_cull_scenes.cpp): no fragment of a cell that the rule calls
 regular may leave its brick's pixel box or come nearer than its bound, down
 to lattice spacings of a unit in the last place of the coordinates."""
@@ -38,3 +38,18 @@ def test_scenes_far_from_the_origin(check):
 
 def test_images_of_extreme_proportions(check):
     check("wide:8", "wide:14")
+
+
+def test_scenes_of_any_length_scale(check):
+    """A power of two changes no rounding, so the same cells are regular at
+    every scale; past the ends of the range that the rule takes, none are."""
+    got = check("scale:0", "scale:20", "scale:40", "scale:54", "scale:62", "scale:90", "scale:120", "scale:200",
+                "scale:-60")
+    assert got["scale:0"][1] > 0
+    for s in ("scale:20", "scale:40", "scale:54", "scale:62", "scale:90"):
+        assert got[s] == got["scale:0"], s
+    assert got["scale:120"][1] == got["scale:200"][1] == got["scale:-60"][1] == 0
+
+
+def test_cells_of_extreme_proportions(check):
+    check("stretch:-10", "stretch:-40", "stretch:-80", "stretch:-120", "stretch:-149", "stretch:2")
