@@ -4,6 +4,7 @@
 #include "contour3d.h"
 #include "contour3d_amd.h"
 #include "c3d_internal.h"
+#include "c3d_pool.h"
 #include "c3d_wait.h"
 
 #include <cerrno>
@@ -71,78 +72,39 @@ bool injected_alloc_failure() {
   return false;
 }
 
-// grow-only device buffer, or (fixed) a region of the static scratch array
-// that never grows
 // A number no device buffer allocation has had before (DevBuf::gen).
 uint64_t next_buf_gen() {
   static std::atomic<uint64_t> g{0};
   return ++g;
 }
 
-// Device blocks of freed meshes, kept for the next mesh: a mesh is built,
-// read and freed again and again (a surface per time step), and at 256^3 and
-// two thresholds the driver took 42 ms to allocate and free what the kernels
-// fill in 1.3 ms.  At most kPoolBytes are held (one FP64 mesh of 512^3 and
-// three thresholds takes 18 GB); the oldest go first, an allocation that
-// fails empties the pool and tries again, and contour3d_amd_finalize gives
-// everything back.  Blocks come here only after the device is done with
-// them, so any stream may take them.
-constexpr size_t kPoolBytes = size_t(24) << 30;
-
-struct BlockPool {
-  struct Block {
-    void* p;
-    size_t bytes;
-  };
-  std::mutex mu;
-  std::vector<Block> blocks;  // oldest first
-  size_t held = 0;
-  // the smallest block of at least `want` bytes that is not more than twice
-  // that (small requests: 64 KiB more)
-  void* take(size_t want, size_t& got) {
-    std::lock_guard<std::mutex> g(mu);
-    size_t best = blocks.size();
-    for (size_t q = 0; q < blocks.size(); q++)
-      if (blocks[q].bytes >= want && blocks[q].bytes <= 2 * want + 65536 &&
-          (best == blocks.size() || blocks[q].bytes < blocks[best].bytes))
-        best = q;
-    if (best == blocks.size()) return nullptr;
-    void* p = blocks[best].p;
-    got = blocks[best].bytes;
-    held -= got;
-    blocks.erase(blocks.begin() + std::ptrdiff_t(best));
-    return p;
-  }
-  void give(void* p, size_t bytes) {
-    std::lock_guard<std::mutex> g(mu);
-    if (bytes > kPoolBytes) {
-      (void)hipFree(p);
-      return;
-    }
-    while (held + bytes > kPoolBytes) {
-      held -= blocks.front().bytes;
-      (void)hipFree(blocks.front().p);
-      blocks.erase(blocks.begin());
-    }
-    blocks.push_back({p, bytes});
-    held += bytes;
-  }
-  // frees every block; false if there was none
-  bool drop() {
-    std::lock_guard<std::mutex> g(mu);
-    const bool any = !blocks.empty();
-    for (const Block& b : blocks) (void)hipFree(b.p);
-    blocks.clear();
-    held = 0;
-    return any;
-  }
-};
-
+// The pool of freed meshes' blocks (one FP64 mesh of 512^3 and three
+// thresholds takes 18 GB).  It holds blocks only while the library is
+// initialised, and of that device (contour3d_amd_mesh_free):
+// contour3d_amd_finalize gives everything back.
 BlockPool& block_pool() {
-  static BlockPool p;
+  static BlockPool p(size_t(24) << 30, [](void* b) { (void)hipFree(b); });
   return p;
 }
 
+// hipMalloc; one that fails for want of memory empties the pool and tries
+// again.  An injected failure fails both times.
+hipError_t device_malloc(void** p, size_t n) {
+  const bool fail = injected_alloc_failure();
+  hipError_t e = fail ? hipErrorOutOfMemory : hipMalloc(p, n);
+  if (e == hipErrorOutOfMemory && block_pool().drop()) {
+    (void)hipGetLastError();  // (a later launch does not report what was handled here)
+    e = fail ? hipErrorOutOfMemory : hipMalloc(p, n);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+  }
+  return e;
+}
+
+// grow-only device buffer, or (fixed) a region of the static scratch array
+// that never grows
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -168,14 +130,8 @@ struct DevBuf {
       gen = next_buf_gen();
       return hipSuccess;
     }
-    if (injected_alloc_failure()) return hipErrorOutOfMemory;
-    hipError_t e = hipMalloc(&p, n);
-    if (e == hipErrorOutOfMemory && block_pool().drop()) {
-      (void)hipGetLastError();
-      e = hipMalloc(&p, n);
-    }
+    const hipError_t e = device_malloc(&p, n);
     if (e != hipSuccess) {
-      p = nullptr;
       gen = 0;
       return e;
     }
@@ -297,10 +253,11 @@ struct contour3d_amd_mesh {
   std::vector<uint32_t> tiles;  // tiles of each object's field
   std::vector<c3d::TileGeo> geo;  // and their layout
   std::vector<contour3d_color_t> color;
+  int device = -1;  // a stored mesh: the device its buffers are on
   // a stored mesh: its buffers come from and go to the block pool, so
   // release() needs the device to be done with them
-  void use_pool() {
-    for (c3d::DevBuf* b : {&pos, &aux, &bstart, &meta, &code, &cstart}) b->pooled = true;
+  void use_pool(bool on) {
+    for (c3d::DevBuf* b : {&pos, &aux, &bstart, &meta, &code, &cstart}) b->pooled = on;
   }
   void release() {
     pos.release();
@@ -2154,11 +2111,7 @@ void* snap_take(Server& S, size_t bytes, size_t& got) {
     }
   }
   void* p = nullptr;
-  if (injected_alloc_failure()) return nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess || !p) {
-    (void)hipGetLastError();
-    if (!block_pool().drop() || hipMalloc(&p, bytes) != hipSuccess || !p) return nullptr;
-  }
+  if (device_malloc(&p, bytes) != hipSuccess || !p) return nullptr;
   std::lock_guard<std::mutex> g(S.pool_mu);
   S.snap_all.push_back({p, bytes});
   S.snap_held += bytes;
@@ -2732,7 +2685,8 @@ int contour3d_amd_mesh_build(const contour3d_contour_obj_t* contour_objs, size_t
   std::lock_guard<std::mutex> g(L.mu);
   if (c3d::ensure_init(L, 0)) return 1;
   auto M = std::make_unique<contour3d_amd_mesh>();
-  M->use_pool();
+  M->use_pool(true);
+  M->device = L.device;
   const int rc = c3d::build_mesh(L, L.main, *M, contour_objs, num_contours, precision);
   const hipError_t e = hipStreamSynchronize(L.main.st);
   c3d::release_geoms(L.main);
@@ -2871,7 +2825,10 @@ int contour3d_amd_mesh_free(contour3d_amd_mesh_t* mesh) {
   if (!mesh) return 0;
   auto& L = lib();
   std::lock_guard<std::mutex> g(L.mu);
-  if (L.ready) (void)hipStreamSynchronize(L.main.st);
+  // after finalize, or on another device since, the blocks go back to the
+  // driver (hipFree waits for the device): nothing would give them back later
+  if (L.ready && mesh->device == L.device) (void)hipStreamSynchronize(L.main.st);
+  else mesh->use_pool(false);
   mesh->release();
   delete mesh;
   return 0;

@@ -35,7 +35,8 @@ extern int contour3d_amd_init(int device);
 
 /* Free every device buffer, cached geometry and the stream.  The library
  * keeps device buffers between calls (grow-only) so that repeated frames do
- * not allocate; this returns them. */
+ * not allocate, and up to 24 GiB of freed meshes' (contour3d_amd_mesh_free);
+ * this returns them. */
 extern int contour3d_amd_finalize(void);
 
 /* Arithmetic form used by contour3d_execute (default CONTOUR3D_AMD_FP64). */
@@ -275,6 +276,12 @@ extern int contour3d_amd_mesh_render(
 extern int contour3d_amd_mesh_compare(const contour3d_amd_mesh_t * a, const contour3d_amd_mesh_t * b, size_t obj,
                                       double stats[8]);
 
+/* Free a mesh.  While the library is initialised on the mesh's device, its
+ * device memory is kept for the next mesh_build, up to 24 GiB in all: the
+ * library's own allocations take it back when they need it, but to another
+ * allocator of the process (torch's, hipMalloc) it is in use until
+ * contour3d_amd_finalize.  A mesh freed after contour3d_amd_finalize returns
+ * its memory at once. */
 extern int contour3d_amd_mesh_free(contour3d_amd_mesh_t * mesh);
 
 /* ---- tuning ------------------------------------------------------------- */
