@@ -2719,10 +2719,26 @@ int contour3d_amd_mesh_copy(const contour3d_amd_mesh_t* mesh, size_t obj, double
   auto& L = lib();
   std::lock_guard<std::mutex> g(L.mu);
   if (mesh->count[obj] == 0 || !(pos || wfn || vn || cell || edges)) return 0;
-  if (c3d::ensure_init(L, 0)) return 1;
-  return mesh->precision == CONTOUR3D_AMD_FP64
-             ? c3d::mesh_copy_t<double>(L.main, *mesh, obj, pos, wfn, vn, cell, edges)
-             : c3d::mesh_copy_t<float>(L.main, *mesh, obj, pos, wfn, vn, cell, edges);
+  if (c3d::ensure_init(L, mesh->device)) return 1;
+  const auto copy = [&](c3d::Frame& F) {
+    return mesh->precision == CONTOUR3D_AMD_FP64 ? c3d::mesh_copy_t<double>(F, *mesh, obj, pos, wfn, vn, cell, edges)
+                                                 : c3d::mesh_copy_t<float>(F, *mesh, obj, pos, wfn, vn, cell, edges);
+  };
+  if (mesh->device == L.device) return copy(L.main);
+  // The library has gone to another device since the mesh was built, whose
+  // kernels may not be able to read this one's memory: the records are
+  // unpacked where they are, on a stream of their own.  Vertex normals need
+  // tables that only the library's device has.
+  if (vn) {
+    c3d::log_error("mesh_copy: vertex normals of a mesh on device %d, the library is on device %d", mesh->device,
+                   L.device);
+    return 1;
+  }
+  c3d::Frame there;
+  const int rc = hipSetDevice(mesh->device) == hipSuccess && there.create() == hipSuccess ? copy(there) : 1;
+  if (rc) c3d::log_error("mesh_copy failed on device %d", mesh->device);
+  there.release();
+  return hipSetDevice(L.device) == hipSuccess ? rc : 1;
 }
 
 int contour3d_amd_mesh_normals(const contour3d_amd_mesh_t* mesh, size_t obj, void* vn) {
