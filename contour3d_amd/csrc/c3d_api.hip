@@ -1543,7 +1543,9 @@ int raster_prepare(Frame& F, uint64_t npx, bool stored) {
   F.h_nline = nf;
   if (upload_table(F, F.hdr, offsetof(FrameHdr, nline), &F.h_nline, sizeof(uint32_t))) return 1;
   if (F.frag_cap == 0) F.frag_cap = kDefaultFragCap;
-  C3D_HIP(F.frags.ensure(size_t(F.frag_cap) * sizeof(Frag64)));
+  // a stored mesh's entries are smaller, and in FP32 it keeps no list
+  const size_t entry = !stored ? sizeof(Frag64) : fp64 ? sizeof(Frag) : 0;
+  C3D_HIP(F.frags.ensure(size_t(F.frag_cap) * entry));
   return 0;
 }
 
