@@ -110,13 +110,15 @@ C3D_HD void set_cv(ViewDev<R>& v) {
 // constant).  The compiler's IEEE division is v_div_scale of the
 // denominator, v_rcp and two Newton steps on it, then v_div_scale of the
 // numerator, a product, an FMA, v_div_fmas and v_div_fixup.  Here the
-// denominator half is rb, computed once for all numerators (recip_shared, or
-// 1 / b rounded once), and the rest is the same instructions: with such an
-// rb the quotient before the last FMA is within a unit in the last place,
-// and the FMA rounds it correctly (Markstein).  The denominator's
+// denominator half is rb = 1 / b rounded once (by the host: set_recips), and
+// the rest is the same instructions: with such an rb the quotient before the
+// last FMA is within a unit in the last place, and the FMA rounds it correctly
+// (Markstein).  The denominator's
 // v_div_scale depends on a too: it leaves b unchanged except at extreme
 // exponent ratios, which is checked per numerator, and any other case takes
 // the plain division.  Every result therefore equals a / b bit for bit.
+// (recip_shared, the sequence's own reciprocal, would do as well; only
+// tests/div_check/check_div.hip takes it.)
 __device__ __forceinline__ double recip_shared(double b) {
   const double r0 = __builtin_amdgcn_rcp(b);
   const double e0 = __builtin_fma(-b, r0, 1.0);
