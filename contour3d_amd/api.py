@@ -485,20 +485,28 @@ def tune(param, value):
         raise RuntimeError("contour3d_amd_tune failed")
 
 
+# what the frame path tells apart; 0 is the default of each, and with rows and
+# planes both 0 the bricks follow the work of every view
 AUTOTUNE_KNOBS = {
-    TUNE_TESS_GRID: (0, 16384, 1 << 30),   # persistent workgroups (0: 128 per CU), or one per work item
-    TUNE_TESS_ROWS: (0, 2, 1),             # rows of cells per tile (0: as many as fit in 2048 cells)
-    TUNE_TESS_ZPLANES: (2, 4, 8, 16),      # z-planes per work item (4 by default)
+    TUNE_TESS_GRID: (0, 1024),         # workgroups that draw (0: 6 per CU)
+    TUNE_TESS_ROWS: (0, 2),            # rows of cells of every brick, of at most 64 columns
+    TUNE_TESS_ZPLANES: (0, 2, 4, 8),   # planes of every brick (0 beside rows: 8)
 }
 KNOB_NAMES = {TUNE_TESS_GRID: "tess_grid", TUNE_TESS_ROWS: "tess_rows", TUNE_TESS_ZPLANES: "tess_zplanes"}
 
 
+AUTOTUNE_GAIN = 0.02
+
+
 def autotune(run, knobs=None, reps=2):
     """Times run() under every combination of the launch-shape knobs (a dict
-    tune parameter -> values; default AUTOTUNE_KNOBS: the tessellation
-    workgroup cap and brick shape, which the frame path reads) and keeps the
-    fastest.  Every setting renders the same bits.  Returns (best settings
-    by knob name, best ms, the sweep as a list of (settings, ms))."""
+    tune parameter -> values; default AUTOTUNE_KNOBS: the drawing workgroups
+    and the brick shape, which the frame path reads) and keeps the fastest,
+    or the defaults (every knob 0, if among them) where nothing is faster by
+    more than AUTOTUNE_GAIN: a brick shape that is set holds for every later
+    view, however different.  Every setting renders the same bits.  Returns
+    (the settings kept by knob name, their ms, the sweep as a list of
+    (settings, ms))."""
     import itertools
     import time
 
@@ -520,6 +528,9 @@ def autotune(run, knobs=None, reps=2):
         ms = (time.perf_counter() - t0) / reps * 1e3
         sweep.append(({KNOB_NAMES.get(p, str(p)): v for p, v in zip(params, values)}, ms))
     best = min(range(len(sweep)), key=lambda q: sweep[q][1])
+    plain = (0,) * len(params)
+    if plain in combos and sweep[best][1] > (1.0 - AUTOTUNE_GAIN) * sweep[combos.index(plain)][1]:
+        best = combos.index(plain)
     for p, v in zip(params, combos[best]):
         tune(p, v)
     return sweep[best][0], sweep[best][1], sweep
