@@ -315,6 +315,7 @@ struct Frame {
   DevBuf cnt, tiles, tjobs, rjobs, hdr, jimg, order, take;
   DevBuf key, id, rgb, depth, fpix, fdep, frgb, frags, vntmp;
   uint32_t frag_cap = 0;
+  uint32_t frag_most = ~0u;  // what the fragment list may grow to: less once there was no memory for more
   HostBuf hrgb, hstage;
   // host sources of asynchronous uploads stay alive until the frame ends
   std::vector<TessJob> h_tjobs;
@@ -358,6 +359,7 @@ struct Frame {
     for (auto* b : bufs) b->release();
     mesh.release();
     if (!noalloc) frag_cap = 0;
+    frag_most = ~0u;
     hrgb.release();
     if (hstage.p) (void)hipHostFree(hstage.p);
     hstage.p = nullptr;
@@ -1545,7 +1547,14 @@ int raster_prepare(Frame& F, uint64_t npx, bool stored) {
   if (F.frag_cap == 0) F.frag_cap = kDefaultFragCap;
   // a stored mesh's entries are smaller, and in FP32 it keeps no list
   const size_t entry = !stored ? sizeof(Frag64) : fp64 ? sizeof(Frag) : 0;
-  C3D_HIP(F.frags.ensure(size_t(F.frag_cap) * entry));
+  hipError_t e = F.frags.ensure(size_t(F.frag_cap) * entry);
+  if (e == hipErrorOutOfMemory && F.frag_cap > kDefaultFragCap) {
+    // a long list is not worth the frame: with the first one it takes the id
+    // pass over the geometry
+    F.frag_cap = F.frag_most = kDefaultFragCap;
+    e = F.frags.ensure(size_t(F.frag_cap) * entry);
+  }
+  C3D_HIP(e);
   return 0;
 }
 
@@ -1661,7 +1670,7 @@ int frame_finish(Frame& F) {
   F.drawn = false;
   if ((fin.overflow & 2u) && fin.nfrag > F.frag_cap && !F.noalloc) {
     const uint64_t grow = uint64_t(fin.nfrag) + fin.nfrag / 4;
-    F.frag_cap = uint32_t(grow > 0xffffffffull ? 0xffffffffull : grow);
+    F.frag_cap = uint32_t(std::max<uint64_t>(F.frag_cap, std::min<uint64_t>(grow, F.frag_most)));
   }
   if (refused) {
     if (F.noalloc)
@@ -2525,6 +2534,7 @@ int contour3d_amd_tune(int param, int64_t value) {
       return 0;
     case CONTOUR3D_AMD_TUNE_FRAG_CAPACITY:
       L.main.frag_cap = value > 0 ? uint32_t(std::min<int64_t>(value, 0xffffffffll)) : c3d::kDefaultFragCap;
+      L.main.frag_most = ~0u;
       return 0;
     case CONTOUR3D_AMD_TUNE_GRAPHS:
       L.graphs = value != 0;

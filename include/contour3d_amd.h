@@ -295,8 +295,9 @@ enum {
                                            128 per CU for count, and one per tile for emit) */
   CONTOUR3D_AMD_TUNE_RASTER_GRID = 1,   /* max workgroups of the raster passes (0 = one per 256 triangles) */
   CONTOUR3D_AMD_TUNE_FRAG_CAPACITY = 2, /* fragment list entries, 24 B each (0: the default, 2^24; grows by
-                                           itself after an overflow; an overflowing frame takes the slower
-                                           id pass over the geometry) */
+                                           itself after an overflow, and goes back to 2^24 where there is
+                                           no memory for more; an overflowing frame takes the slower id
+                                           pass over the geometry) */
   CONTOUR3D_AMD_TUNE_GRAPHS = 3,        /* 1: contour3d_execute, _execute_rgb and _execute_batch capture
                                            their launch sequence as a HIP graph and replay it while the
                                            frame layout (image sizes, objects' fields and lattices,
