@@ -398,8 +398,8 @@ struct Lib {
   // workgroups of the tessellation and raster kernels (0: built-in choice)
   uint32_t tess_cap = 0;
   uint32_t raster_cap = 0;
-  // tessellation brick shape: rows of cells per tile (0: as many as fit in
-  // kTileCells) and planes per work item (0: kDefaultZPlanes)
+  // rows of cells and planes of a mesh's tiles (0: as many rows as fit in
+  // kTileCells, kDefaultZPlanes) and of a frame's bricks (0: choose_bricks)
   uint32_t tess_rows = 0;
   uint32_t tess_zc = 0;
   bool graphs = false;  // replay captured launch sequences of repeated frame layouts
@@ -410,8 +410,9 @@ struct Lib {
     const uint32_t g = cap < nitems ? cap : nitems;
     return g < 8 ? 8 : g;
   }
-  // workgroups of a frame's draw: as many as are resident at once (they take
-  // their bricks one by one)
+  // workgroups of a frame's draw, which take their bricks one by one: six per
+  // CU, as many as are resident at once in FP32 (in FP64 four are, and the
+  // others find what bricks are left)
   uint32_t frame_grid() const {
     const uint32_t g = uint32_t(persistent_blocks()) / 8u * 6u;
     return tess_cap && tess_cap < g ? tess_cap : g;
@@ -626,11 +627,6 @@ uint64_t fnv(const void* data, size_t bytes, uint64_t h) {
 
 using ConvFn = contour3d_vector_t (*)(const contour3d_vector_t);
 
-// Device coordinates of an object's lattice.  The converter maps each
-// lattice point (grids[0][i], grids[1][j], grids[2][k]) to Cartesian
-// (triangulate.c:165-170); it is evaluated once per point and the result
-// cached for as long as the converter, grid pointers and grid values stay
-// the same.  A map that returns every point unchanged needs no table.
 // whether the values are finite and never turn back
 bool ordered_grid(const double* g, size_t n) {
   bool up = true, down = true, fin = true;
@@ -666,6 +662,11 @@ LatticeMid lattice_mid(const double* const g[3], const size_t n[3], const double
   return m;
 }
 
+// Device coordinates of an object's lattice.  The converter maps each
+// lattice point (grids[0][i], grids[1][j], grids[2][k]) to Cartesian
+// (triangulate.c:165-170); it is evaluated once per point and the result
+// cached for as long as the converter, grid pointers and grid values stay
+// the same.  A map that returns every point unchanged needs no table.
 int get_geometry(Lib& L, const contour3d_contour_obj_t& o, Geom** out) {
   const size_t nx = o.glsizes[0], ny = o.glsizes[1], nz = o.glsizes[2];
   std::vector<double> hg[3];
@@ -1118,10 +1119,11 @@ void choose_bricks(const std::vector<TessJob>& tj, const std::vector<const Latti
   }
 }
 
-// Host half of a frame's tessellation (or, with `stored`, a mesh's): validates the objects, resolves
-// fields (host fields are uploaded) and lattices, groups thresholds of a
-// shared field into field passes, sizes the buffers and enqueues the uploads
-// of the pass and object tables.  The layout goes to F.tl.
+// Host half of a frame's tessellation (or, with `stored`, a mesh's): validates
+// the objects, resolves fields (host fields are uploaded) and lattices, groups
+// thresholds of a shared field into field passes, sizes the buffers and
+// enqueues the uploads of the pass and object tables.  The layout goes to F.tl.
+// by_view: a frame's bricks follow the work of its views.
 template <typename R>
 int tess_prepare(Lib& L, Frame& F, contour3d_amd_mesh& M, const std::vector<const contour3d_contour_obj_t*>& objs,
                  bool stored, bool by_view = true) {
@@ -1914,8 +1916,9 @@ int run_frame_t(Lib& L, Frame& F, std::vector<Image>& imgs, bool graph) {
   if (upload_pass_images(F, imgs)) return 1;
   if (raster_prepare<R>(F, npx, false)) return 1;
   if (graph ? graph_frame<R>(L, F, rjd, njobs, npx) : frame_launch<R>(L, F, rjd, njobs, npx, F.h_nline)) return 1;
+  if (raster_copies(F, imgs, sizeof(R) == 8)) return 1;
   F.drawn = true;
-  return raster_copies(F, imgs, sizeof(R) == 8);
+  return 0;
 }
 
 // Renders the images as one frame into F; with wait, also waits for the
@@ -2144,6 +2147,9 @@ void snap_give(Server& S, Request& r) {
 
 std::mutex g_server_mu;  // server start/stop against submit/wait/stats
 
+// device bytes a request adds to a frame: z-buffer, ids and image buffers, a
+// share of the fragment list (four fragments per pixel), and host fields to
+// upload
 uint64_t estimate_bytes(const contour3d_amd_image_t& im) {
   double upload = 0;
   for (size_t o = 0; o < im.num_contours; o++) {

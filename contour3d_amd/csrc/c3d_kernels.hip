@@ -14,9 +14,6 @@
 namespace c3d {
 
 // ----------------------------------------------------------------------
-// small helpers
-
-// ----------------------------------------------------------------------
 // block-wide exclusive scan of one value per thread (256 threads)
 
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
@@ -161,21 +158,6 @@ __device__ __forceinline__ uint32_t corner_code(double thr, const double v[8]) {
 #pragma unroll
   for (int n = 0; n < 8; n++) code |= uint32_t(thr < v[n]) << n;
   return code;
-}
-
-// triangle counts of up to four thresholds packed 16 bits apart, from an
-// LDS copy of c_ntri
-__device__ __forceinline__ uint64_t packed_counts(const ThrSet& ts, const double v[8], uint32_t code[kMaxThr],
-                                                  const uint8_t* s_ntri) {
-  uint64_t packed = 0;
-#pragma unroll
-  for (int q = 0; q < kMaxThr; q++) {
-    uint32_t cd = 0;
-    if (q < ts.n) cd = corner_code(ts.thr[q], v);
-    code[q] = cd;
-    packed |= uint64_t(s_ntri[cd]) << (16 * q);
-  }
-  return packed;
 }
 
 // ----------------------------------------------------------------------
@@ -552,8 +534,6 @@ __device__ __forceinline__ bool interior_cell(const FieldDev& f, const CellLoc& 
 
 __constant__ NbrTable c_nbr;
 
-
-
 // the edge word of stored triangle u (in the gather record in FP64, in the
 // position record in FP32)
 template <typename R>
@@ -901,10 +881,11 @@ __global__ __launch_bounds__(kThreads) void k_raster(MeshView<R> m, const Raster
 //
 // A brick that lies behind what the z-buffer holds is counted but not drawn,
 // except for cells whose triangles' projections may be too small for the
-// depth bound to hold (c3d_cull.h; FP64 only: in FP32 rounding leaves too
-// many such cells).  With the bricks taken front to back, most of a dense
-// field is behind its first surfaces: at 512^3, three thresholds and
-// 1920 x 1080, 42 M of 129 M triangles are drawn.
+// depth bound to hold (c3d_cull.h; FP64 only: with FP32's rounding the rule,
+// which judges a cell by its brick's extent, holds of next to none at 512^3).
+// With the bricks taken front to back, most of a dense field is behind its
+// first surfaces: at 512^3, three thresholds and 1920 x 1080, 42 M of 129 M
+// triangles are drawn.
 //
 // What bounds it: vector-ALU issue (1000 instructions per 64 triangles in
 // FP32 before the pixel box was formed directly, divisions by view constants
